@@ -48,13 +48,13 @@ namespace {
 
 constexpr int kBlock = 256;
 // block size of k_flux_hlld_fast (it ends without a block barrier): FP64 in one-wave blocks
-// (33.6 ms of sweeps per plain 256^3 step, against 34.1 with 2-wave and 35.5 with 4-wave
-// blocks), FP32 in blocks of 4 (8-wave blocks: 16.1 against 14.6 ms; 2-wave blocks: 14.5)
+// (1.55 ms for the slowest 256^3 sweep, 1.67 with 4-wave blocks), FP32 in blocks of 4
+// (8-wave blocks: 16.1 against 14.6 ms of sweeps per step; 2-wave blocks: 14.5)
 template <typename R> constexpr int kFluxBlock = sizeof(R) == 4 ? 256 : 64;
 // occupancy targets of k_flux_hlld_fast (waves per SIMD), measured at 256^3 WENO5/HLLD:
-// FP64 at 2 (213 VGPRs, no scratch; 4.0 ms, against 4.7 at 3 with 184 B spilled),
-// FP32 at 5 (96 VGPRs, 40 B/lane scratch; at 4 waves, with none, 9 % slower)
-constexpr int kFastFluxWaves64 = 2;
+// FP64 at 3 (166 VGPRs, no scratch: 1.48-1.55 ms a sweep, against 1.92-2.23 at 4, which
+// spills), FP32 at 5 (92 VGPRs; at 4 waves 9 % slower)
+constexpr int kFastFluxWaves64 = 3;
 constexpr int kFastFluxWaves32 = 5;
 constexpr int kRedoBlocks = 1024;    // grid of k_flux_redo (a grid-stride loop over its queue)
 
@@ -496,25 +496,7 @@ __device__ __forceinline__ int interface_flux(const double *__restrict__ P, long
                                               int &retried)
 {
   R ql[8], qr[8];
-  const R theta = (R)pp.theta;
-  for (int q = 0; q < 8; ++q) {
-    const double *Pq = P + q * T + z;
-    const R v0 = (R)Pq[0], v1 = (R)Pq[S];
-    if (recon == RECON_WENO5) {
-      const R vm2 = (R)Pq[-2 * S], vm1 = (R)Pq[-S], v2 = (R)Pq[2 * S], v3 = (R)Pq[3 * S];
-      ql[q] = weno5<R, true>(vm2, vm1, v0, v1, v2, pp.IS, (R)pp.sz10A);
-      qr[q] = weno5<R, false>(vm1, v0, v1, v2, v3, pp.IS, (R)pp.sz10A);
-    }
-    else if (recon == RECON_PLM) {
-      const R vm1 = (R)Pq[-S], v2 = (R)Pq[2 * S];
-      ql[q] = plm<R>(vm1, v0, v1, R(+1.0), theta);
-      qr[q] = plm<R>(v0, v1, v2, R(-1.0), theta);
-    }
-    else {
-      ql[q] = v0;
-      qr[q] = v1;
-    }
-  }
+  reconstruct_states<R, false>(P, T, S, z, recon, pp, ql, qr);
   int err = 1;
   retried = 0;
   // one call site: the reconstructed states, then the zone-centred states
@@ -537,33 +519,26 @@ __device__ __forceinline__ int interface_flux(const double *__restrict__ P, long
   return err;
 }
 
-/* The common path of an HLLD interface: reconstruction and riemann_hlld in FAST mode.
- * Returns kHlldDefer, with F unwritten, where the full solver is needed. */
+/* The common path of an HLLD interface, the flux written to its planes: reconstruction and
+ * riemann_hlld_lean in FP64, riemann_hlld in FAST mode in FP32. Returns kHlldDefer where the
+ * full solver is needed. */
 template <typename R, int DIM>
-__device__ __forceinline__ int interface_flux_fast(const double *__restrict__ P, long T, long S, long z,
-                                                   int recon, const PhysParams &pp, R *F, R &lam,
-                                                   FluxCounters &fc)
+__device__ __forceinline__ int interface_flux_fast(const double *__restrict__ P, R *__restrict__ Fout, long T, long S,
+                                                   long z, int recon, const PhysParams &pp, R &lam, FluxCounters &fc)
 {
   R ql[8], qr[8];
-  const R theta = (R)pp.theta;
-  for (int q = 0; q < 8; ++q) {
-    const double *Pq = P + q * T + z;
-    const R v0 = (R)Pq[0], v1 = (R)Pq[S];
-    if (recon == RECON_WENO5) {
-      const R vm2 = (R)Pq[-2 * S], vm1 = (R)Pq[-S], v2 = (R)Pq[2 * S], v3 = (R)Pq[3 * S];
-      ql[q] = weno5<R, true>(vm2, vm1, v0, v1, v2, pp.IS, (R)pp.sz10A);
-      qr[q] = weno5<R, false>(vm1, v0, v1, v2, v3, pp.IS, (R)pp.sz10A);
+  reconstruct_states<R, sizeof(R) == 8>(P, T, S, z, recon, pp, ql, qr);
+  if constexpr (sizeof(R) == 8)
+    return riemann_hlld_lean<DIM>(ql, qr, pp, lam, fc, [&](int q, double f) { Fout[q * T + z] = f; });
+  else {
+    R F[8];
+    const int rc = riemann_hlld<R, DIM, true>(ql, qr, F, (R)pp.gamma, pp.pfloor, lam, fc);
+    if (rc == 0) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) Fout[q * T + z] = F[q];
     }
-    else if (recon == RECON_PLM) {
-      ql[q] = plm<R>((R)Pq[-S], v0, v1, R(+1.0), theta);
-      qr[q] = plm<R>(v0, v1, (R)Pq[2 * S], R(-1.0), theta);
-    }
-    else {
-      ql[q] = v0;
-      qr[q] = v1;
-    }
+    return rc;
   }
-  return riemann_hlld<R, DIM, true>(ql, qr, F, (R)pp.gamma, pp.pfloor, lam, fc);
 }
 
 /* Flux sweep along DIM, one thread per interface. With a redo queue (mixed form, HLLD),
@@ -739,11 +714,8 @@ void k_flux_hlld_fast(const double *__restrict__ P, R *__restrict__ Fout, GridDe
   if (has) {
     R lam = R(0);
     FluxCounters fc = {0, 0, 0, 0};
-    R F[8];
-    defer = interface_flux_fast<R, DIM>(P, T, S, z, recon, pp, F, lam, fc) != 0;
+    defer = interface_flux_fast<R, DIM>(P, Fout, T, S, z, recon, pp, lam, fc) != 0;
     if (!defer) {
-#pragma unroll
-      for (int q = 0; q < 8; ++q) Fout[q * T + z] = F[q];
       cnt[0] = 1;
       cnt[1] = (unsigned long long)fc.c2p_iters;
       cnt[2] = (unsigned long long)fc.newton_iters;
@@ -1026,8 +998,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_ctu_faces(const double *__restric
   block_add<5>(cnt, dst);
 }
 
-/* The HLLD faces of k_ctu_faces on the common path (riemann_hlld in FAST mode, a lower
- * register peak): a face that needs the c2p cascade, a later Newton attempt, the small
+/* The HLLD faces of k_ctu_faces on the common path (riemann_hlld_lean): a face that needs the c2p cascade, a later Newton attempt, the small
  * normal field branch or the HLLC fallback is queued for k_ctu_faces_redo. The queue holds
  * every face, so it cannot overflow. */
 template <int DIM>
@@ -1046,12 +1017,10 @@ void k_ctu_faces_fast(const double *__restrict__ P, const double *__restrict__ P
     ctu_face_states(P, Ps, T, sxz, S, z, pp.theta, pl, pr);
     if (check_prim(pl) || check_prim(pr)) cnt[0] = 1;
     else {
-      double f[8], lam = 0.0;
+      double lam = 0.0;
       FluxCounters fc = {0, 0, 0, 0};
-      defer = riemann_hlld<double, DIM, true>(pl, pr, f, pp.gamma, pp.pfloor, lam, fc) != 0;
+      defer = riemann_hlld_lean<DIM>(pl, pr, pp, lam, fc, [&](int q, double f) { F[q * T + z] = f; }) != 0;
       if (!defer) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) F[q * T + z] = f[q];
         cnt[1] = 1;
         cnt[2] = (unsigned long long)fc.c2p_iters;
         cnt[3] = (unsigned long long)fc.newton_iters;
@@ -2454,6 +2423,9 @@ int maragpu_advance(maragpu_ctx *c, double dt, maragpu_stats *stats)
   pp.theta = c->cfg.theta;
   pp.IS = c->cfg.IS;
   pp.sz10A = c->cfg.sz10A;
+  pp.g1 = pp.gamma / (pp.gamma - 1.0);
+  pp.gamf = (pp.gamma - 1.0) / pp.gamma;
+  pp.igamma = 1.0 / pp.gamma;
   const bool mixed = c->cfg.precision == MARAGPU_MIXED;
   int evi = 0;
   std::vector<EventPair> ef, ec, eu;

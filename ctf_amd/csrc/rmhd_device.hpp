@@ -41,7 +41,14 @@ template <> struct Tol<double> {
   static constexpr bool nested_c2p_from_average = true;
   static constexpr bool nested_c2p_fp32 = false;  // that attempt in FP64
   static constexpr double newton_ftol = 1e-12;   // NewtonRaphesonSolver(15, 1e-12), riemann_hlld-rmhd.cpp:220
-  static constexpr int newton_fast_max_it = 15;  // the common path's p* solve: the reference's
+  // common path (riemann_hlld_lean): Newton steps of the p* solve (the reference's); the last
+  // one, from a residual within newton_ftol, reuses the derivative of the one before where
+  // it moves p by at most reuse_step, relatively; step tolerance and cap of the nested c2p,
+  // whose result only starts the p* solve
+  static constexpr int newton_fast_max_it = 15;
+  static constexpr double reuse_step = 1e-11;
+  static constexpr double nested_step = 1e-6;
+  static constexpr int nested_max_it = 16;
   static constexpr double fd_dp = 1e-8;          // HlldEquation48::Jacobian, :313
   static constexpr bool fd_relative = false;
   static constexpr bool fd_one_sided = false;    // the reference's centred difference
@@ -97,6 +104,7 @@ struct PhysParams {
   double theta;
   int IS;
   double sz10A;
+  double g1, gamf, igamma;     // Gamma/(Gamma-1), (Gamma-1)/Gamma, 1/Gamma
 };
 
 __device__ __forceinline__ double dsqrt(double x) { return sqrt(x); }
@@ -131,6 +139,44 @@ __device__ __forceinline__ double rcp(double x)
 }
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
+/* The lean forms of the FP64 sweeps. The hardware approximations of 1/x and 1/sqrt(x) are
+ * good to 2^-23 or better, so one step of third order, y (1 + e + e^2) with the residual
+ * e = 1 - x y formed exactly by an FMA, is within an ulp (what is left of e is 2^-69): three
+ * FMAs, where two Newton steps take four. No fix-up of special cases: 1/0, 1/inf and the
+ * roots of 0 and inf are NaN, for callers that hand such a state to the full solver or
+ * select around it. */
+__device__ __forceinline__ double rcp_normal(double x)
+{
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
+}
+__device__ __forceinline__ float rcp_normal(float x) { return __builtin_amdgcn_rcpf(x); }
+/* 1/sqrt(x): y (1 + e/2 + 3/8 e^2), e = 1 - x y^2 */
+__device__ __forceinline__ double rsqrt_normal(double x)
+{
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y, e * fma(0.375, e, 0.5), y);
+}
+/* sqrt(x) by one coupled step on (sqrt x, 1/(2 sqrt x)) and a last residual, 0 and inf as they
+ * are: 11 instructions. sqrt() also scales x against underflow of the residual (x < 1e-290)
+ * and takes 18. */
+__device__ __forceinline__ double sqrt_lean(double x)
+{
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  g = fma(fma(-g, g, x), h, g);
+  return (x == 0.0 || x == INFINITY) ? x : g;
+}
+
+__device__ __forceinline__ double dfmin(double a, double b) { return fmin(a, b); }
+__device__ __forceinline__ float dfmin(float a, float b) { return fminf(a, b); }
+__device__ __forceinline__ double dfmax(double a, double b) { return fmax(a, b); }
+__device__ __forceinline__ float dfmax(float a, float b) { return fmaxf(a, b); }
 template <typename R> __device__ __forceinline__ bool is_nan(R x) { return x != x; }
 template <typename R> __device__ __forceinline__ bool is_inf(R x) { return dfabs(x) == R(INFINITY); }
 
@@ -270,6 +316,131 @@ template <typename R> __device__ __forceinline__ void quartic_extremes(R d4, R d
     if (r3 < rmin) rmin = r3;
     if (r4 > rmax) rmax = r4;
     if (r4 < rmin) rmin = r4;
+    nr += 2;
+  }
+}
+
+/* cos(2/3 acos(s)) = T_{2/3}(s) for s in [0, 1] and, where s > 1, its continuation
+ * cosh(2/3 acosh(s)) up to s = 1.01: a polynomial of degree 19 in 2 s - 1, from the function's
+ * Chebyshev series (computed with 60 digits; the nearest singularity is s = -1, so the terms
+ * fall by 5.8 each), within 1.3e-16. With s = sqrt((1 + x)/2) it is cos(acos(x)/3), the
+ * trigonometric root of a cubic, without the arc cosine and cosine and their range
+ * reductions (120 instructions; 21 here, in two chains). */
+__device__ __forceinline__ double cos_two_thirds_acos(double s)
+{
+  const double u = fma(2.0, s, -1.0), w = u*u;
+  double e = -1.6089233320740645e-11, o = 5.082538322352577e-12;
+  e = fma(e, w, -9.128174258928075e-11); o = fma(o, w, 2.7036688125375587e-11);
+  e = fma(e, w, -1.1880162409356414e-09); o = fma(o, w, 3.575095124594894e-10);
+  e = fma(e, w, -1.334519367092948e-08); o = fma(o, w, 3.929463288067197e-09);
+  e = fma(e, w, -1.5954537531426307e-07); o = fma(o, w, 4.586042851669284e-08);
+  e = fma(e, w, -2.0358689700992568e-06); o = fma(o, w, 5.641509636123585e-07);
+  e = fma(e, w, -2.8919936440265828e-05); o = fma(o, w, 7.541078640701342e-06);
+  e = fma(e, w, -0.0005041246911250438); o = fma(o, w, 0.00011642545293476212);
+  e = fma(e, w, -0.015509188436486424); o = fma(o, w, 0.002466352815087338);
+  e = fma(e, w, 0.766044443118978); o = fma(o, w, 0.24740906632285303);
+  return fma(o, u, e);
+}
+
+/* quartic_extremes in lean FP64. The quartic of RMHD has four real roots, so its resolvent cubic has three (delta <= 0)
+ * and Ferrari's method uses the largest, 2 sqrt(-q) cos(acos(x)/3) with
+ * x = r (-q)^(-3/2): of the reference's x1 and x3 the first is the larger one on the whole
+ * range, so the sine of the other is not needed. Where the normal field vanishes two roots
+ * coincide (x = -1) and round-off decides the sign of delta; for delta > 0 the reference
+ * takes the cubic's one real root, which is +-2 sqrt(-q) cosh(acosh|x|/3), the same function
+ * continued to s > 1. Only where q >= 0 or |x| > 1.02 (not met by such states) do the cube
+ * roots remain. In FP64 that takes 140 instructions, of 450 with acos, cos, sin and cbrt and
+ * their divergence (half the lanes of an axis without normal field take either sign of
+ * delta). FULL = false leaves the cube roots out and returns no roots there. */
+template <bool FULL = true>
+__device__ __forceinline__ double resolvent_root(double ca2, double ca1, double ca0)
+{
+  const double q = ca1*(1.0/3.0) - ca2*ca2*(1.0/9.0);
+  const double r = (ca1*ca2 - 3.0*ca0)*(1.0/6.0) - ca2*ca2*ca2*(1.0/27.0);
+  const double delta = q*q*q + r*r;
+  const double y = rsqrt_normal(-q);
+  const double x = r*(y*y*y);
+  if (dfabs(x) < 1.02) {                        // false where q >= 0 (y is inf or NaN)
+    const bool one = delta > 0.0;
+    const double t = one ? dfabs(x) : x;
+    const double s2 = dfmax(0.5 + 0.5*t, 0.0);
+    const double c = cos_two_thirds_acos(sqrt_lean(s2));
+    const double m = -2.0*q*y;                  // 2 sqrt(-q)
+    return (one && r < 0.0 ? -m : m)*c - ca2*(1.0/3.0);
+  }
+  if constexpr (!FULL) return NAN;              // the caller hands such a state on
+  double x1, x3;
+  int ncub;
+  if (delta > 0.0) {
+    double s1 = r + sqrt_lean(delta);
+    s1 = (s1 >= 0.0) ? cbrt(s1) : -cbrt(-s1);
+    double s2 = r - sqrt_lean(delta);
+    s2 = (s2 >= 0.0) ? cbrt(s2) : -cbrt(-s2);
+    x1 = (s1+s2) - ca2*(1.0/3.0);
+    x3 = x1;
+    ncub = 1;
+  }
+  else if (delta < 0.0) {
+    const double theta = acos(r/sqrt(-q*q*q)) * (1.0/3.0);
+    const double costh = cos(theta);
+    const double sinth = sin(theta);
+    const double sq = sqrt(-q);
+    x1 = 2.0*sq*costh - ca2*(1.0/3.0);
+    x3 = -sq*costh - ca2*(1.0/3.0) + sqrt(3.0) * sq * sinth;
+    ncub = 3;
+  }
+  else {
+    const double s = (r >= 0.0) ? cbrt(r) : -cbrt(-r);
+    x1 = 2.0*s - ca2*(1.0/3.0);
+    x3 = -s - ca2*(1.0/3.0);
+    ncub = 3;
+  }
+  return (ncub == 1) ? x1 : ((x1 > x3) ? x1 : x3);
+}
+
+template <bool FULL = true>
+__device__ __forceinline__ void quartic_extremes_lean(double d4, double d3, double d2, double d1, double d0, double &rmax,
+                                                 double &rmin, int &nr)
+{
+  const double id4 = rcp_normal(d4);
+  const double a3 = d3*id4, a2 = d2*id4, a1 = d1*id4, a0 = d0*id4;
+  const double au2 = -a2;
+  const double au1 = (a1*a3 - 4.0*a0);
+  const double au0 = 4.0*a0*a2 - a1*a1 - a0*a3*a3;
+  const double u1 = resolvent_root<FULL>(au2, au1, au0);
+  const double R2 = 0.25*a3*a3 + u1 - a2;
+  double D2, E2, Rr = 0.0;
+  if (R2 > 0.0) {
+    const double iR = rsqrt_normal(R2);
+    Rr = R2*iR;
+    const double foo1 = 0.75*a3*a3 - R2 - 2.0*a2;
+    const double foo2 = 0.25*(4.0*a3*a2 - 8.0*a1 - a3*a3*a3) * iR;
+    D2 = foo1 + foo2;
+    E2 = foo1 - foo2;
+  }
+  else {
+    const double foo1 = 0.75*a3*a3 - 2.0*a2;
+    const double foo2 = 2.0 * sqrt_lean(u1*u1 - 4.0*a0);
+    D2 = foo1 + foo2;
+    E2 = foo1 - foo2;
+  }
+  // roots r1 <= r2 (if D2 >= 0) and r3 <= r4 (if E2 >= 0)
+  rmax = -1.0;
+  rmin = 1.0;
+  nr = 0;
+  const double m = -0.25*a3;
+  if (D2 >= 0.0) {
+    const double D = 0.5*sqrt_lean(D2), c = m + 0.5*Rr;
+    const double r1 = c - D, r2 = c + D;
+    if (r2 > rmax) rmax = r2;
+    if (r1 < rmin) rmin = r1;
+    nr += 2;
+  }
+  if (E2 >= 0.0) {
+    const double E = 0.5*sqrt_lean(E2), c = m - 0.5*Rr;
+    const double r3 = c - E, r4 = c + E;
+    if (r4 > rmax) rmax = r4;
+    if (r3 < rmin) rmin = r3;
     nr += 2;
   }
 }
@@ -731,20 +902,17 @@ __device__ __forceinline__ int cons_to_prim(const double *U, double *P, double g
 /* ---------------------------------------------------------------------------
  * Reconstruction, Mara/weno.c
  * ------------------------------------------------------------------------- */
-template <typename R> __device__ __forceinline__ int sgn(R x) { return (x > R(0)) - (x < R(0)); }
-
 /* __plm with __plm_minmod, weno.c:85-96: v points at the centre zone */
 template <typename R> __device__ __forceinline__ R plm(R vm, R v0, R vp, R sg, R theta)
 {
   const R a = theta * (v0 - vm);
   const R b = R(0.5) * (vp - vm);
   const R c = theta * (vp - v0);
-  const R fa = dfabs(a), fb = dfabs(b), fc = dfabs(c);
-  const R m01 = fa < fb ? fa : fb;
-  const R mn = m01 < fc ? m01 : fc;
-  const int s1 = sgn(a) + sgn(b);
-  const int as1 = s1 < 0 ? -s1 : s1;
-  const R lim = R(0.25)*R(as1)*R(sgn(a) + sgn(c))*mn;
+  // minmod: the smallest of the three where all are positive, the largest where all are
+  // negative, else zero. The reference's product of signs and the smallest magnitude is the
+  // same value; as minima and maxima it takes 7 operations instead of 25.
+  const R lo = dfmin(dfmin(a, b), c), hi = dfmax(dfmax(a, b), c);
+  const R lim = dfmax(lo, R(0)) + dfmin(hi, R(0));
   return v0 + sg*R(0.5)*lim;
 }
 
@@ -813,6 +981,85 @@ __device__ __forceinline__ R weno5(R vm2, R vm1, R v0, R vp1, R vp2, int IS, R s
   }
   const R wtot = w0 + w1 + w2;
   return (w0*vs0 + w1*vs1 + w2*vs2) * rcp(wtot);
+}
+
+/* Both finite-volume WENO5 states of an interface with the Jiang-Shu weights: the right face
+ * of v0 and the left face of v1 (weno.c:24-31,97-154), from v[-2..3] in one go. Written in
+ * the stencil's first and second differences g and t: every substencil's value is the
+ * midpoint (v0 + v1)/2 plus a multiple of second differences, and its smoothness indicator
+ * x 4 is 13/3 t^2 + u^2 with u one fused step from g and t, so the two sides share the
+ * midpoint, the differences and the t^2 terms (the inner two stencils belong to both). The
+ * weights are the reference's scaled by a common factor. Instruction bound: 80 FP64 operations
+ * for the pair where two weno5 calls take 130, and the corrections are sums of small
+ * differences, so they round no worse. */
+__device__ __forceinline__ void weno5_js_pair(double vm2, double vm1, double v0, double v1, double v2, double v3,
+                                              double &ql, double &qr)
+{
+  const double ga = vm1 - vm2, gb = v0 - vm1, gc = v1 - v0, gd = v2 - v1, ge = v3 - v2;
+  const double tb = gb - ga, tc = gc - gb, td = gd - gc, te = ge - gd;
+  const double c = 13./3., e4 = 4e-6;
+  const double Tb = (c*tb)*tb + e4, Tc = (c*tc)*tc + e4, Td = (c*td)*td + e4, Te = (c*te)*te + e4;
+  const double mid = 0.5*(v0 + v1);
+  // one side: indicators x 4 (+ 4 eps) of the downwind, centred and upwind stencils, and the
+  // corrections x -8 of the last two from the first's second difference on
+  auto side = [&](double T0, double u0, double T1, double u1, double T2, double u2, double t0, double t1, double t2) {
+    const double B0 = u0*u0 + T0, B1 = u1*u1 + T1, B2 = u2*u2 + T2;
+    const double a0 = B0*B0, a1 = B1*B1, a2 = B2*B2;
+    const double w0 = 5.0*(a1*a2), w1 = 10.0*(a0*a2), w2 = a0*a1;
+    const double num = w0*t0 + w1*t1 + w2*(4.0*t1 - 3.0*t2);
+    return mid - 0.125*(num * rcp_normal(w0 + w1 + w2));
+  };
+  // u of the three stencils: 3 v0 - 4 v1 + v2, v[-1] - v1 and v[-2] - 4 v[-1] + 3 v0 (signs
+  // do not matter), and mirrored about the interface
+  ql = side(Td, td - 2.0*gc, Tc, gb + gc, Tb, tb + 2.0*gb, td, tc, tb);
+  qr = side(Tc, tc + 2.0*gc, Td, gc + gd, Te, te - 2.0*gd, tc, td, te);
+}
+
+/* The two states of interface z | z+S from its 6-point stencil. LEAN (FP64): the paired
+ * WENO5, and the choice of method outside the fields' loop, so that the loads of all fields
+ * can be in flight. */
+template <typename R, bool LEAN>
+__device__ __forceinline__ void reconstruct_states(const double *__restrict__ P, long T, long S, long z, int recon,
+                                                   const PhysParams &pp, R *ql, R *qr)
+{
+  if constexpr (LEAN) {
+    if (recon == RECON_WENO5 && pp.IS == IS_JS96) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const double *v = P + q * T + z;
+        weno5_js_pair(v[-2 * S], v[-S], v[0], v[S], v[2 * S], v[3 * S], ql[q], qr[q]);
+      }
+      return;
+    }
+    if (recon == RECON_PLM) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const double *v = P + q * T + z;
+        const double v0 = v[0], v1 = v[S];
+        ql[q] = plm<double>(v[-S], v0, v1, +1.0, pp.theta);
+        qr[q] = plm<double>(v0, v1, v[2 * S], -1.0, pp.theta);
+      }
+      return;
+    }
+  }
+  const R theta = (R)pp.theta;
+  for (int q = 0; q < 8; ++q) {
+    const double *Pq = P + q * T + z;
+    const R v0 = (R)Pq[0], v1 = (R)Pq[S];
+    if (recon == RECON_WENO5) {
+      const R vm2 = (R)Pq[-2 * S], vm1 = (R)Pq[-S], v2 = (R)Pq[2 * S], v3 = (R)Pq[3 * S];
+      ql[q] = weno5<R, true>(vm2, vm1, v0, v1, v2, pp.IS, (R)pp.sz10A);
+      qr[q] = weno5<R, false>(vm1, v0, v1, v2, v3, pp.IS, (R)pp.sz10A);
+    }
+    else if (recon == RECON_PLM) {
+      ql[q] = plm<R>((R)Pq[-S], v0, v1, R(+1.0), theta);
+      qr[q] = plm<R>(v0, v1, (R)Pq[2 * S], R(-1.0), theta);
+    }
+    else {
+      ql[q] = v0;
+      qr[q] = v1;
+    }
+  }
 }
 
 /* ---------------------------------------------------------------------------
@@ -1253,13 +1500,13 @@ struct FluxCounters {
  * nested c2p, after which the outer U and F are dead; only the primitive states are
  * kept (to rebuild the flux side at the end and for the HLLC fallback, which averages
  * the normal field exactly as here, riemann_hllc-rmhd.cpp:60).
- * FAST = true is the common path alone: the nested c2p from the average state and the
+ * FAST = true (the FP32 sweeps; FP64 has riemann_hlld_lean) is the common path alone: the nested c2p from the average state and the
  * first Newton attempt from EstimateSolution(0), or with a small normal field the flux at
  * EstimateSolution(1). Anything else (an invalid state, the c2p cascade, attempts 2 and
  * 3, the HLLC fallback) returns kHlldDefer without writing f; the caller hands the
  * interface to the full solver, which then takes the same steps up to that point and
  * gives the same result. */
-constexpr int kHlldDefer = 100;   // FAST mode: the interface needs the full solver
+constexpr int kHlldDefer = 100;   // common path: the interface needs the full solver
 
 template <typename R, int DIM, bool FAST = false>
 __device__ __forceinline__ int riemann_hlld(const R *pl, const R *pr, R *f, R gamma, double pfloor, R &lam,
@@ -1446,6 +1693,425 @@ __device__ __forceinline__ int riemann_hlld(const R *pl, const R *pr, R *f, R ga
   ql[Pm::B2] = Pl[By]; qr[Pm::B2] = Pr[By];
   ql[Pm::B3] = Pl[Bz]; qr[Pm::B3] = Pr[Bz];
   return riemann_hllc<R, DIM>(ql, qr, f, gamma, lam);
+}
+
+/* ---------------------------------------------------------------------------
+ * HLLD, the common path of the sweeps (one interface per lane)
+ *
+ * The steps of riemann_hlld that nearly every interface takes: the nested c2p from the average
+ * state, the first Newton attempt from EstimateSolution(0) (with a small normal field the
+ * flux at EstimateSolution(1)), and the flux. Whatever leaves them (an invalid state, a
+ * failed nested c2p, a Newton solve that does not settle, a rejected fan) returns
+ * kHlldDefer, and the caller hands the interface to the full FP64 solver.
+ *
+ * What it computes is the reference's flux to round-off; what it leaves out are operations
+ * whose result is already known, since the sweep is bound by instruction issue (its HBM
+ * traffic is the algorithmic minimum). Against the full solver's common branches in the same
+ * kernel: 2 600-3 200 VALU instructions per wave of interfaces where there were 5 300-5 800,
+ * 166 VGPRs where there were 213 (3 waves per SIMD, not 2), and at 256^3 WENO5 1.48-1.55 ms
+ * a sweep where it took 3.2-3.7 (82 % of the issue rate, from 67 %).
+ *   - Conserved state, flux and speeds of a side come from one pass over its primitives with
+ *     one reciprocal square root; the energy flux is the normal momentum.
+ *   - Of U and F only the jumps across the fast waves (eqn 12), L = am Ul - Fl and
+ *     R = ap Ur - Fr, are kept: the HLL state and flux are (R - L)/(ap - am) and
+ *     (am R - ap L)/(ap - am), and the flux behind the left fast wave is am U - L.
+ *   - The nested c2p only starts the p* solve: it stops at a relative step of 1e-6 (1e-12
+ *     left of the error, Newton being quadratic), and the total pressure follows from (Z, W)
+ *     without the velocity: p + (B^2/W^2 + (B.S)^2/Z^2)/2.
+ *   - In the fan everything that does not depend on p is formed once, pairs of reciprocals
+ *     share one division in FP64, and the residual needs the numerators of the contact field
+ *     only.
+ *   - The derivative is a one-sided difference from the residual at hand, and the last
+ *     Newton step (from a residual within the tolerance) takes the derivative of the step
+ *     before it, if the residual fell by 20 times (so the derivative changed by less than a
+ *     tenth) and the step is below 1e-11 of p (so what a tenth of it changes is round-off):
+ *     four evaluations of the fan per interface where centred differences take seven.
+ * ------------------------------------------------------------------------- */
+/* One side of an interface in the x-normal frame: D, E = tau + D, S, the fluxes and the
+ * fast speeds (Mara/rmhd.cpp:133-265). False for a state that prim_to_cons would refuse or
+ * whose speeds need the general cubic. */
+struct FastSide {
+  double D, E, S[3], B[3];
+  double FD, FS[3], FB2, FB3;      // the energy flux is S[0], the normal field's is zero
+  double ep, em;
+  __device__ __forceinline__ bool set(const double *P, double gamma, double g1, double igamma)
+  {
+    const double V2 = P[vx]*P[vx] + P[vy]*P[vy] + P[vz]*P[vz];
+    const double B2 = P[Bx]*P[Bx] + P[By]*P[By] + P[Bz]*P[Bz];
+    const double Bv = P[Bx]*P[vx] + P[By]*P[vy] + P[Bz]*P[vz];
+    const double om = 1.0 - V2;
+    if (!(om > 0.0)) return false;
+    const double W = rsqrt_normal(om), iW = om*W, W2 = W*W;
+    const double b0 = W*Bv;
+    const double b2 = (B2 + b0*b0)*om;
+    const double bx = P[Bx]*iW + b0*P[vx], by = P[By]*iW + b0*P[vy], bz = P[Bz]*iW + b0*P[vz];
+    const double rhoh = P[rho] + g1*P[pre];
+    const double wW2 = (rhoh + b2)*W2;
+    const double pt = P[pre] + 0.5*b2;
+    D = P[rho]*W;
+    E = wW2 - pt - b0*b0;
+    // NaN in any primitive reaches E
+    if (!(D >= 0.0) || !(E - D >= 0.0)) return false;
+    S[0] = wW2*P[vx] - b0*bx;
+    S[1] = wW2*P[vy] - b0*by;
+    S[2] = wW2*P[vz] - b0*bz;
+    B[0] = P[Bx]; B[1] = P[By]; B[2] = P[Bz];
+    const double v = P[vx], BiW = P[Bx]*iW;
+    FD = D*v;
+    FS[0] = S[0]*v - bx*BiW + pt;
+    FS[1] = S[1]*v - by*BiW;
+    FS[2] = S[2]*v - bz*BiW;
+    FB2 = v*P[By] - P[vy]*P[Bx];
+    FB3 = v*P[Bz] - P[vz]*P[Bx];
+
+    const double ics2 = rhoh*igamma*rcp_normal(P[pre]);
+    const double K = rhoh*(ics2 - 1.0)*(W2*W2);
+    const double L = -(rhoh + b2*ics2)*W2;
+    const double v2 = v*v, v3 = v*v2, v4 = v*v3;
+    const double A4 = K - L - b0*b0;
+    const double A3 = -4.0*K*v + L*v*2.0 + 2.0*b0*bx;
+    const double A2 = 6.0*K*v2 + L*(1.0 - v2) + b0*b0 - bx*bx;
+    const double A1 = -4.0*K*v3 - L*v*2.0 - 2.0*b0*bx;
+    const double A0 = K*v4 + L*v2 + bx*bx;
+    int nr;
+    quartic_extremes_lean<false>(A4, A3, A2, A1, A0, ep, em, nr);
+    if (nr == 0) return false;
+    if (dfabs(ep) > 1.0 || dfabs(em) > 1.0) {
+      ep = 1.0;
+      em = -1.0;
+    }
+    return true;
+  }
+};
+
+/* One side's part of the fan as a function of the total pressure p (FillInnerWaveStates,
+ * riemann_hlld-rmhd.cpp:321-384), with its p-independent terms. J: the jump across its fast
+ * wave of speed lam. */
+struct FanSide {
+  double lam, D, E, m0, m1, m2, B0, B1, B2;     // the jump (eqn 12)
+  double A0, A1, G, K1, a, b, c, c3, c4;        // p-independent terms
+  __device__ __forceinline__ void set(const FastSide &s, double l)
+  {
+    lam = l;
+    D = l*s.D - s.FD;
+    E = l*s.E - s.S[0];
+    m0 = l*s.S[0] - s.FS[0];
+    m1 = l*s.S[1] - s.FS[1];
+    m2 = l*s.S[2] - s.FS[2];
+    B0 = l*s.B[0];
+    B1 = l*s.B[1] - s.FB2;
+    B2 = l*s.B[2] - s.FB3;
+  }
+  __device__ __forceinline__ void constants(double Bn, double Bn2)
+  {
+    A0 = m0 - lam*E;
+    A1 = 1.0 - lam*lam;
+    G = B1*B1 + B2*B2;
+    const double C = B1*m1 + B2*m2;
+    K1 = Bn2*A1 - G;
+    a = lam*Bn2;
+    b = Bn*C;
+    c = lam*b;
+    const double CB = C + Bn*(lam*m0 - E);
+    c3 = B1*CB;
+    c4 = B2*CB;
+  }
+  // velocity and field behind the fast wave, 1/(lam - v0), total enthalpy and the
+  // denominator of K, at p
+  __device__ __forceinline__ void fill(double p, double Bn, double Bn2, double sgn, double (&v)[3], double (&B)[3], double &id, double &w, double &eta, double &den) const
+  {
+    const double A = p*A1 + A0, AG = A + G, Q = K1 - A;
+    const double lpE = lam*p + E;
+    double X = (A*a + b) - AG*lpE;
+    if (dfabs(X) < Tol<double>::X_floor) X = Tol<double>::X_floor;
+    const double n0 = (A*Bn2 + c) - AG*(p + m0);
+    // 1/X and 1/(lam - v0) = X/(lam X - n0) from one reciprocal
+    const double Y = lam*X - n0;
+    const double r = rcp_normal(X*Y);
+    const double iX = r*Y;
+    id = (r*X)*X;
+    v[0] = n0*iX;
+    v[1] = (Q*m1 + c3)*iX;
+    v[2] = (Q*m2 + c4)*iX;
+    B[0] = (B0 - Bn*v[0])*id;
+    B[1] = (B1 - Bn*v[1])*id;
+    B[2] = (B2 - Bn*v[2])*id;
+    w = dfabs(p + (E - (v[0]*m0 + v[1]*m1 + v[2]*m2))*id);
+    eta = sgn*sqrt_lean(w);
+    den = lpE + Bn*eta;
+  }
+};
+
+__device__ __forceinline__ void rcp_pair(double x, double y, double &ix, double &iy)
+{
+  const double r = rcp_normal(x*y);
+  ix = r*y;
+  iy = r*x;
+}
+
+/* `store(q, f)` receives the flux of conserved field q in the lab frame */
+template <int DIM, typename Store>
+__device__ __forceinline__ int riemann_hlld_lean(const double *pl, const double *pr, const PhysParams &pp, double &lam_max,
+                                                 FluxCounters &cnt, Store store)
+{
+  using T = Tol<double>;
+  using Pm = Perm<DIM>;
+  const double gamma = pp.gamma, g1 = pp.g1, gamf = pp.gamf;
+  const double Bn = 0.5*(pl[Pm::B1] + pr[Pm::B1]);
+  const double Bn2 = Bn*Bn;
+  auto out = [&](double fD, double fE, double f0, double f1, double f2, double g0, double g1_, double g2) {
+    store((int)ddd, fD);
+    store((int)tau, fE - fD);
+    store(Pm::S1, f0);
+    store(Pm::S2, f1);
+    store(Pm::S3, f2);
+    store(Pm::B1, g0);
+    store(Pm::B2, g1_);
+    store(Pm::B3, g2);
+  };
+
+  FanSide L, Rt;
+  double Z, W;                       // the nested c2p's start: the average of the two states
+  bool supersonic;
+  {
+    FastSide sl, sr;
+    {
+      const double Pl[8] = { pl[rho], pl[pre], pl[Pm::v1], pl[Pm::v2], pl[Pm::v3], Bn, pl[Pm::B2], pl[Pm::B3] };
+      const double Pr[8] = { pr[rho], pr[pre], pr[Pm::v1], pr[Pm::v2], pr[Pm::v3], Bn, pr[Pm::B2], pr[Pm::B3] };
+      {
+        const double ax = Pl[vx] + Pr[vx], ay = Pl[vy] + Pr[vy], az = Pl[vz] + Pr[vz];
+        const double om = 1.0 - 0.25*(ax*ax + ay*ay + az*az);
+        W = rsqrt_normal(om);
+        Z = (0.5*((Pl[rho] + Pr[rho]) + g1*(Pl[pre] + Pr[pre])))*(W*W);
+      }
+      if (!sl.set(Pl, gamma, g1, pp.igamma)) return kHlldDefer;
+      if (!sr.set(Pr, gamma, g1, pp.igamma)) return kHlldDefer;
+    }
+    const double am = (sl.em < sr.em) ? sl.em : sr.em;
+    const double ap = (sl.ep > sr.ep) ? sl.ep : sr.ep;
+    note_lambda(lam_max, am, ap);
+    L.set(sl, am);
+    Rt.set(sr, ap);
+    // both fast waves on one side: the flux is that side's own, stored now so that its state
+    // need not be kept (the solve below still decides whether HLLD is counted a success)
+    supersonic = 0.0 <= am || !(0.0 <= ap);
+    if (supersonic) {
+      const bool l = 0.0 <= am;
+      out(l ? sl.FD : sr.FD, l ? sl.S[0] : sr.S[0], l ? sl.FS[0] : sr.FS[0], l ? sl.FS[1] : sr.FS[1],
+          l ? sl.FS[2] : sr.FS[2], 0.0, l ? sl.FB2 : sr.FB2, l ? sl.FB3 : sr.FB3);
+    }
+  }
+
+  // EstimateSolution(0) by anton2dzw (c2p_anton2dzw) on the HLL state, :208-218,543-555
+  const double ida = rcp_normal(Rt.lam - L.lam);
+  const bool small_bn = dfabs(Bn) < T::small_bn;
+  double p;
+  {
+    const double D = (Rt.D - L.D)*ida, E = (Rt.E - L.E)*ida, tau_ = E - D;
+    const double S0 = (Rt.m0 - L.m0)*ida, S1 = (Rt.m1 - L.m1)*ida, S2v = (Rt.m2 - L.m2)*ida;
+    const double b1 = (Rt.B1 - L.B1)*ida, b2 = (Rt.B2 - L.B2)*ida;
+    const double S2 = S0*S0 + S1*S1 + S2v*S2v;
+    const double B2 = Bn2 + b1*b1 + b2*b2;
+    const double BS = Bn*S0 + b1*S1 + b2*S2v, BS2 = BS*BS;
+    if (!(D >= 0.0) || !(tau_ >= 0.0)) return kHlldDefer;
+    double iZ, iW;
+    rcp_pair(Z, W, iZ, iW);
+    double error;
+    int it = 0;
+    do {
+      const double Z3 = Z*Z*Z, W2 = W*W;
+      const double iZ2 = iZ*iZ, iZ3 = iZ2*iZ, iW2 = iW*iW, iW3 = iW2*iW;
+      const double ZB = Z + B2, gW3 = gamf*iW3;
+      const double Pre = gamf*(Z*iW2 - D*iW);
+      const double df0dZ = 2.0*ZB*(BS2*W2 + (W2 - 1.0)*Z3)*(iW2*iZ3);
+      const double df0dW = 2.0*(ZB*ZB)*iW3;
+      const double df1dZ = 1.0 + BS2*iZ3 - gamf*iW2;
+      const double df1dW = B2*iW3 + (2.0*Z - D*W)*gW3;
+      const double f0 = (ZB*ZB)*(W2 - 1.0)*iW2 - (2.0*Z + B2)*BS2*iZ2 - S2;
+      const double f1 = ZB - Pre - 0.5*(B2*iW2 + BS2*iZ2) - E;
+      const double idet = rcp_normal(df0dZ*df1dW - df0dW*df1dZ);
+      const double dZ = (df0dW*f1 - df1dW*f0)*idet;
+      const double dW = (df1dZ*f0 - df0dZ*f1)*idet;
+      Z = dfabs(Z + dZ);
+      W = W + dW;
+      W = W > 1.0 ? W : 1.0;
+      rcp_pair(Z, W, iZ, iW);
+      error = dfabs(dZ*iZ) + dfabs(dW*iW);
+      ++it;
+      if (it == T::nested_max_it) { cnt.c2p_iters += it; return kHlldDefer; }
+    } while (error > T::nested_step);
+    cnt.c2p_iters += it;
+    const double iW2 = iW*iW;
+    double pg = gamf*(Z*iW2 - D*iW);
+    if (pg < pp.pfloor && pp.pfloor > 0.0) pg = pp.pfloor;
+    if (!(pg >= 0.0)) return kHlldDefer;
+    p = pg + 0.5*(B2*iW2 + BS2*(iZ*iZ));
+  }
+  if (small_bn) {
+    // EstimateSolution(1), eqn (55), :558-574
+    const double Uh = (Rt.E - L.E)*ida, Us = (Rt.m0 - L.m0)*ida;
+    const double Fh = (L.lam*Rt.E - Rt.lam*L.E)*ida, Fs = (L.lam*Rt.m0 - Rt.lam*L.m0)*ida;
+    const double bb = Uh - Fs, cc = Fh*Us - Uh*Fs;
+    const double rt = sqrt_lean(bb*bb - 4.0*cc);
+    const double p1 = dfabs(0.5*(rt - bb)), p2 = dfabs(0.5*(bb + rt));
+    p = (p1 < p2) ? p1 : p2;
+  }
+  L.constants(Bn, Bn2);
+  Rt.constants(Bn, Bn2);
+
+  // NewtonRaphesonSolver(15, 1e-12)::Solve (Mara/nrsolver.cpp:20-83) on HlldEquation48, then
+  // the fan at the solution: one copy of the fan in a loop over its evaluations
+  const double sg = double((Bn > 0.0) - (Bn < 0.0));
+  double vL[3], vR[3], bL[3], bR[3], KL[3], KR[3], N[3], idL, idR, wL, wR, etaL, etaR, delK;
+  {
+    enum { RESIDUAL, DERIVATIVE, SOLUTION };
+    int mode = small_bn ? SOLUTION : RESIDUAL;
+    int it = 0, worse = 0;
+    bool have = false;
+    double pe = p, y0 = 0.0, Gd = 0.0, eps = 0.0;
+    for (;;) {
+      double denL, denR, iL, iR;
+      L.fill(pe, Bn, Bn2, -sg, vL, bL, idL, wL, etaL, denL);
+      Rt.fill(pe, Bn, Bn2, sg, vR, bR, idR, wR, etaR, denR);
+      rcp_pair(denL, denR, iL, iR);
+      KL[0] = (L.m0 + pe + L.B0*etaL)*iL;
+      KL[1] = (L.m1 + L.B1*etaL)*iL;
+      KL[2] = (L.m2 + L.B2*etaL)*iL;
+      KR[0] = (Rt.m0 + pe + Rt.B0*etaR)*iR;
+      KR[1] = (Rt.m1 + Rt.B1*etaR)*iR;
+      KR[2] = (Rt.m2 + Rt.B2*etaR)*iR;
+      delK = KR[0] - KL[0];
+      const double kr = KR[0] - vR[0], kl = KL[0] - vL[0];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) N[k] = (bR[k]*kr + bR[0]*vR[k]) - (bL[k]*kl + bL[0]*vL[k]);
+      if (mode == SOLUTION) break;
+      // HlldEquation48::Function, :386-415, with N = delK Bc
+      double y;
+      {
+        const double dl = etaL*delK - (KL[0]*N[0] + KL[1]*N[1] + KL[2]*N[2]);
+        const double dr = etaR*delK - (KR[0]*N[0] + KR[1]*N[1] + KR[2]*N[2]);
+        double il, ir;
+        rcp_pair(dl, dr, il, ir);
+        const double yl = (1.0 - (KL[0]*KL[0] + KL[1]*KL[1] + KL[2]*KL[2]))*il;
+        const double yr = (1.0 - (KR[0]*KR[0] + KR[1]*KR[1] + KR[2]*KR[2]))*ir;
+        const double ad = dfabs(delK);
+        y = delK - N[0]*(yr - yl);
+        if (dfabs(N[0]) < T::small_Bc*ad) y = delK;
+        if (ad < T::small_delK) y = 0.0;
+      }
+      if (mode == RESIDUAL) {
+        const double ay = dfabs(y);
+        const double dx = Gd*y;
+        if (have && ay <= T::newton_ftol && ay <= 0.05*dfabs(y0) && dfabs(dx) <= T::reuse_step*dfabs(p)) {
+          p -= dx;
+          pe = p;
+          mode = SOLUTION;
+        }
+        else {
+          y0 = y;
+          pe = p + T::fd_dp;
+          mode = DERIVATIVE;
+        }
+      }
+      else {
+        Gd = (pe - p)*rcp(y - y0);
+        p -= Gd*y0;
+        const double last = eps;
+        eps = dfabs(y0);
+        worse += (eps > last);
+        if (worse >= 10 || it == T::newton_fast_max_it || is_nan(eps)) { cnt.newton_iters += it; return kHlldDefer; }
+        mode = SOLUTION;
+        if (eps > T::newton_ftol) {
+          ++it;
+          have = true;
+          mode = RESIDUAL;
+        }
+        pe = p;
+      }
+    }
+    cnt.newton_iters += it;
+    p = pe;
+  }
+
+  // ReconstructSolution, :417-538, for s = 0
+  double Bc[3];
+  {
+    const bool zero = dfabs(delK) < T::small_delK;
+    const double idK = zero ? 0.0 : rcp_normal(delK);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) Bc[k] = N[k]*idK;
+  }
+  double sL, sR;                    // c = K - s Bc on each side (c = a where the denominator is small)
+  bool aL, aR;
+  {
+    const double dL = etaL - (KL[0]*Bc[0] + KL[1]*Bc[1] + KL[2]*Bc[2]);
+    const double dR = etaR - (KR[0]*Bc[0] + KR[1]*Bc[1] + KR[2]*Bc[2]);
+    aL = dfabs(dL) < T::small_denom_c;
+    aR = dfabs(dR) < T::small_denom_c;
+    double iL, iR;
+    rcp_pair(aL ? 1.0 : dL, aR ? 1.0 : dR, iL, iR);
+    sL = (1.0 - (KL[0]*KL[0] + KL[1]*KL[1] + KL[2]*KL[2]))*iL;
+    sR = (1.0 - (KR[0]*KR[0] + KR[1]*KR[1] + KR[2]*KR[2]))*iR;
+  }
+  const double cL0 = aL ? vL[0] : KL[0] - Bc[0]*sL, cR0 = aR ? vR[0] : KR[0] - Bc[0]*sR;
+  {
+    const double TOL = T::tol54;
+    const double lmaL = KL[0], lmaR = KR[0];
+    if (p < 0.0) return kHlldDefer;
+    if (lmaL < -1.0 || lmaR > 1.0 || dfabs(cR0) > 1.0) return kHlldDefer;
+    if (!((wL > p) && (vL[0] > L.lam - TOL) && (cL0 > lmaL - TOL))) return kHlldDefer;
+    if (!((wR > p) && (vR[0] < Rt.lam + TOL) && (cR0 < lmaR + TOL))) return kHlldDefer;
+    if (dfabs(cR0 - cL0) > T::contact) return kHlldDefer;
+  }
+  if (!supersonic) {
+    // the first region of the reference's chain (:518-524) whose upper speed bounds s = 0;
+    // left of the contact up to region 2
+    const bool left = 0.0 <= KL[0] || 0.0 <= cR0;
+    const bool outer = left ? 0.0 <= KL[0] : !(0.0 <= KR[0]);   // between the fast and the Alfven wave
+    const double lam = left ? L.lam : Rt.lam;
+    const double v0 = left ? vL[0] : vR[0], v1 = left ? vL[1] : vR[1], v2 = left ? vL[2] : vR[2];
+    const double B0 = left ? bL[0] : bR[0], B1 = left ? bL[1] : bR[1], B2 = left ? bL[2] : bR[2];
+    const double jD = left ? L.D : Rt.D, jE = left ? L.E : Rt.E;
+    const double id = left ? idL : idR;
+    if (dfabs(lam - v0) < T::small_denom) return kHlldDefer;      // the outer state itself, :456
+    // state behind the fast wave, :455-484, and the flux lam U - J there
+    const double vB = v0*B0 + v1*B1 + v2*B2;
+    const double aD = jD*id;
+    const double aE = (jE + p*v0 - vB*B0)*id;
+    const double h = aE + p;
+    const double a0 = h*v0 - vB*B0, a1 = h*v1 - vB*B1, a2 = h*v2 - vB*B2;
+    double fD = lam*aD - jD, fE = lam*aE - jE;
+    double f0 = lam*a0 - (left ? L.m0 : Rt.m0), f1 = lam*a1 - (left ? L.m1 : Rt.m1), f2 = lam*a2 - (left ? L.m2 : Rt.m2);
+    double h0 = lam*B0 - (left ? L.B0 : Rt.B0), h1 = lam*B1 - (left ? L.B1 : Rt.B1), h2 = lam*B2 - (left ? L.B2 : Rt.B2);
+    if (!outer) {
+      // the state between the Alfven wave and the contact, :486-516
+      const double lma = left ? KL[0] : KR[0];
+      const bool a = left ? aL : aR;
+      const double s = left ? sL : sR;
+      const double c0 = left ? cL0 : cR0;
+      const double c1 = a ? v1 : (left ? KL[1] : KR[1]) - Bc[1]*s;
+      const double c2 = a ? v2 : (left ? KL[2] : KR[2]) - Bc[2]*s;
+      const double dn = lma - cR0;
+      if (!(dfabs(dn) < T::small_denom)) {
+        const double idn = rcp_normal(dn);
+        const double vBc = c0*Bc[0] + c1*Bc[1] + c2*Bc[2];
+        const double cD = aD*(lma - v0)*idn;
+        const double cE = (lma*aE - a0 + p*cR0 - vBc*Bc[0])*idn;
+        const double hc = cE + p;
+        fD += lma*(cD - aD);
+        fE += lma*(cE - aE);
+        f0 += lma*((hc*c0 - vBc*Bc[0]) - a0);
+        f1 += lma*((hc*c1 - vBc*Bc[1]) - a1);
+        f2 += lma*((hc*c2 - vBc*Bc[2]) - a2);
+        h0 += lma*(Bc[0] - B0);
+        h1 += lma*(Bc[1] - B1);
+        h2 += lma*(Bc[2] - B2);
+      }
+    }
+    out(fD, fE, f0, f1, f2, h0, h1, h2);
+  }
+  ++cnt.hlld_ok;
+  return 0;
 }
 
 }  // namespace maragpu

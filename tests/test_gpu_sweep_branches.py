@@ -1,0 +1,68 @@
+"""The FP64 HLLD sweep where its common path branches, against the oracle: both fast waves on
+one side of the interface (the flux of that side, in either direction), the reconstruction
+methods it dispatches on, and grids whose sweeps end inside a block.
+
+Tolerances: error counts identical, HLLD counts within 2. The common path takes the
+reference's formulas in another order, so it agrees to round-off; at these flow speeds
+(W > 2) round-off alone moves the reference's quartic roots, so MaxLambda and the states are
+held to the plain form's tolerances (1e-12; 1e-10 in L1, 1e-7 at any zone) or, where that is
+more, to 4x of how far the oracle's own run moves under 1-ulp noise on the initial state.
+"""
+import numpy as np
+import pytest
+
+from oracle.oracle import Setup, synchronize
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("extrap,IS,flow,N", [
+    ("weno5", "js96", (0.95, 0.0, 0.0), (13, 18, 11)),
+    ("weno5", "js96", (0.0, -0.9, 0.3), (9, 14, 22)),
+    ("weno5", "sz10", (0.2, 0.1, 0.93), (12, 10, 19)),
+    ("plm", "js96", (-0.93, 0.2, 0.0), (17, 8, 15)),
+    ("pcm", "js96", (0.0, 0.0, -0.95), (10, 11, 33)),
+])
+def test_supersonic_sweeps(gpu, oracle_lib, extrap, IS, flow, N):
+    rng = np.random.default_rng(sum(N))
+    x = [2 * np.pi * (np.arange(n) + 0.5) / n for n in N]
+    X, Y, Z = np.meshgrid(*x, indexing="ij")
+    P = np.empty(tuple(n + 6 for n in N) + (8,))
+    it = (slice(3, -3),) * 3
+    wave = [np.sin(X + p) * np.cos(Y + q) + np.sin(Z + r) for p, q, r in rng.uniform(0, 6, (8, 3))]
+    P[it + (0,)] = 1.0 + 0.2 * wave[0]
+    P[it + (1,)] = 0.2 * (1.0 + 0.2 * wave[1])
+    for d in range(3):
+        P[it + (2 + d,)] = flow[d] + 0.01 * wave[2 + d]
+        P[it + (5 + d,)] = (0.2, 0.15, 0.25)[d] + 0.02 * wave[5 + d]
+    P = synchronize(P, 3)
+    s = Setup(N=N, extrap=extrap, IS=IS, riemann="hlld", advance="rk2")
+    def march(P0):
+        so = oracle_lib.solver(s)
+        Po, dt, out = P0.copy(), 0.0, []
+        for _ in range(3):
+            eo, sto = so.advance(Po, dt)
+            out.append((eo, sto.hlld_success, sto.max_lambda, dt))
+            dt = so.get_timestep(0.4)
+        return Po, out
+
+    Po, ref = march(P)
+    lam_tol = np.full(3, 1e-12)
+    L1_tol, max_tol = np.full(8, 1e-10), np.full(8, 1e-7)
+    L1 = lambda A: np.abs(A - Po).sum(axis=(0, 1, 2)) / np.abs(Po).sum(axis=(0, 1, 2))  # noqa: E731
+    worst = lambda A: np.abs(A - Po).max(axis=(0, 1, 2)) / np.abs(Po).max(axis=(0, 1, 2))  # noqa: E731
+    for _ in range(8):
+        Pn, noisy = march(P * (1 + 2.3e-16 * rng.choice([-1, 0, 1], size=P.shape)))
+        lam_tol = np.maximum(lam_tol, [4 * abs(a[2] - b[2]) / b[2] for a, b in zip(noisy, ref)])
+        L1_tol, max_tol = np.maximum(L1_tol, 4 * L1(Pn)), np.maximum(max_tol, 4 * worst(Pn))
+
+    ctx = gpu.Context(gpu.make_config(N=N, extrap=extrap, IS=IS, riemann="hlld", advance="rk2"))
+    ctx.upload(P)
+    for (eo, ok, lam, dt), tol in zip(ref, lam_tol):
+        eg, stg = ctx.advance(dt)
+        assert eo == eg == 0
+        assert abs(stg.max_lambda - lam) <= tol * lam
+        assert abs(stg.hlld_success - ok) <= 2
+    Pg = ctx.download()
+    assert (L1(Pg) <= L1_tol).all()
+    assert (worst(Pg) <= max_tol).all()
