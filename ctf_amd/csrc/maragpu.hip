@@ -56,7 +56,9 @@ template <typename R> constexpr int kFluxBlock = sizeof(R) == 4 ? 256 : 64;
 // spills), FP32 at 5 (92 VGPRs; at 4 waves 9 % slower)
 constexpr int kFastFluxWaves64 = 3;
 constexpr int kFastFluxWaves32 = 5;
-constexpr int kRedoBlocks = 1024;    // grid of k_flux_redo (a grid-stride loop over its queue)
+// grid of the redo kernels (a grid-stride loop over the queue): one block per CU, all that their
+// registers let be resident
+constexpr int kRedoBlocks = 256;
 
 /* Device-side counters of one step; reduced per block, then atomically. */
 struct DevStats {
@@ -80,16 +82,23 @@ struct DevStats {
   unsigned long long ctu_failed[4][4]; // plm-muscl: failed checks per stage and abort point
 };
 
-/* Interfaces of an HLLD sweep handed to the full FP64 solver (k_flux_redo) before the
+/* Interfaces of the HLLD sweeps handed to the full FP64 solver (k_flux_redo) before the
  * update reads the fluxes: in the mixed form those whose FP32 HLLD solve failed, in the
- * plain form those outside the common path of the lean sweep (k_flux_hlld_fast). */
+ * plain form those outside the common path of the lean sweep (k_flux_hlld_fast). One list
+ * per axis. */
 struct RedoQueue {
-  unsigned int *count;     // device counter, cleared before each sweep
-  unsigned int cap;        // slots
-  unsigned int *z;         // device slots: interface index z (left zone; T < 2^32)
-  uint4 *part;             // per wave of the HLLD sweep: its counters, summed by the redo
-  unsigned int part_cap;   // waves
+  unsigned int *count;     // device counters, one per axis; cleared before the sweeps (clear_queue)
+  unsigned int cap;        // slots of an axis
+  unsigned int *z;         // device slots, cap per axis: interface index z (left zone; T < 2^32)
+  uint4 *part;             // per wave of the sweeps: its counters, summed by the redo
 };
+
+/* The kernel before a stage's sweeps (the step start, or the previous stage's update) clears
+ * the queue's counts: whoever read them has finished, and the sweeps follow in stream order. */
+__device__ __forceinline__ void clear_queue(unsigned int *count)
+{
+  if (count && blockIdx.x == 0 && threadIdx.x < 3) count[threadIdx.x] = 0u;
+}
 
 struct GridDesc {
   int N[3], Ng, n[3];
@@ -209,19 +218,19 @@ __device__ __forceinline__ void sweep_counters_wave(double lam, bool success, un
 
 /* Appends z for every lane of the wave with push set, with one atomic per wave; every
  * lane of the wave calls it. Returns false on a lane whose slot lies past the capacity. */
-__device__ __forceinline__ bool queue_push(const RedoQueue &rq, bool push, long z)
+__device__ __forceinline__ bool queue_push(const RedoQueue &rq, int axis, bool push, long z)
 {
   const unsigned long long m = __ballot(push);
   if (m == 0ull) return true;
   const int lane = (int)(threadIdx.x & 63);
   const int leader = __ffsll((unsigned long long)m) - 1;
   unsigned int base = 0u;
-  if (lane == leader) base = atomicAdd(rq.count, (unsigned int)__popcll(m));
+  if (lane == leader) base = atomicAdd(rq.count + axis, (unsigned int)__popcll(m));
   base = (unsigned int)__shfl((int)base, leader);
   if (!push) return true;
   const unsigned int k = base + (unsigned int)__popcll(m & ((1ull << lane) - 1ull));
   if (k >= rq.cap) return false;
-  rq.z[k] = (unsigned int)z;
+  rq.z[(size_t)axis * rq.cap + k] = (unsigned int)z;
   return true;
 }
 
@@ -487,16 +496,17 @@ __device__ __forceinline__ int riemann_dispatch(int solver, const R *pl, const R
   return riemann_hll<R, DIM>(pl, pr, F, gamma, lam);
 }
 
-/* One interface z | z+S of the sweep along DIM: reconstruction from the 6-point stencil,
+/* One interface z | z+S of the sweep along `axis`: reconstruction from the 6-point stencil,
  * the Riemann solve, and the retry with the zone-centred states of the two neighbours
- * (Mara/plm-split.cpp:51-71). Returns the error of the last attempt (flux 0 then). */
-template <typename R, int DIM, int SOLVER>
-__device__ __forceinline__ int interface_flux(const double *__restrict__ P, long T, long S, long z, int recon,
+ * (Mara/plm-split.cpp:51-71). F in the axis's frame. Returns the error of the last attempt
+ * (flux 0 then). */
+template <typename R, int SOLVER>
+__device__ __forceinline__ int interface_flux(const double *__restrict__ P, long T, long S, int axis, long z, int recon,
                                               const PhysParams &pp, R *F, R &lam, FluxCounters &fc,
                                               int &retried)
 {
   R ql[8], qr[8];
-  reconstruct_states<R, false>(P, T, S, z, recon, pp, ql, qr);
+  reconstruct_states<R, false>(P, T, S, axis, z, recon, pp, ql, qr);
   int err = 1;
   retried = 0;
   // one call site: the reconstructed states, then the zone-centred states
@@ -506,11 +516,12 @@ __device__ __forceinline__ int interface_flux(const double *__restrict__ P, long
       retried = 1;
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
-        ql[q] = (R)P[q * T + z];
-        qr[q] = (R)P[q * T + z + S];
+        const double *v = P + axis_plane(q, axis) * T + z;
+        ql[q] = (R)v[0];
+        qr[q] = (R)v[S];
       }
     }
-    err = riemann_dispatch<R, DIM>(SOLVER, ql, qr, F, (R)pp.gamma, pp.pfloor, lam, fc);
+    err = riemann_dispatch<R, 1>(SOLVER, ql, qr, F, (R)pp.gamma, pp.pfloor, lam, fc);
   }
   if (err) {
 #pragma unroll
@@ -522,75 +533,32 @@ __device__ __forceinline__ int interface_flux(const double *__restrict__ P, long
 /* The common path of an HLLD interface, the flux written to its planes: reconstruction and
  * riemann_hlld_lean in FP64, riemann_hlld in FAST mode in FP32. Returns kHlldDefer where the
  * full solver is needed. */
-template <typename R, int DIM>
+template <typename R>
 __device__ __forceinline__ int interface_flux_fast(const double *__restrict__ P, R *__restrict__ Fout, long T, long S,
-                                                   long z, int recon, const PhysParams &pp, R &lam, FluxCounters &fc)
+                                                   int axis, long z, int recon, const PhysParams &pp, R &lam,
+                                                   FluxCounters &fc)
 {
   R ql[8], qr[8];
-  reconstruct_states<R, sizeof(R) == 8>(P, T, S, z, recon, pp, ql, qr);
+  reconstruct_states<R, sizeof(R) == 8>(P, T, S, axis, z, recon, pp, ql, qr);
   if constexpr (sizeof(R) == 8)
-    return riemann_hlld_lean<DIM>(ql, qr, pp, lam, fc, [&](int q, double f) { Fout[q * T + z] = f; });
+    return riemann_hlld_lean<1>(ql, qr, pp, lam, fc,
+                                [&](int q, double f) { Fout[axis_plane(q, axis) * T + z] = f; });
   else {
     R F[8];
-    const int rc = riemann_hlld<R, DIM, true>(ql, qr, F, (R)pp.gamma, pp.pfloor, lam, fc);
+    const int rc = riemann_hlld<R, 1, true>(ql, qr, F, (R)pp.gamma, pp.pfloor, lam, fc);
     if (rc == 0) {
 #pragma unroll
-      for (int q = 0; q < 8; ++q) Fout[q * T + z] = F[q];
+      for (int q = 0; q < 8; ++q) Fout[axis_plane(q, axis) * T + z] = F[q];
     }
     return rc;
   }
-}
-
-/* Flux sweep along DIM, one thread per interface. With a redo queue (mixed form, HLLD),
- * an interface whose FP32 HLLD solve fell back to HLLC or failed is queued for
- * k_flux_redo instead; its FP32 result stays only if the queue is full. */
-/* Occupancy targets (waves per SIMD) of the full sweep, which runs HLL and HLLC: FP32 at
- * 3, FP64 at 2 even where 256 registers spill (the spill traffic costs less than the
- * latency that a single wave cannot hide). */
-template <typename R, typename FT, int DIM, int SOLVER>
-__global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 3 : 2) void k_flux(const double *__restrict__ P, FT *__restrict__ Fout,
-                                                 GridDesc g, int recon, PhysParams pp, DevStats *st,
-                                                 RedoQueue rq)
-{
-  const long T = g.T;
-  const long S = DIM == 1 ? g.sx : DIM == 2 ? g.sy : g.sz;
-  const long z = 2 * S + (long)blockIdx.x * blockDim.x + threadIdx.x;
-  double lam_out = 0.0;
-  unsigned long long cnt[7] = {0, 0, 0, 0, 0, 0, 0};
-  bool want = false;
-  if (z < T - 3 * S) {
-    R lam = R(0);
-    FluxCounters fc = {0, 0, 0, 0};
-    R F[8];
-    int retried;
-    const int err = interface_flux<R, DIM, SOLVER>(P, T, S, z, recon, pp, F, lam, fc, retried);
-    want = rq.z && (fc.hlld_fail || err);
-#pragma unroll
-    for (int q = 0; q < 8; ++q) Fout[q * T + z] = (FT)F[q];
-    lam_out = (double)lam;
-    cnt[0] = (unsigned long long)fc.hlld_ok;
-    cnt[1] = (unsigned long long)fc.hlld_fail;
-    cnt[2] = (unsigned long long)retried;
-    cnt[3] = err ? 1ull : 0ull;
-    cnt[4] = (unsigned long long)fc.c2p_iters;
-    cnt[5] = (unsigned long long)fc.newton_iters;
-  }
-  if (rq.z) {
-    if (!queue_push(rq, want, z)) cnt[6] = 1;     // full: the FP32 result stays
-    else if (want) cnt[0] = cnt[1] = cnt[2] = cnt[3] = 0;   // counted by the redo
-  }
-  block_max_lambda(lam_out, &st->lam_bits);
-  unsigned long long *const dst[7] = { &st->hlld_success, &st->hlld_failure, &st->retries,
-                                       &st->failures, &st->hlld_c2p_iters, &st->hlld_newton_iters,
-                                       &st->redo_overflow };
-  block_add<7>(cnt, dst);
 }
 
 /* Block order of the HLLD sweeps. The interfaces of a sweep along an axis of stride S are
  * z = a S + r over planes a in [2, T/S - 3) and offsets r in [0, S) (the reference's flat
  * range [2S, T-3S)); an interface's stencil lies at a-3..a+2 in the same column r.
  *   - The hardware hands blocks to the eight XCDs (each with its own L2) round-robin.
- *     Logical block L is given to XCD L / (nb/8): each XCD works through one contiguous
+ *     Of an axis's nb blocks, logical block L is given to XCD L / (nb/8): each XCD works through one contiguous
  *     eighth of the logical order, so the planes a stencil re-reads are in its own L2.
  *   - Along x (S = one i-plane, 4.4 MB of primitives at 256^3) the logical order is tiled:
  *     columns of kSweepChunk tiles of r are swept over every plane before the next
@@ -600,30 +568,65 @@ __global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 3 : 2) void k_flux(const d
  * the chip changes. */
 constexpr long kSweepChunk = 8;
 
-/* Number of blocks of BLK threads of the sweep along DIM. */
-template <int DIM>
-long sweep_blocks(const GridDesc &g, long BLK)
+/* The three axis sweeps of a stage are one launch, z, y, then x: their results do not depend
+ * on the order, a small grid's sweeps run side by side (20x16x24 zones are 215 waves an axis
+ * on 1024 SIMDs: 104 -> 22 us a stage; 64^3: 123 -> 99 us), a large grid's drain only once,
+ * and a step has 12 launches where it had 43 with the copies of the queue's counts and the
+ * waits between two streams. Each axis has its own range of blocks, a multiple of 8 long, so
+ * that the XCD of a block is the same in every range. */
+struct SweepGrid {
+  unsigned first[4];       // first block of the z, y and x ranges, and the end
+  long z0[3], z1[3];       // per axis (x, y, z): the interfaces z | z+S with z in [z0, z1)
+  unsigned planes, tiles;  // along x: planes of interfaces, tiles of a plane
+};
+
+__host__ __device__ __forceinline__ long axis_stride(const GridDesc &g, int axis)
 {
-  const long S = DIM == 1 ? g.sx : DIM == 2 ? g.sy : g.sz;
-  if (DIM == 1) return (g.T / S - 5) * ((S + BLK - 1) / BLK);
-  return (g.T - 5 * S + BLK - 1) / BLK;
+  return axis == 0 ? g.sx : axis == 1 ? g.sy : g.sz;
 }
 
-/* The calling thread's interface z of the sweep; false where it has none. The block
- * arithmetic is 32-bit: it runs once per wave on the scalar unit, and 64-bit divisions
- * there cost several hundred instructions (block counts stay far below 2^31). */
-template <int DIM>
-__device__ __forceinline__ bool sweep_interface(const GridDesc &g, long &z)
+/* The grid of BLK-thread blocks over the interfaces [z0[a], z1[a]) of each axis. */
+inline SweepGrid make_sweep_grid(const GridDesc &g, const long (&z0)[3], const long (&z1)[3], long BLK)
 {
-  const long S = DIM == 1 ? g.sx : DIM == 2 ? g.sy : g.sz;
-  const unsigned BLK = blockDim.x, nb = gridDim.x, b = blockIdx.x;
-  const unsigned q = nb >> 3;
-  const unsigned L = b < 8 * q ? (b & 7) * q + (b >> 3) : b;
-  if constexpr (DIM == 1) {
+  SweepGrid sg;
+  sg.planes = z1[0] > z0[0] ? (unsigned)((z1[0] - z0[0]) / g.sx) : 0u;
+  sg.tiles = (unsigned)((g.sx + BLK - 1) / BLK);
+  sg.first[0] = 0;
+  for (int r = 0; r < 3; ++r) {
+    const int a = 2 - r;
+    sg.z0[a] = z0[a];
+    sg.z1[a] = z1[a];
+    const long nb = a == 0 ? (long)sg.planes * sg.tiles : z1[a] > z0[a] ? (z1[a] - z0[a] + BLK - 1) / BLK : 0;
+    sg.first[r + 1] = sg.first[r] + (unsigned)((nb + 7) / 8 * 8);
+  }
+  return sg;
+}
+
+/* the sweeps' interfaces: the reference's flat range [2S, T - 3S) of each axis */
+inline SweepGrid sweep_grid(const GridDesc &g, long BLK)
+{
+  const long z0[3] = { 2 * g.sx, 2 * g.sy, 2 * g.sz };
+  const long z1[3] = { g.T - 3 * g.sx, g.T - 3 * g.sy, g.T - 3 * g.sz };
+  return make_sweep_grid(g, z0, z1, BLK);
+}
+
+/* The calling thread's axis (uniform over the block) and interface z; false where it has
+ * none. The block arithmetic is 32-bit: it runs once per wave on the scalar unit, and 64-bit
+ * divisions there cost several hundred instructions (block counts stay far below 2^31). */
+__device__ __forceinline__ bool sweep_interface(const GridDesc &g, const SweepGrid &sg, int &axis, long &z)
+{
+  const unsigned BLK = blockDim.x;
+  const int r = blockIdx.x < sg.first[1] ? 0 : blockIdx.x < sg.first[2] ? 1 : 2;
+  axis = 2 - r;
+  const unsigned b0 = r == 0 ? 0u : r == 1 ? sg.first[1] : sg.first[2];
+  const unsigned b1 = r == 0 ? sg.first[1] : r == 1 ? sg.first[2] : sg.first[3];
+  const unsigned b = blockIdx.x - b0;
+  const unsigned L = (b & 7) * ((b1 - b0) >> 3) + (b >> 3);
+  if (axis == 0) {
     constexpr unsigned C = (unsigned)kSweepChunk;
-    const unsigned ntiles = (unsigned)((S + BLK - 1) / BLK);
-    const unsigned nA = (unsigned)(g.T / S - 5);
-    const unsigned full = ntiles / C, per_full = nA * C;
+    const unsigned nA = sg.planes;
+    if (L >= sg.tiles * nA) return false;
+    const unsigned full = sg.tiles / C, per_full = nA * C;
     unsigned a, tile;
     if (L < full * per_full) {
       const unsigned rem = L % per_full;
@@ -631,19 +634,27 @@ __device__ __forceinline__ bool sweep_interface(const GridDesc &g, long &z)
       tile = (L / per_full) * C + rem % C;
     }
     else {
-      const unsigned width = ntiles - full * C, rem = L - full * per_full;
+      const unsigned width = sg.tiles - full * C, rem = L - full * per_full;
       a = rem / width;
       tile = full * C + rem % width;
     }
-    const long r = (long)tile * BLK + threadIdx.x;
-    z = (2 + (long)a) * S + r;
-    return r < S;
+    const long k = (long)tile * BLK + threadIdx.x;
+    z = sg.z0[0] + (long)a * g.sx + k;
+    return k < g.sx;
   }
-  else {
-    z = 2 * S + (long)L * BLK + threadIdx.x;
-    return z < g.T - 3 * S;
-  }
+  const long z1 = axis == 1 ? sg.z1[1] : sg.z1[2];
+  z = (axis == 1 ? sg.z0[1] : sg.z0[2]) + (long)L * BLK + threadIdx.x;
+  return z < z1;
 }
+
+/* plm-muscl's faces: z in [begin, T - sx) on every axis, begin = 0 (step 2) or sx (step 4) */
+inline SweepGrid face_grid(const GridDesc &g, long begin, long BLK)
+{
+  const long z0[3] = { begin, begin, begin }, z1[3] = { g.T - g.sx, g.T - g.sx, g.T - g.sx };
+  return make_sweep_grid(g, z0, z1, BLK);
+}
+
+template <typename FT> struct FluxPlanes { FT *f[3]; };
 
 /* Block order of the stage update. A zone's update reads the flux planes at its own
  * index and at +-1 in i, j and k (the constrained-transport averages), so in the flat order
@@ -692,29 +703,59 @@ __device__ __forceinline__ bool update_zone_index(const GridDesc &g, long &t)
   return r < plane;
 }
 
-/* HLLD sweep along DIM, common path only (interface_flux_fast): interfaces that need
- * the c2p cascade, a later Newton attempt, the small-normal-field branch, the HLLC
- * fallback or the retry are queued for k_flux_redo, which computes them with the full
- * FP64 solver. In the plain form that is the result the full sweep gives; in the mixed
- * form (R = float) the rare branches run in FP64 instead of FP32. Leaving them out of this
- * kernel lowers its register peak. The queue holds every interface of the sweep, so it
- * cannot overflow. */
-template <typename R, int DIM>
-__global__ __launch_bounds__(kFluxBlock<R>, sizeof(R) == 4 ? kFastFluxWaves32 : kFastFluxWaves64)
-void k_flux_hlld_fast(const double *__restrict__ P, R *__restrict__ Fout, GridDesc g, int recon, PhysParams pp,
-                      DevStats *st, RedoQueue rq)
+/* HLL and HLLC sweeps of a stage: one thread per interface, all three axes in one launch.
+ * Occupancy targets (waves per SIMD): FP32 at 3, FP64 at 2 even where 256 registers spill
+ * (the spill traffic costs less than the latency that a single wave cannot hide). */
+template <typename R, typename FT, int SOLVER>
+__global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 3 : 2) void k_flux(const double *__restrict__ P, FluxPlanes<FT> Fo,
+                                                                        GridDesc g, SweepGrid sg, int recon,
+                                                                        PhysParams pp, DevStats *st)
 {
   const long T = g.T;
-  const long S = DIM == 1 ? g.sx : DIM == 2 ? g.sy : g.sz;
-  long z;
-  const bool has = sweep_interface<DIM>(g, z);
+  int axis;
+  long z = 0;
+  const bool has = sweep_interface(g, sg, axis, z);
+  double lam_out = 0.0;
+  unsigned long long cnt[2] = {0, 0};
+  if (has) {
+    R lam = R(0);
+    FluxCounters fc = {0, 0, 0, 0};
+    R F[8];
+    int retried;
+    const int err = interface_flux<R, SOLVER>(P, T, axis_stride(g, axis), axis, z, recon, pp, F, lam, fc, retried);
+    FT *__restrict__ Fout = Fo.f[axis];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) Fout[axis_plane(q, axis) * T + z] = (FT)F[q];
+    lam_out = (double)lam;
+    cnt[0] = (unsigned long long)retried;
+    cnt[1] = err ? 1ull : 0ull;
+  }
+  block_max_lambda(lam_out, &st->lam_bits);
+  unsigned long long *const dst[2] = { &st->retries, &st->failures };
+  block_add<2>(cnt, dst);
+}
+
+/* HLLD sweeps of a stage, common path only (interface_flux_fast): interfaces that need
+ * the c2p cascade, a later Newton attempt, the HLLC fallback or the retry are queued for
+ * k_flux_redo, which computes them with the full FP64 solver. In the plain form that is the
+ * result the full sweep gives; in the mixed form (R = float) the rare branches run in FP64
+ * instead of FP32. Leaving them out of this kernel lowers its register peak. The queue holds
+ * every interface of a sweep, so it cannot overflow. */
+template <typename R>
+__global__ __launch_bounds__(kFluxBlock<R>, sizeof(R) == 4 ? kFastFluxWaves32 : kFastFluxWaves64)
+void k_flux_hlld_fast(const double *__restrict__ P, FluxPlanes<R> Fo, GridDesc g, SweepGrid sg, int recon,
+                      PhysParams pp, RedoQueue rq)
+{
+  int axis;
+  long z = 0;
+  const bool has = sweep_interface(g, sg, axis, z);
   double lam_out = 0.0;
   unsigned long long cnt[3] = {0, 0, 0};
   bool defer = false;
   if (has) {
     R lam = R(0);
     FluxCounters fc = {0, 0, 0, 0};
-    defer = interface_flux_fast<R, DIM>(P, Fout, T, S, z, recon, pp, lam, fc) != 0;
+    defer = interface_flux_fast<R>(P, Fo.f[axis], g.T, axis_stride(g, axis), axis, z, recon, pp, lam, fc) != 0;
     if (!defer) {
       cnt[0] = 1;
       cnt[1] = (unsigned long long)fc.c2p_iters;
@@ -722,22 +763,22 @@ void k_flux_hlld_fast(const double *__restrict__ P, R *__restrict__ Fout, GridDe
     }
     lam_out = (double)lam;
   }
-  queue_push(rq, defer, z);
+  queue_push(rq, axis, defer, z);
   sweep_counters_wave(lam_out, cnt[0] != 0, (unsigned)cnt[1], (unsigned)cnt[2], false, rq.part);
 }
 
-/* The queued interfaces of a sweep, recomputed by the full FP64 method (reconstruction,
+/* The queued interfaces of the sweeps, recomputed by the full FP64 method (reconstruction,
  * HLLD attempt ladder, HLLC fallback, retry) and written over the sweep's fluxes (FP32
- * in the mixed form, FP64 in the plain one). A grid-stride loop over the queue count. */
-template <typename FT, int DIM, int SOLVER>
-__global__ __launch_bounds__(kBlock) void k_flux_redo(const double *__restrict__ P, FT *__restrict__ Fout,
-                                                      GridDesc g, int recon, PhysParams pp, DevStats *st,
-                                                      RedoQueue rq, unsigned int nparts)
+ * in the mixed form, FP64 in the plain one). A grid-stride loop over each axis's list; the
+ * grid is one block per CU, which at this kernel's registers is all that can be resident. */
+template <typename FT, int SOLVER>
+__global__ __launch_bounds__(kBlock) void k_flux_redo(const double *__restrict__ P, FluxPlanes<FT> Fo, GridDesc g,
+                                                      int recon, PhysParams pp, DevStats *st, RedoQueue rq,
+                                                      unsigned int nparts)
 {
-  const unsigned int n = min(*rq.count, rq.cap);
   double lam_out = 0.0;
   unsigned long long cnt[7] = {0, 0, 0, 0, 0, 0, 0};
-  // the sweep's per-wave counters (nparts waves; 0 for a pass without them)
+  // the sweeps' per-wave counters (nparts waves)
   for (unsigned int w = blockIdx.x * blockDim.x + threadIdx.x; w < nparts; w += gridDim.x * blockDim.x) {
     const uint4 v = rq.part[w];
     lam_out = fmax(lam_out, __longlong_as_double((long long)(((unsigned long long)v.y << 32) | v.x)));
@@ -745,17 +786,22 @@ __global__ __launch_bounds__(kBlock) void k_flux_redo(const double *__restrict__
     cnt[4] += (unsigned long long)(v.z >> 8);
     cnt[5] += (unsigned long long)(v.w & 0xffffu);
   }
-  for (unsigned int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-    const long T = g.T;
-    const long S = DIM == 1 ? g.sx : DIM == 2 ? g.sy : g.sz;
-    const long z = (long)rq.z[k];
+  const long T = g.T;
+  // k counts through the three lists
+  const unsigned int n0 = min(rq.count[0], rq.cap), n1 = min(rq.count[1], rq.cap), n2 = min(rq.count[2], rq.cap);
+  const unsigned long n = (unsigned long)n0 + n1 + n2;
+  for (unsigned long k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+    const int axis = k < n0 ? 0 : k < (unsigned long)n0 + n1 ? 1 : 2;
+    const unsigned long i = axis == 0 ? k : axis == 1 ? k - n0 : k - n0 - n1;
+    const long z = (long)rq.z[(size_t)axis * rq.cap + i];
     double lam = 0.0;
     FluxCounters fc = {0, 0, 0, 0};
     double F[8];
     int retried;
-    const int err = interface_flux<double, DIM, SOLVER>(P, T, S, z, recon, pp, F, lam, fc, retried);
+    const int err = interface_flux<double, SOLVER>(P, T, axis_stride(g, axis), axis, z, recon, pp, F, lam, fc, retried);
+    FT *__restrict__ Fout = axis == 0 ? Fo.f[0] : axis == 1 ? Fo.f[1] : Fo.f[2];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) Fout[q * T + z] = (FT)F[q];
+    for (int q = 0; q < 8; ++q) Fout[axis_plane(q, axis) * T + z] = (FT)F[q];
     lam_out = fmax(lam_out, lam);
     cnt[0] += (unsigned long long)fc.hlld_ok;
     cnt[1] += (unsigned long long)fc.hlld_fail;
@@ -927,99 +973,101 @@ __global__ __launch_bounds__(kBlock) void k_flux_weno_split_char(const double *_
  * counted per abort point (ctu_failed[stage][point]); the step reports the first nonzero
  * count, as the reference throws at the first abort point with failures.
  * ------------------------------------------------------------------------ */
-/* the operator's own limited slope (plm_minmod with its theta, :22-31) of field q along S at
- * zone z, zero outside the flat range [sx, T - sx) where the reference computes slopes */
-__device__ __forceinline__ double ctu_slope(const double *__restrict__ P, long T, long sxz, long z, long S, int q,
-                                            double theta)
+/* the operator's own limited slope (plm_minmod with its theta, :22-31) of a field's plane Pq
+ * along S at zone z, zero outside the flat range [sx, T - sx) where the reference computes
+ * slopes; the minmod as in plm() */
+__device__ __forceinline__ double ctu_slope(const double *__restrict__ Pq, long T, long sxz, long z, long S, double theta)
 {
 #pragma clang fp contract(off)
   if (z < sxz || z >= T - sxz) return 0.0;
-  const double ul = P[q * T + z - S], u0 = P[q * T + z], ur = P[q * T + z + S];
+  const double ul = Pq[z - S], u0 = Pq[z], ur = Pq[z + S];
   const double a = theta * (u0 - ul);
   const double b = 0.5 * (ur - ul);
   const double c = theta * (ur - u0);
-  const double sa = (double)((a > 0) - (a < 0)), sb = (double)((b > 0) - (b < 0)), sc = (double)((c > 0) - (c < 0));
-  const double ab = fabs(a) < fabs(b) ? fabs(a) : fabs(b);
-  const double m = ab < fabs(c) ? ab : fabs(c);
-  return 0.25 * fabs(sa + sb) * (sa + sc) * m;
+  return fmax(fmin(fmin(a, b), c), 0.0) + fmin(fmax(fmax(a, b), c), 0.0);
 }
 
-/* the half-slope states of face z | z+S along S: from P with its own slopes (step 2) or
- * from a predictor Ps with P's slopes (step 4) */
-__device__ __forceinline__ void ctu_face_states(const double *__restrict__ P, const double *__restrict__ Ps, long T,
-                                                long sxz, long S, long z, double theta, double *pl, double *pr)
+/* the half-slope states, in the axis's frame, of face z | z+S along the axis: from P with its
+ * own slopes (step 2) or from a predictor Ps with P's slopes (step 4) */
+__device__ __forceinline__ void ctu_face_states(const double *__restrict__ P, const double *__restrict__ Ps,
+                                                const GridDesc &g, int axis, long z, double theta, double *pl, double *pr)
 {
 #pragma clang fp contract(off)
+  const long T = g.T, sxz = g.sx, S = axis_stride(g, axis);
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
-    pr[q] = Ps[q * T + z + S] - 0.5 * ctu_slope(P, T, sxz, z + S, S, q, theta);
-    pl[q] = Ps[q * T + z] + 0.5 * ctu_slope(P, T, sxz, z, S, q, theta);
+    const long o = axis_plane(q, axis) * T;
+    pr[q] = Ps[o + z + S] - 0.5 * ctu_slope(P + o, T, sxz, z + S, S, theta);
+    pl[q] = Ps[o + z] + 0.5 * ctu_slope(P + o, T, sxz, z, S, theta);
   }
 }
 
-/* Godunov fluxes along DIM of the half-slope states over faces z | z+S, z in [begin, T - sx),
- * with the full solver (HLL, HLLC; HLLD through the redo). An unphysical state counts a
- * failure and leaves the flux unwritten. A solver error also leaves it: then the flux is
- * what the reference's array holds there, zero in step 2 (fresh arrays) and the step-2
- * flux in step 4 (`keep`). */
-template <int DIM>
-__global__ __launch_bounds__(kBlock, 2) void k_ctu_faces(const double *__restrict__ P, const double *__restrict__ Ps,
-                                                         double *__restrict__ F, GridDesc g, PhysParams pp, int solver,
-                                                         long begin, int keep, DevStats *st,
+/* The states of a face pass: P itself on every axis (step 2) or the axis's own predictor
+ * (step 4). */
+struct FaceStates { const double *p[3]; };
+
+/* Godunov fluxes of the half-slope states over the faces z | z+S, z in [begin, T - sx), of the
+ * three axes in one launch, with the full solver (HLL, HLLC; HLLD through the redo). An
+ * unphysical state counts a failure and leaves the flux unwritten. A solver error also leaves
+ * it: then the flux is what the reference's array holds there, zero in step 2 (fresh arrays)
+ * and the step-2 flux in step 4 (`keep`). */
+template <int SOLVER>
+__global__ __launch_bounds__(kBlock, 2) void k_ctu_faces(const double *__restrict__ P, FaceStates Ps, FluxPlanes<double> Fo,
+                                                         GridDesc g, SweepGrid sg, PhysParams pp, int keep, DevStats *st,
                                                          unsigned long long *fail)
 {
-  const long T = g.T, sxz = g.sx;
-  const long S = DIM == 1 ? g.sx : DIM == 2 ? g.sy : g.sz;
-  const long z = begin + (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long T = g.T;
+  int axis;
+  long z = 0;
+  const bool has = sweep_interface(g, sg, axis, z);
   double lam_out = 0.0;
-  unsigned long long cnt[5] = {0, 0, 0, 0, 0};
-  if (z < T - sxz) {
+  unsigned long long cnt[1] = {0};
+  if (has) {
     double pl[8], pr[8];
-    ctu_face_states(P, Ps, T, sxz, S, z, pp.theta, pl, pr);
+    ctu_face_states(P, Ps.p[axis], g, axis, z, pp.theta, pl, pr);
     if (check_prim(pl) || check_prim(pr)) cnt[0] = 1;
     else {
+      double *__restrict__ F = Fo.f[axis];
       double f[8], lam = 0.0;
 #pragma unroll
-      for (int q = 0; q < 8; ++q) f[q] = keep ? F[q * T + z] : 0.0;
+      for (int q = 0; q < 8; ++q) f[q] = keep ? F[axis_plane(q, axis) * T + z] : 0.0;
       FluxCounters fc = {0, 0, 0, 0};
-      riemann_dispatch<double, DIM>(solver, pl, pr, f, pp.gamma, pp.pfloor, lam, fc);
+      riemann_dispatch<double, 1>(SOLVER, pl, pr, f, pp.gamma, pp.pfloor, lam, fc);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) F[q * T + z] = f[q];
+      for (int q = 0; q < 8; ++q) F[axis_plane(q, axis) * T + z] = f[q];
       lam_out = lam;
-      cnt[1] = (unsigned long long)fc.hlld_ok;
-      cnt[2] = (unsigned long long)fc.hlld_fail;
-      cnt[3] = (unsigned long long)fc.c2p_iters;
-      cnt[4] = (unsigned long long)fc.newton_iters;
     }
   }
   block_max_lambda(lam_out, &st->lam_bits);
-  unsigned long long *const dst[5] = { fail, &st->hlld_success, &st->hlld_failure, &st->hlld_c2p_iters,
-                                       &st->hlld_newton_iters };
-  block_add<5>(cnt, dst);
+  unsigned long long *const dst[1] = { fail };
+  block_add<1>(cnt, dst);
 }
 
-/* The HLLD faces of k_ctu_faces on the common path (riemann_hlld_lean): a face that needs the c2p cascade, a later Newton attempt, the small
- * normal field branch or the HLLC fallback is queued for k_ctu_faces_redo. The queue holds
- * every face, so it cannot overflow. */
-template <int DIM>
-__global__ __launch_bounds__(kBlock, kFastFluxWaves64)
-void k_ctu_faces_fast(const double *__restrict__ P, const double *__restrict__ Ps, double *__restrict__ F,
-                      GridDesc g, PhysParams pp, long begin, DevStats *st, unsigned long long *fail, RedoQueue rq)
+/* The HLLD faces on the common path (riemann_hlld_lean): a face that needs the c2p cascade, a
+ * later Newton attempt or the HLLC fallback is queued for k_ctu_faces_redo. The queue holds
+ * every face of an axis, so it cannot overflow. Grid, blocks and occupancy as
+ * k_flux_hlld_fast<double>. */
+__global__ __launch_bounds__(kFluxBlock<double>, kFastFluxWaves64)
+void k_ctu_faces_fast(const double *__restrict__ P, FaceStates Ps, FluxPlanes<double> Fo, GridDesc g, SweepGrid sg,
+                      PhysParams pp, RedoQueue rq)
 {
-  const long T = g.T, sxz = g.sx;
-  const long S = DIM == 1 ? g.sx : DIM == 2 ? g.sy : g.sz;
-  const long z = begin + (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long T = g.T;
+  int axis;
+  long z = 0;
+  const bool has = sweep_interface(g, sg, axis, z);
   double lam_out = 0.0;
   unsigned long long cnt[4] = {0, 0, 0, 0};
   bool defer = false;
-  if (z < T - sxz) {
+  if (has) {
     double pl[8], pr[8];
-    ctu_face_states(P, Ps, T, sxz, S, z, pp.theta, pl, pr);
+    ctu_face_states(P, Ps.p[axis], g, axis, z, pp.theta, pl, pr);
     if (check_prim(pl) || check_prim(pr)) cnt[0] = 1;
     else {
+      double *__restrict__ F = Fo.f[axis];
       double lam = 0.0;
       FluxCounters fc = {0, 0, 0, 0};
-      defer = riemann_hlld_lean<DIM>(pl, pr, pp, lam, fc, [&](int q, double f) { F[q * T + z] = f; }) != 0;
+      defer = riemann_hlld_lean<1>(pl, pr, pp, lam, fc,
+                                   [&](int q, double f) { F[axis_plane(q, axis) * T + z] = f; }) != 0;
       if (!defer) {
         cnt[1] = 1;
         cnt[2] = (unsigned long long)fc.c2p_iters;
@@ -1028,22 +1076,20 @@ void k_ctu_faces_fast(const double *__restrict__ P, const double *__restrict__ P
       lam_out = lam;
     }
   }
-  queue_push(rq, defer, z);
+  queue_push(rq, axis, defer, z);
   sweep_counters_wave(lam_out, cnt[1] != 0, (unsigned)cnt[2], (unsigned)cnt[3], cnt[0] != 0, rq.part);
 }
 
 /* The queued faces of k_ctu_faces_fast by the full HLLD method (attempt ladder, HLLC
- * fallback); a grid-stride loop over the queue count. Their states passed the physical
- * check in the fast pass. */
-template <int DIM>
-__global__ __launch_bounds__(kBlock) void k_ctu_faces_redo(const double *__restrict__ P, const double *__restrict__ Ps,
-                                                           double *__restrict__ F, GridDesc g, PhysParams pp, int keep,
+ * fallback), as k_flux_redo does it for the sweeps. Their states passed the physical check in
+ * the fast pass. A face whose fast waves both lie on one side may hold that side's flux
+ * already; the solver then never fails there, so `keep` finds the flux it needs. */
+__global__ __launch_bounds__(kBlock) void k_ctu_faces_redo(const double *__restrict__ P, FaceStates Ps,
+                                                           FluxPlanes<double> Fo, GridDesc g, PhysParams pp, int keep,
                                                            DevStats *st, unsigned long long *fail, RedoQueue rq,
                                                            unsigned int nparts)
 {
-  const unsigned int n = min(*rq.count, rq.cap);
-  const long T = g.T, sxz = g.sx;
-  const long S = DIM == 1 ? g.sx : DIM == 2 ? g.sy : g.sz;
+  const long T = g.T;
   double lam_out = 0.0;
   unsigned long long cnt[6] = {0, 0, 0, 0, 0, 0};
   // the fast pass's per-wave counters
@@ -1055,16 +1101,21 @@ __global__ __launch_bounds__(kBlock) void k_ctu_faces_redo(const double *__restr
     cnt[3] += (unsigned long long)(v.w & 0xffffu);
     cnt[5] += (unsigned long long)(v.w >> 16);
   }
-  for (unsigned int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-    const long z = (long)rq.z[k];
+  const unsigned int n0 = min(rq.count[0], rq.cap), n1 = min(rq.count[1], rq.cap), n2 = min(rq.count[2], rq.cap);
+  const unsigned long n = (unsigned long)n0 + n1 + n2;
+  for (unsigned long k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+    const int axis = k < n0 ? 0 : k < (unsigned long)n0 + n1 ? 1 : 2;
+    const unsigned long i = axis == 0 ? k : axis == 1 ? k - n0 : k - n0 - n1;
+    const long z = (long)rq.z[(size_t)axis * rq.cap + i];
+    double *__restrict__ F = axis == 0 ? Fo.f[0] : axis == 1 ? Fo.f[1] : Fo.f[2];
     double pl[8], pr[8], f[8], lam = 0.0;
-    ctu_face_states(P, Ps, T, sxz, S, z, pp.theta, pl, pr);
+    ctu_face_states(P, axis == 0 ? Ps.p[0] : axis == 1 ? Ps.p[1] : Ps.p[2], g, axis, z, pp.theta, pl, pr);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) f[q] = keep ? F[q * T + z] : 0.0;
+    for (int q = 0; q < 8; ++q) f[q] = keep ? F[axis_plane(q, axis) * T + z] : 0.0;
     FluxCounters fc = {0, 0, 0, 0};
-    riemann_hlld<double, DIM>(pl, pr, f, pp.gamma, pp.pfloor, lam, fc);
+    riemann_hlld<double, 1>(pl, pr, f, pp.gamma, pp.pfloor, lam, fc);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) F[q * T + z] = f[q];
+    for (int q = 0; q < 8; ++q) F[axis_plane(q, axis) * T + z] = f[q];
     lam_out = fmax(lam_out, lam);
     cnt[0] += (unsigned long long)fc.hlld_ok;
     cnt[1] += (unsigned long long)fc.hlld_fail;
@@ -1093,9 +1144,11 @@ __global__ __launch_bounds__(kBlock, 2) void k_ctu_predict(const double *__restr
                                                            const double *__restrict__ F, const double *__restrict__ G,
                                                            const double *__restrict__ H, double *__restrict__ Ux,
                                                            double *__restrict__ Uy, double *__restrict__ Uz, GridDesc g,
-                                                           PhysParams pp, double dt, unsigned long long *fail)
+                                                           PhysParams pp, double dt, unsigned long long *fail,
+                                                           unsigned int *redo_count)
 {
 #pragma clang fp contract(off)
+  clear_queue(redo_count);       // between the stage's two face passes
   const long T = g.T, sxz = g.sx, sy = g.sy, sz = g.sz;
   const long z = sxz + (long)blockIdx.x * blockDim.x + threadIdx.x;
   unsigned long long cnt[1] = {0};
@@ -1108,7 +1161,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_ctu_predict(const double *__restr
       double PL[8], PR[8];
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
-        const double s = ctu_slope(P, T, sxz, z, Sd[d], q, pp.theta);
+        const double s = ctu_slope(P + q * T, T, sxz, z, Sd[d], pp.theta);
         PL[q] = P[q * T + z] - 0.5 * s;
         PR[q] = P[q * T + z] + 0.5 * s;
       }
@@ -1385,10 +1438,12 @@ __global__ __launch_bounds__(kBlock, 3) void k_update_c2p(
     const FT *__restrict__ Fx, const FT *__restrict__ Fy, const FT *__restrict__ Fz,
     const double *__restrict__ U0, double *__restrict__ U, double *__restrict__ A, double *__restrict__ P,
     GridDesc g, double dt, int kind, int write_u, double gamma, double pfloor, int ereset, double preset,
-    double dreset, DevStats *st, int pass, double *__restrict__ Uw, float2 *__restrict__ start, uint4 *part)
+    double dreset, DevStats *st, int pass, double *__restrict__ Uw, float2 *__restrict__ start, uint4 *part,
+    unsigned int *redo_count)
 {
   static_assert(MODE == C2P_CASCADE || MODE == C2P_STORED, "stage passes start from the cascade or a stored start");
   constexpr int NC = 4;
+  clear_queue(redo_count);
   const long T = g.T;
   unsigned long long cnt[NC] = {};
   {
@@ -1443,11 +1498,13 @@ __global__ __launch_bounds__(kBlock, MODE == C2P_NET ? 3 : 4) void k_p2c_c2p(con
                                                                     double pfloor, int ereset, double preset,
                                                                     double dreset, DevStats *st, int pass,
                                                                     double *__restrict__ Uw, MlpDev net,
-                                                                    float2 *__restrict__ start, uint4 *part)
+                                                                    float2 *__restrict__ start, uint4 *part,
+                                                                    unsigned int *redo_count)
 {
   static_assert(MODE == C2P_CASCADE || MODE == C2P_NET, "the first pass starts from the cascade or the network");
   constexpr bool LEARNED = MODE == C2P_NET;
   constexpr int NC = LEARNED ? 6 : 4;
+  clear_queue(redo_count);
   MlpLds *L = nullptr;
   if constexpr (LEARNED) {
     __shared__ __align__(16) MlpLds lds;
@@ -2038,11 +2095,6 @@ struct maragpu_ctx {
   GridDesc g;
   int device = 0;                    // the HIP device current at create
   hipStream_t stream = nullptr;
-  // HLLD sweeps: the redo of an axis runs on `side`, beside the next axis's sweep, and the
-  // update waits for all three (redo_done); each axis has its own queue and counter slots
-  hipStream_t side = nullptr;
-  hipEvent_t sweep_done[3] = {nullptr, nullptr, nullptr}, redo_done[3] = {nullptr, nullptr, nullptr};
-  unsigned redo_pending = 0;         // bit d: the redo of axis d+1 may still run on `side`
   double *Pc = nullptr, *Pw = nullptr, *U0 = nullptr, *U = nullptr, *A = nullptr;
   void *F[3] = {nullptr, nullptr, nullptr};
   DevStats *dstats = nullptr;
@@ -2061,8 +2113,8 @@ struct maragpu_ctx {
   float2 *start = nullptr;
   // the c2p passes' per-wave counters (one slot per wave of a pass)
   uint4 *c2p_part = nullptr;
-  // mixed form with HLLD: the FP64 redo queue of each sweep
-  RedoQueue redo[3] = {};           // one per axis (plm-muscl's face passes use the first)
+  // HLLD: the interfaces of the sweeps or face passes left to the full solver
+  RedoQueue redo = {};
   // weno-split: U with its ghost images, and the zone fluxes (8 planes) and speeds (1 plane)
   // of the current sweep in the flux precision
   double *Uw = nullptr;
@@ -2118,38 +2170,29 @@ GridDesc make_grid(const maragpu_config &c)
   return g;
 }
 
-template <typename R, typename FT, int DIM>
+/* the three axis sweeps of a stage: HLLD on the common path and, for what it queued (in the
+ * mixed form the FP32 HLLD failures, in the plain form whatever left the common path), the
+ * full FP64 solver; HLL and HLLC by the full kernel */
+template <typename R>
 void launch_flux(maragpu_ctx *c, const PhysParams &pp)
 {
-  const long S = DIM == 1 ? c->g.sx : DIM == 2 ? c->g.sy : c->g.sz;
-  const long n = c->g.T - 5 * S;
-  if (n <= 0) return;
-  FT *F = static_cast<FT *>(c->F[DIM - 1]);
-  RedoQueue none = { nullptr, 0u, nullptr, nullptr, 0u };
-  switch (c->cfg.riemann) {
-  case MARAGPU_HLL:
-    k_flux<R, FT, DIM, RIEMANN_HLL><<<nblocks(n), kBlock, 0, c->stream>>>(c->Pw, F, c->g, c->cfg.recon, pp, c->dstats, none);
-    break;
-  case MARAGPU_HLLC:
-    k_flux<R, FT, DIM, RIEMANN_HLLC><<<nblocks(n), kBlock, 0, c->stream>>>(c->Pw, F, c->g, c->cfg.recon, pp, c->dstats, none);
-    break;
-  default:
-    // the sweep, then its queued interfaces by the full FP64 solver: in the mixed form the
-    // FP32 HLLD failures, in the plain form whatever left the common path
-    // the redo of this axis runs on the side stream while the next axis is swept: it reads
-    // only P and this axis's queue and slots, and writes only this axis's fluxes
-    RedoQueue &q = c->redo[DIM - 1];
-    hipMemsetAsync(q.count, 0, sizeof(unsigned int), c->stream);
-    const unsigned nb = (unsigned)sweep_blocks<DIM>(c->g, kFluxBlock<R>);
-    k_flux_hlld_fast<R, DIM><<<nb, kFluxBlock<R>, 0, c->stream>>>(c->Pw, F, c->g, c->cfg.recon, pp, c->dstats, q);
-    hipEventRecord(c->sweep_done[DIM - 1], c->stream);
-    hipStreamWaitEvent(c->side, c->sweep_done[DIM - 1], 0);
-    k_flux_redo<FT, DIM, RIEMANN_HLLD><<<kRedoBlocks, kBlock, 0, c->side>>>(c->Pw, F, c->g, c->cfg.recon, pp,
-                                                                            c->dstats, q, nb * (kFluxBlock<R> / 64));
-    hipEventRecord(c->redo_done[DIM - 1], c->side);
-    c->redo_pending |= 1u << (DIM - 1);
-    break;
+  FluxPlanes<R> F;
+  for (int d = 0; d < 3; ++d) F.f[d] = static_cast<R *>(c->F[d]);
+  if (c->cfg.riemann == MARAGPU_HLLD) {
+    const SweepGrid sg = sweep_grid(c->g, kFluxBlock<R>);
+    const unsigned nb = sg.first[3];
+    if (!nb) return;
+    k_flux_hlld_fast<R><<<nb, kFluxBlock<R>, 0, c->stream>>>(c->Pw, F, c->g, sg, c->cfg.recon, pp, c->redo);
+    k_flux_redo<R, RIEMANN_HLLD><<<kRedoBlocks, kBlock, 0, c->stream>>>(c->Pw, F, c->g, c->cfg.recon, pp, c->dstats,
+                                                                       c->redo, nb * (kFluxBlock<R> / 64));
+    return;
   }
+  const SweepGrid sg = sweep_grid(c->g, kBlock);
+  if (!sg.first[3]) return;
+  if (c->cfg.riemann == MARAGPU_HLL)
+    k_flux<R, R, RIEMANN_HLL><<<sg.first[3], kBlock, 0, c->stream>>>(c->Pw, F, c->g, sg, c->cfg.recon, pp, c->dstats);
+  else
+    k_flux<R, R, RIEMANN_HLLC><<<sg.first[3], kBlock, 0, c->stream>>>(c->Pw, F, c->g, sg, c->cfg.recon, pp, c->dstats);
 }
 
 /* weno-split sweep along DIM: zone fluxes and speeds, then the split interface fluxes */
@@ -2169,8 +2212,6 @@ void launch_weno_split(maragpu_ctx *c, const PhysParams &pp)
     k_flux_weno_split<R, R, DIM><<<nblocks(cnt), kBlock, 0, c->stream>>>(c->Uw, FZ, AZ,
                                                                           static_cast<R *>(c->F[DIM - 1]), g, pp);
 }
-
-struct EventPair { int a, b; };
 
 /* Per-block partials of the measure table for maragpu_measure_noalloc, in a file-scope
  * device array: (kMeasBlocks + 1) rows of kMeasQ doubles, 270 KB per device, held from
@@ -2246,11 +2287,6 @@ int maragpu_create(const maragpu_config *cfg, maragpu_ctx **out)
   c->g = make_grid(*cfg);
   if (c->g.T >= (1L << 32)) { delete c; return MARAGPU_E_INVALID; }   // 32-bit queue slots
   if (hipStreamCreate(&c->stream) != hipSuccess) { delete c; return MARAGPU_E_HIP; }
-  if (hipStreamCreate(&c->side) != hipSuccess) return fail_free(c);
-  for (int d = 0; d < 3; ++d)
-    if (hipEventCreateWithFlags(&c->sweep_done[d], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->redo_done[d], hipEventDisableTiming) != hipSuccess)
-      return fail_free(c);
   const size_t nd = 8 * (size_t)c->g.T;
   const size_t fbytes = nd * (cfg->precision == MARAGPU_MIXED ? sizeof(float) : sizeof(double));
   if (hipMalloc(&c->Pc, nd * sizeof(double)) != hipSuccess) return fail_free(c);
@@ -2284,31 +2320,25 @@ int maragpu_create(const maragpu_config *cfg, maragpu_ctx **out)
       return fail_free(c);
   }
   if (cfg->riemann == MARAGPU_HLLD && cfg->godunov != MARAGPU_WENO_SPLIT) {
-    // a slot for every interface of a sweep or face pass (4 bytes a slot: half a state plane)
-    const long cap = c->g.T;
-    // the HLLD sweeps' per-wave counters: one slot per wave of the largest sweep
-    long parts = 0;
-    parts = std::max(parts, sweep_blocks<1>(c->g, kFluxBlock<float>) * (kFluxBlock<float> / 64));
-    parts = std::max(parts, sweep_blocks<2>(c->g, kFluxBlock<float>) * (kFluxBlock<float> / 64));
-    parts = std::max(parts, sweep_blocks<3>(c->g, kFluxBlock<float>) * (kFluxBlock<float> / 64));
-    parts = std::max(parts, sweep_blocks<1>(c->g, kFluxBlock<double>) * (kFluxBlock<double> / 64));
-    parts = std::max(parts, sweep_blocks<2>(c->g, kFluxBlock<double>) * (kFluxBlock<double> / 64));
-    parts = std::max(parts, sweep_blocks<3>(c->g, kFluxBlock<double>) * (kFluxBlock<double> / 64));
-    parts = std::max(parts, (long)nblocks(c->g.T) * (kBlock / 64));   // plm-muscl's face passes
-    for (RedoQueue &q : c->redo) {
-      q.cap = (unsigned int)cap;
-      q.part_cap = (unsigned int)parts;
-      if (hipMalloc(&q.count, sizeof(unsigned int)) != hipSuccess ||
-          hipMalloc(&q.z, (size_t)cap * sizeof(unsigned int)) != hipSuccess ||
-          hipMalloc(&q.part, (size_t)parts * sizeof(uint4)) != hipSuccess)
-        return fail_free(c);
-    }
+    // a slot for every interface of a sweep or face pass (4 bytes a slot: half a state plane
+    // for an axis), and per-wave counters of the three sweeps
+    RedoQueue &q = c->redo;
+    q.cap = (unsigned int)c->g.T;
+    unsigned waves;
+    if (cfg->godunov == MARAGPU_PLM_MUSCL) waves = face_grid(c->g, 0, kFluxBlock<double>).first[3];
+    else if (cfg->precision == MARAGPU_MIXED) waves = sweep_grid(c->g, kFluxBlock<float>).first[3] * (kFluxBlock<float> / 64);
+    else waves = sweep_grid(c->g, kFluxBlock<double>).first[3];
+    static_assert(kFluxBlock<double> == 64, "one wave per FP64 block");
+    if (hipMalloc(&q.count, 3 * sizeof(unsigned int)) != hipSuccess ||
+        hipMalloc(&q.z, 3 * (size_t)q.cap * sizeof(unsigned int)) != hipSuccess ||
+        hipMalloc(&q.part, (size_t)std::max(waves, 1u) * sizeof(uint4)) != hipSuccess)
+      return fail_free(c);
   }
   // fluxes outside the sweep ranges are never written; keep them defined
   for (int d = 0; d < 3; ++d)
     if (hipMemsetAsync(c->F[d], 0, fbytes, c->stream) != hipSuccess) return fail_free(c);
   if (hipMemsetAsync(c->Pc, 0, nd * sizeof(double), c->stream) != hipSuccess) return fail_free(c);
-  c->ev.resize(64);
+  c->ev.resize(10);       // a step's phases: its start, the first pass, 2 x 4 stages at most
   for (auto &e : c->ev)
     if (hipEventCreate(&e) != hipSuccess) { e = nullptr; return fail_free(c); }
   if (hipStreamSynchronize(c->stream) != hipSuccess) return fail_free(c);
@@ -2321,7 +2351,6 @@ int maragpu_destroy(maragpu_ctx *c)
 {
   if (!c) return MARAGPU_E_INVALID;
   if (c->stream) hipStreamSynchronize(c->stream);
-  if (c->side) hipStreamSynchronize(c->side);
   hipFree(c->Pc); hipFree(c->Pw); hipFree(c->U0); hipFree(c->U); hipFree(c->A);
   for (int d = 0; d < 3; ++d) hipFree(c->F[d]);
   hipFree(c->dstats);
@@ -2329,11 +2358,9 @@ int maragpu_destroy(maragpu_ctx *c)
   hipFree(c->ddiv);
   hipFree(c->start);
   hipFree(c->c2p_part);
-  for (RedoQueue &q : c->redo) {
-    hipFree(q.count);
-    hipFree(q.z);
-    hipFree(q.part);
-  }
+  hipFree(c->redo.count);
+  hipFree(c->redo.z);
+  hipFree(c->redo.part);
   hipFree(c->Uw);
   hipFree(c->FZ);
   hipFree(c->dmeas);
@@ -2342,11 +2369,6 @@ int maragpu_destroy(maragpu_ctx *c)
   hipFree(c->Fdrive);
   hipFree(c->dcool);
   for (auto &e : c->ev) if (e) hipEventDestroy(e);
-  for (int d = 0; d < 3; ++d) {
-    if (c->sweep_done[d]) hipEventDestroy(c->sweep_done[d]);
-    if (c->redo_done[d]) hipEventDestroy(c->redo_done[d]);
-  }
-  if (c->side) hipStreamDestroy(c->side);
   if (c->stream) hipStreamDestroy(c->stream);
   delete c;
   return MARAGPU_OK;
@@ -2427,18 +2449,13 @@ int maragpu_advance(maragpu_ctx *c, double dt, maragpu_stats *stats)
   pp.gamf = (pp.gamma - 1.0) / pp.gamma;
   pp.igamma = 1.0 / pp.gamma;
   const bool mixed = c->cfg.precision == MARAGPU_MIXED;
+  // one event between consecutive phases: the step's start, then after the first pass and
+  // after every stage's fluxes and update
   int evi = 0;
-  std::vector<EventPair> ef, ec, eu;
-  auto mark = [&](std::vector<EventPair> &v) {
-    EventPair p = { evi, evi + 1 };
-    evi += 2;
-    v.push_back(p);
-    return p;
-  };
+  auto mark = [&]() { return hipEventRecord(c->ev[evi++], c->stream); };
 
   HIP_CHECK(hipMemsetAsync(c->dstats, 0, sizeof(DevStats), c->stream));
-  HIP_CHECK(hipEventRecord(c->ev[evi], c->stream));
-  const int ev_start = evi++;
+  HIP_CHECK(mark());
   // each update runs together with the c2p pass after it, and the step's PrimToCons with
   // its first pass
   const bool learned = c->cfg.c2p == MARAGPU_C2P_LEARNED;
@@ -2447,36 +2464,21 @@ int maragpu_advance(maragpu_ctx *c, double dt, maragpu_stats *stats)
   const unsigned nbl = nblocks(ni) < kLearnedBlocks ? nblocks(ni) : kLearnedBlocks;
   // the non-plain forms chain each zone's Newton start from solution to solution
   const bool chain = c->start != nullptr;
-  // the three axis sweeps, z first: their results do not depend on the order, and with HLLD
-  // the redo of the last axis cannot overlap a sweep, so it is the cheapest one (x at c2)
   auto sweeps = [&]() {
-    for (int d = 3; d >= 1; --d) {
-      EventPair p = mark(ef);
-      hipEventRecord(c->ev[p.a], c->stream);
-      if (c->cfg.godunov == MARAGPU_WENO_SPLIT) {
-        if (mixed) {
-          if (d == 1) launch_weno_split<float, 1>(c, pp);
-          if (d == 2) launch_weno_split<float, 2>(c, pp);
-          if (d == 3) launch_weno_split<float, 3>(c, pp);
-        }
-        else {
-          if (d == 1) launch_weno_split<double, 1>(c, pp);
-          if (d == 2) launch_weno_split<double, 2>(c, pp);
-          if (d == 3) launch_weno_split<double, 3>(c, pp);
-        }
-      }
-      else if (mixed) {
-        if (d == 1) launch_flux<float, float, 1>(c, pp);
-        if (d == 2) launch_flux<float, float, 2>(c, pp);
-        if (d == 3) launch_flux<float, float, 3>(c, pp);
+    if (c->cfg.godunov == MARAGPU_WENO_SPLIT) {
+      if (mixed) {
+        launch_weno_split<float, 3>(c, pp);
+        launch_weno_split<float, 2>(c, pp);
+        launch_weno_split<float, 1>(c, pp);
       }
       else {
-        if (d == 1) launch_flux<double, double, 1>(c, pp);
-        if (d == 2) launch_flux<double, double, 2>(c, pp);
-        if (d == 3) launch_flux<double, double, 3>(c, pp);
+        launch_weno_split<double, 3>(c, pp);
+        launch_weno_split<double, 2>(c, pp);
+        launch_weno_split<double, 1>(c, pp);
       }
-      hipEventRecord(c->ev[p.b], c->stream);
     }
+    else if (mixed) launch_flux<float>(c, pp);
+    else launch_flux<double>(c, pp);
   };
   std::vector<int> kinds;
   switch (c->cfg.rk) {
@@ -2488,62 +2490,44 @@ int maragpu_advance(maragpu_ctx *c, double dt, maragpu_stats *stats)
   const bool ctu = c->cfg.godunov == MARAGPU_PLM_MUSCL;
   auto ctu_fluxes = [&](int s) {
     // PlmCtuHancockOperator::ctu_hancock on the stage primitives Pw and the synchronised U (Uw)
-    EventPair p = mark(ef);
-    hipEventRecord(c->ev[p.a], c->stream);
     const long T = g.T, sxz = g.sx;
     const size_t nd = 8 * (size_t)T;
-    double *F0 = static_cast<double *>(c->F[0]), *F1 = static_cast<double *>(c->F[1]),
-           *F2 = static_cast<double *>(c->F[2]);
+    FluxPlanes<double> F;
+    for (int d = 0; d < 3; ++d) F.f[d] = static_cast<double *>(c->F[d]);
     double *Ux = c->ctuU, *Uy = c->ctuU + nd, *Uz = c->ctuU + 2 * nd;
     double *Px = c->ctuP, *Py = c->ctuP + nd, *Pz = c->ctuP + 2 * nd;
     unsigned long long *fl = c->dstats->ctu_failed[s];
-    const int rs = c->cfg.riemann;
-    // the faces of one axis over [begin, T - sx): HLLD on the common path and its queue,
+    // the faces of the three axes over [begin, T - sx): HLLD on the common path and its queue,
     // HLL and HLLC by the full kernel
-    auto faces = [&](int dim, const double *Ps, double *F, long begin, int keep, unsigned long long *f) {
-      const long n = T - sxz - begin;
-      if (n <= 0) return;
-      if (c->redo[0].z) {
-        hipMemsetAsync(c->redo[0].count, 0, sizeof(unsigned int), c->stream);
-        if (dim == 1) k_ctu_faces_fast<1><<<nblocks(n), kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, pp, begin, c->dstats, f, c->redo[0]);
-        if (dim == 2) k_ctu_faces_fast<2><<<nblocks(n), kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, pp, begin, c->dstats, f, c->redo[0]);
-        if (dim == 3) k_ctu_faces_fast<3><<<nblocks(n), kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, pp, begin, c->dstats, f, c->redo[0]);
-        const unsigned np = nblocks(n) * (kBlock / 64);
-        if (dim == 1) k_ctu_faces_redo<1><<<kRedoBlocks, kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, pp, keep, c->dstats, f, c->redo[0], np);
-        if (dim == 2) k_ctu_faces_redo<2><<<kRedoBlocks, kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, pp, keep, c->dstats, f, c->redo[0], np);
-        if (dim == 3) k_ctu_faces_redo<3><<<kRedoBlocks, kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, pp, keep, c->dstats, f, c->redo[0], np);
+    auto faces = [&](FaceStates Ps, long begin, int keep, unsigned long long *f) {
+      if (c->redo.z) {
+        const SweepGrid sg = face_grid(g, begin, kFluxBlock<double>);
+        const unsigned nb = sg.first[3];
+        if (!nb) return;
+        k_ctu_faces_fast<<<nb, kFluxBlock<double>, 0, c->stream>>>(c->Pw, Ps, F, g, sg, pp, c->redo);
+        k_ctu_faces_redo<<<kRedoBlocks, kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, pp, keep, c->dstats, f, c->redo, nb);
+        return;
       }
-      else {
-        if (dim == 1) k_ctu_faces<1><<<nblocks(n), kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, pp, rs, begin, keep, c->dstats, f);
-        if (dim == 2) k_ctu_faces<2><<<nblocks(n), kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, pp, rs, begin, keep, c->dstats, f);
-        if (dim == 3) k_ctu_faces<3><<<nblocks(n), kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, pp, rs, begin, keep, c->dstats, f);
-      }
+      const SweepGrid sg = face_grid(g, begin, kBlock);
+      const unsigned nb = sg.first[3];
+      if (!nb) return;
+      if (c->cfg.riemann == MARAGPU_HLL)
+        k_ctu_faces<RIEMANN_HLL><<<nb, kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, sg, pp, keep, c->dstats, f);
+      else
+        k_ctu_faces<RIEMANN_HLLC><<<nb, kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, sg, pp, keep, c->dstats, f);
     };
-    faces(1, c->Pw, F0, 0, 0, fl + 0);
-    faces(2, c->Pw, F1, 0, 0, fl + 0);
-    faces(3, c->Pw, F2, 0, 0, fl + 0);
-    k_ctu_predict<<<nblocks(T - sxz), kBlock, 0, c->stream>>>(c->Pw, c->Uw, F0, F1, F2, Ux, Uy, Uz, g, pp, dt, fl + 1);
+    faces(FaceStates{ { c->Pw, c->Pw, c->Pw } }, 0, 0, fl + 0);
+    k_ctu_predict<<<nblocks(T - sxz), kBlock, 0, c->stream>>>(c->Pw, c->Uw, F.f[0], F.f[1], F.f[2], Ux, Uy, Uz, g, pp, dt,
+                                                              fl + 1, c->redo.count);
     k_ctu_c2p<<<nblocks(T), kBlock, 0, c->stream>>>(c->Pw, Ux, Uy, Uz, Px, Py, Pz, g, c->cfg.gamma, c->cfg.pfloor,
                                                     c->dstats, fl + 2);
-    faces(1, Px, F0, sxz, 1, fl + 3);
-    faces(2, Py, F1, sxz, 1, fl + 3);
-    faces(3, Pz, F2, sxz, 1, fl + 3);
-    hipEventRecord(c->ev[p.b], c->stream);
-  };
-  // the update reads the fluxes of all three axes: wait for the redo kernels on the side stream
-  auto join_redo = [&]() {
-    for (int d = 0; d < 3; ++d)
-      if (c->redo_pending & (1u << d)) hipStreamWaitEvent(c->stream, c->redo_done[d], 0);
-    c->redo_pending = 0;
+    faces(FaceStates{ { Px, Py, Pz } }, sxz, 1, fl + 3);
   };
   auto update_c2p = [&](int kind, int write_u, int pass) {
-    join_redo();
-    EventPair p = mark(eu);
-    hipEventRecord(c->ev[p.a], c->stream);
     const unsigned nb = update_blocks(g.N);
 #define UPDATE_ARGS(FT) (const FT *)c->F[0], (const FT *)c->F[1], (const FT *)c->F[2], c->U0, c->U, c->A, c->Pw, \
     g, dt, kind, write_u, c->cfg.gamma, c->cfg.pfloor, c->cfg.ereset, c->cfg.preset, c->cfg.dreset, c->dstats, pass, c->Uw, \
-    c->start, c->c2p_part
+    c->start, c->c2p_part, c->redo.count
     if (chain && mixed) k_update_c2p<float, C2P_STORED><<<nb, kBlock, 0, c->stream>>>(UPDATE_ARGS(float));
     else if (chain) k_update_c2p<double, C2P_STORED><<<nb, kBlock, 0, c->stream>>>(UPDATE_ARGS(double));
     else if (mixed) k_update_c2p<float, C2P_CASCADE><<<nb, kBlock, 0, c->stream>>>(UPDATE_ARGS(float));
@@ -2553,19 +2537,18 @@ int maragpu_advance(maragpu_ctx *c, double dt, maragpu_stats *stats)
     if (c->Uw && c->cfg.ereset)
       k_conserved_after_reset<<<nblocks(g.T), kBlock, 0, c->stream>>>(c->Pw, c->Uw, g, c->cfg.gamma,
                                                                       &c->dstats->stage_reset[pass]);
-    hipEventRecord(c->ev[p.b], c->stream);
+    mark();
   };
   auto p2c_c2p = [&](int pass) {
-    EventPair p = mark(ec);
-    hipEventRecord(c->ev[p.a], c->stream);
 #define P2C_ARGS c->Pc, c->U0, c->Pw, g, c->cfg.gamma, c->cfg.pfloor, c->cfg.ereset, c->cfg.preset, c->cfg.dreset, \
     c->dstats, pass, c->Uw, net
     if (learned) {
-      k_p2c_c2p<C2P_NET><<<nbl, kBlock, 0, c->stream>>>(P2C_ARGS, c->start, c->c2p_part);
+      k_p2c_c2p<C2P_NET><<<nbl, kBlock, 0, c->stream>>>(P2C_ARGS, c->start, c->c2p_part, c->redo.count);
       k_c2p_parts<6><<<kPartBlocks, kBlock, 0, c->stream>>>(c->c2p_part, nbl * (kBlock / 64), c->dstats, pass);
     }
     else {
-      k_p2c_c2p<C2P_CASCADE><<<nblocks(ni), kBlock, 0, c->stream>>>(P2C_ARGS, chain ? c->start : nullptr, c->c2p_part);
+      k_p2c_c2p<C2P_CASCADE><<<nblocks(ni), kBlock, 0, c->stream>>>(P2C_ARGS, chain ? c->start : nullptr, c->c2p_part,
+                                                               c->redo.count);
       k_c2p_parts<4><<<kPartBlocks, kBlock, 0, c->stream>>>(c->c2p_part, nblocks(ni) * (kBlock / 64), c->dstats,
                                                              pass);
     }
@@ -2573,19 +2556,17 @@ int maragpu_advance(maragpu_ctx *c, double dt, maragpu_stats *stats)
     if (c->Uw && c->cfg.ereset)
       k_conserved_after_reset<<<nblocks(g.T), kBlock, 0, c->stream>>>(c->Pw, c->Uw, g, c->cfg.gamma,
                                                                       &c->dstats->stage_reset[pass]);
-    hipEventRecord(c->ev[p.b], c->stream);
+    mark();
   };
   int pass = 0;
   for (size_t s = 0; s < kinds.size(); ++s) {
     if (s == 0) p2c_c2p(pass++);
     if (ctu) ctu_fluxes((int)s);
     else sweeps();
+    mark();
     update_c2p(kinds[s], s + 1 < kinds.size() && stage_reads_u(kinds[s + 1]) ? 1 : 0, pass++);
   }
-  join_redo();
   HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipEventRecord(c->ev[evi], c->stream));
-  const int ev_end = evi++;
   HIP_CHECK(hipMemcpyAsync(c->hstats, c->dstats, sizeof(DevStats), hipMemcpyDeviceToHost, c->stream));
   HIP_CHECK(hipStreamSynchronize(c->stream));
 
@@ -2622,18 +2603,20 @@ int maragpu_advance(maragpu_ctx *c, double dt, maragpu_stats *stats)
     if (c->Fdrive || c->cool_kind) HIP_CHECK(hipGetLastError());
   }
 
-  auto sum_ms = [&](const std::vector<EventPair> &v) {
-    double t = 0.0;
-    for (auto &p : v) {
-      float ms = 0.f;
-      hipEventElapsedTime(&ms, c->ev[p.a], c->ev[p.b]);
-      t += ms;
-    }
-    return t;
+  auto ms_between = [&](int a, int b) {
+    float ms = 0.f;
+    hipEventElapsedTime(&ms, c->ev[a], c->ev[b]);
+    return (double)ms;
   };
-  c->flux_ms = sum_ms(ef); c->flux_n = (int)ef.size();
-  c->c2p_ms = sum_ms(ec); c->c2p_n = (int)ec.size();
-  c->upd_ms = sum_ms(eu); c->upd_n = (int)eu.size();
+  const int stages = (int)kinds.size();
+  c->c2p_ms = ms_between(0, 1); c->c2p_n = 1;
+  c->flux_ms = c->upd_ms = 0.0;
+  for (int t = 0; t < stages; ++t) {
+    c->flux_ms += ms_between(1 + 2 * t, 2 + 2 * t);
+    c->upd_ms += ms_between(2 + 2 * t, 3 + 2 * t);
+  }
+  c->flux_n = ctu ? stages : 3 * stages;      // a stage's axis sweeps count one each
+  c->upd_n = stages;
   if (stats) {
     std::memset(stats, 0, sizeof(*stats));
     stats->max_lambda = lam;
@@ -2652,9 +2635,7 @@ int maragpu_advance(maragpu_ctx *c, double dt, maragpu_stats *stats)
     stats->fp64_redo = (int64_t)h.redo;
     stats->fp64_redo_overflow = (int64_t)h.redo_overflow;
     stats->eig_identity = (int64_t)h.eig_identity;
-    float ms = 0.f;
-    hipEventElapsedTime(&ms, c->ev[ev_start], c->ev[ev_end]);
-    stats->device_ms = ms;
+    stats->device_ms = ms_between(0, evi - 1);
   }
   return errors;
 }

@@ -1015,18 +1015,30 @@ __device__ __forceinline__ void weno5_js_pair(double vm2, double vm1, double v0,
   qr = side(Tc, tc + 2.0*gc, Td, gc + gd, Te, te - 2.0*gd, tc, td, te);
 }
 
-/* The two states of interface z | z+S from its 6-point stencil. LEAN (FP64): the paired
- * WENO5, and the choice of method outside the fields' loop, so that the loads of all fields
- * can be in flight. */
+/* The plane of field q of a state held in the frame whose first axis is `axis` (0, 1, 2):
+ * (rho, p, v1, v2, v3, B1, B2, B3), or a conserved state or flux in that order. Uniform over
+ * a launch's block, so it costs scalar instructions only, and one copy of the sweep's code
+ * serves all three axes. */
+__device__ __forceinline__ int axis_plane(int q, int axis)
+{
+  if (q < 2) return q;
+  const int b = q < 5 ? 2 : 5;
+  const int k = axis + q - b;
+  return b + (k >= 3 ? k - 3 : k);
+}
+
+/* The two states, in the axis's frame, of interface z | z+S (S the axis's zone stride) from its
+ * 6-point stencil. LEAN (FP64): the paired WENO5, and the choice of method outside the
+ * fields' loop, so that the loads of all fields can be in flight. */
 template <typename R, bool LEAN>
-__device__ __forceinline__ void reconstruct_states(const double *__restrict__ P, long T, long S, long z, int recon,
-                                                   const PhysParams &pp, R *ql, R *qr)
+__device__ __forceinline__ void reconstruct_states(const double *__restrict__ P, long T, long S, int axis, long z,
+                                                   int recon, const PhysParams &pp, R *ql, R *qr)
 {
   if constexpr (LEAN) {
     if (recon == RECON_WENO5 && pp.IS == IS_JS96) {
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
-        const double *v = P + q * T + z;
+        const double *v = P + axis_plane(q, axis) * T + z;
         weno5_js_pair(v[-2 * S], v[-S], v[0], v[S], v[2 * S], v[3 * S], ql[q], qr[q]);
       }
       return;
@@ -1034,7 +1046,7 @@ __device__ __forceinline__ void reconstruct_states(const double *__restrict__ P,
     if (recon == RECON_PLM) {
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
-        const double *v = P + q * T + z;
+        const double *v = P + axis_plane(q, axis) * T + z;
         const double v0 = v[0], v1 = v[S];
         ql[q] = plm<double>(v[-S], v0, v1, +1.0, pp.theta);
         qr[q] = plm<double>(v0, v1, v[2 * S], -1.0, pp.theta);
@@ -1044,7 +1056,7 @@ __device__ __forceinline__ void reconstruct_states(const double *__restrict__ P,
   }
   const R theta = (R)pp.theta;
   for (int q = 0; q < 8; ++q) {
-    const double *Pq = P + q * T + z;
+    const double *Pq = P + axis_plane(q, axis) * T + z;
     const R v0 = (R)Pq[0], v1 = (R)Pq[S];
     if (recon == RECON_WENO5) {
       const R vm2 = (R)Pq[-2 * S], vm1 = (R)Pq[-S], v2 = (R)Pq[2 * S], v3 = (R)Pq[3 * S];

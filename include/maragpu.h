@@ -1,7 +1,7 @@
 /* maragpu — MI355X (gfx950) relativistic-MHD update, C ABI.
  *
- * One context owns one device-resident grid and two HIP streams (the second runs the HLLD
- * sweeps' redo kernels beside the next sweep; maragpu_advance returns with both drained).
+ * One context owns one device-resident grid and one HIP stream; maragpu_advance returns with
+ * it drained.
  * Nothing in this header uses HIP or torch types; all pointers are host pointers unless
  * stated otherwise.
  * Every entry point returns instead of throwing. Return codes: 0 success, > 0 a count
@@ -181,7 +181,9 @@ int maragpu_set_cooling(maragpu_ctx *ctx, int kind, double ref, double t0, const
 /* EnergyRemoved: the energy taken out since the last call (then reset) */
 int maragpu_cooling_energy_removed(maragpu_ctx *ctx, double *removed);
 
-/* device time of the dominant kernel over the last advance (ms, per launch) and launches */
+/* device time over the last advance (ms) and counts: the axis sweeps (the three of a stage are
+ * one launch and count three; plm-muscl: one flux evaluation per stage), the step's first c2p
+ * pass, the stage updates */
 int maragpu_kernel_times(maragpu_ctx *ctx, double *flux_ms, int *flux_launches, double *c2p_ms,
                          int *c2p_launches, double *update_ms, int *update_launches);
 const char *maragpu_strerror(int code);

@@ -66,3 +66,47 @@ def test_supersonic_sweeps(gpu, oracle_lib, extrap, IS, flow, N):
     Pg = ctx.download()
     assert (L1(Pg) <= L1_tol).all()
     assert (worst(Pg) <= max_tol).all()
+
+
+@pytest.mark.parametrize("N,Ng,extrap,riemann,precision", [
+    ((3, 3, 3), 3, "weno5", "hlld", "fp64"),
+    ((3, 3, 3), 3, "weno5", "hlld", "mixed"),
+    ((4, 3, 67), 2, "plm", "hlld", "fp64"),
+    ((5, 40, 4), 3, "plm", "hllc", "fp64"),
+    ((33, 3, 5), 3, "weno5", "hlld", "mixed"),
+])
+def test_smallest_grids(gpu, oracle_lib, N, Ng, extrap, riemann, precision):
+    """The three sweeps of a stage share one launch, each with its own range of blocks: grids
+    whose ranges are empty, shorter than a block, or end inside a block or a tile column.
+    Plain-form tolerances (mixed: 1e-6 in L1, its bound against FP64)."""
+    rng = np.random.default_rng(sum(N) + Ng)
+    P = np.empty(tuple(n + 2 * Ng for n in N) + (8,))
+    it = (slice(Ng, -Ng),) * 3
+    P[it] = [1.0, 0.6, 0.1, -0.05, 0.08, 0.3, 0.2, 0.4]
+    P[it] *= 1.0 + 0.02 * rng.uniform(-1, 1, tuple(N) + (8,))
+    P = synchronize(P, Ng)
+    so = oracle_lib.solver(Setup(N=N, Ng=Ng, extrap=extrap, riemann=riemann, advance="rk3"))
+    ctx = gpu.Context(gpu.make_config(N=N, Ng=Ng, extrap=extrap, riemann=riemann, advance="rk3", precision=precision))
+    ctx.upload(P)
+    Po, dt = P.copy(), 0.1 / max(N)
+    for _ in range(2):
+        eo, sto = so.advance(Po, dt)
+        eg, stg = ctx.advance(dt)
+        assert eo == eg == 0
+        tol = 1e-12 if precision == "fp64" else 1e-5
+        assert abs(stg.max_lambda - sto.max_lambda) <= tol * sto.max_lambda
+    Pg = ctx.download()
+    L1 = np.abs(Pg - Po).sum(axis=(0, 1, 2)) / np.abs(Po).sum(axis=(0, 1, 2))
+    assert L1.max() < (1e-10 if precision == "fp64" else 1e-6)
+
+
+@pytest.mark.parametrize("riemann", ["hll", "hlld"])
+def test_single_zone(gpu, riemann):
+    """One zone with one ghost zone a side: no interface along x at all (an empty range of
+    blocks), and a uniform state, which no step changes beyond round-off."""
+    P = np.tile(np.array([1.0, 0.6, 0.1, -0.05, 0.08, 0.3, 0.2, 0.4]), (3, 3, 3, 1))
+    ctx = gpu.Context(gpu.make_config(N=(1, 1, 1), Ng=1, extrap="pcm", riemann=riemann, advance="rk3"))
+    ctx.upload(P)
+    for _ in range(2):
+        assert ctx.advance(0.1)[0] == 0
+    assert np.abs(ctx.download() - P).max() < 1e-14
