@@ -499,11 +499,11 @@ __device__ __forceinline__ int riemann_dispatch(int solver, const R *pl, const R
 /* One interface z | z+S of the sweep along `axis`: reconstruction from the 6-point stencil,
  * the Riemann solve, and the retry with the zone-centred states of the two neighbours
  * (Mara/plm-split.cpp:51-71). F in the axis's frame. Returns the error of the last attempt
- * (flux 0 then). */
-template <typename R, int SOLVER>
+ * (flux 0 then). GROUP: HLLD by 16 lanes with the same z; the lead lane has the result. */
+template <typename R, int SOLVER, bool GROUP = false>
 __device__ __forceinline__ int interface_flux(const double *__restrict__ P, long T, long S, int axis, long z, int recon,
                                               const PhysParams &pp, R *F, R &lam, FluxCounters &fc,
-                                              int &retried)
+                                              int &retried, bool *lead = nullptr)
 {
   R ql[8], qr[8];
   reconstruct_states<R, false>(P, T, S, axis, z, recon, pp, ql, qr);
@@ -521,7 +521,11 @@ __device__ __forceinline__ int interface_flux(const double *__restrict__ P, long
         qr[q] = (R)v[S];
       }
     }
-    err = riemann_dispatch<R, 1>(SOLVER, ql, qr, F, (R)pp.gamma, pp.pfloor, lam, fc);
+    if constexpr (GROUP) {
+      *lead = (threadIdx.x & 15) == 0;
+      err = riemann_hlld<R, 1, false, true>(ql, qr, F, (R)pp.gamma, pp.pfloor, lam, fc, lead);
+    }
+    else err = riemann_dispatch<R, 1>(SOLVER, ql, qr, F, (R)pp.gamma, pp.pfloor, lam, fc);
   }
   if (err) {
 #pragma unroll
@@ -787,10 +791,15 @@ __global__ __launch_bounds__(kBlock) void k_flux_redo(const double *__restrict__
     cnt[5] += (unsigned long long)(v.w & 0xffffu);
   }
   const long T = g.T;
-  // k counts through the three lists
+  // k counts through the three lists. Up to 4096 interfaces (16 lanes each fill the grid once)
+  // the kernel is bound by the latency of one interface's attempt ladder, and 16 lanes share
+  // an interface: 52 -> 29 us for the 8 a stage of a 64^3 step, 105 -> 39 us at 131x94x113.
+  // Above, one lane each, dealt out over the waves first, so that every SIMD has a few.
   const unsigned int n0 = min(rq.count[0], rq.cap), n1 = min(rq.count[1], rq.cap), n2 = min(rq.count[2], rq.cap);
   const unsigned long n = (unsigned long)n0 + n1 + n2;
-  for (unsigned long k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+  const unsigned tid = blockIdx.x * blockDim.x + threadIdx.x, nthreads = gridDim.x * blockDim.x;
+  auto redo = [&](unsigned long k, auto group) {
+    constexpr bool GROUP = decltype(group)::value;
     const int axis = k < n0 ? 0 : k < (unsigned long)n0 + n1 ? 1 : 2;
     const unsigned long i = axis == 0 ? k : axis == 1 ? k - n0 : k - n0 - n1;
     const long z = (long)rq.z[(size_t)axis * rq.cap + i];
@@ -798,7 +807,10 @@ __global__ __launch_bounds__(kBlock) void k_flux_redo(const double *__restrict__
     FluxCounters fc = {0, 0, 0, 0};
     double F[8];
     int retried;
-    const int err = interface_flux<double, SOLVER>(P, T, axis_stride(g, axis), axis, z, recon, pp, F, lam, fc, retried);
+    bool lead = true;
+    const int err = interface_flux<double, SOLVER, GROUP>(P, T, axis_stride(g, axis), axis, z, recon, pp, F, lam, fc,
+                                                          retried, &lead);
+    if (!lead) return;
     FT *__restrict__ Fout = axis == 0 ? Fo.f[0] : axis == 1 ? Fo.f[1] : Fo.f[2];
 #pragma unroll
     for (int q = 0; q < 8; ++q) Fout[axis_plane(q, axis) * T + z] = (FT)F[q];
@@ -810,7 +822,11 @@ __global__ __launch_bounds__(kBlock) void k_flux_redo(const double *__restrict__
     cnt[4] += (unsigned long long)fc.c2p_iters;
     cnt[5] += (unsigned long long)fc.newton_iters;
     cnt[6] += 1;
-  }
+  };
+  if (n * 16 <= nthreads)
+    for (unsigned long k = tid >> 4; k < n; k += nthreads >> 4) redo(k, std::true_type());
+  else
+    for (unsigned long k = (tid & 63) * (nthreads >> 6) + (tid >> 6); k < n; k += nthreads) redo(k, std::false_type());
   block_max_lambda(lam_out, &st->lam_bits);
   unsigned long long *const dst[7] = { &st->hlld_success, &st->hlld_failure, &st->retries,
                                        &st->failures, &st->hlld_c2p_iters, &st->hlld_newton_iters,

@@ -1230,6 +1230,19 @@ template <typename R, int DIM> __device__ __forceinline__ int riemann_hllc(const
   return 0;
 }
 
+/* lane K of the calling lane's quad to all four (a DPP move; every lane of the quad is active) */
+template <int K> __device__ __forceinline__ int quad_bcast(int v)
+{
+  return __builtin_amdgcn_update_dpp(0, v, K * 0x55, 0xF, 0xF, false);
+}
+template <int K> __device__ __forceinline__ double quad_bcast(double v)
+{
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)quad_bcast<K>((int)(unsigned)b), hi = (unsigned)quad_bcast<K>((int)(unsigned)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <int K> __device__ __forceinline__ float quad_bcast(float v) { return __int_as_float(quad_bcast<K>(__float_as_int(v))); }
+
 /* HLLD (Mignone, Ugliano & Bodo 2008), Mara/riemann_hlld-rmhd.cpp:143-579, in the
  * x-normal frame. Holds the jump states across the fast waves (eqn 12). */
 template <typename R> struct Hlld {
@@ -1332,7 +1345,10 @@ template <typename R> struct Hlld {
    * FP32 (the mixed form) takes the derivative by a one-sided difference from the residual
    * already evaluated: two evaluations per step instead of three, the same L1 error; and it
    * takes a start whose residual is below newton_accept as the root without a step.
-   * max_it: the reference's 15, fewer on the FP32 common path (Tol<float>). */
+   * max_it: the reference's 15, fewer on the FP32 common path (Tol<float>).
+   * GROUP: the four lanes of a quad hold the same problem, and each evaluates the residual at
+   * one of the three points (see riemann_hlld). */
+  template <bool GROUP = false>
   __device__ __forceinline__ bool newton(R &x, int &iters, int max_it = 15) const
   {
     using T = Tol<R>;
@@ -1346,6 +1362,18 @@ template <typename R> struct Hlld {
       // FP32: the residual, then (one-sided) f(x + dp); FP64: the reference's f(x),
       // f(x - dp/2), f(x + dp/2)
       constexpr int nev = T::fd_one_sided ? 2 : 3;
+      if constexpr (GROUP) {
+        static_assert(!GROUP || !T::fd_one_sided, "the FP64 form");
+        const int k = (int)(threadIdx.x & 3);
+        const R pk = k == 1 ? x - R(0.5)*dp : k == 2 ? x + R(0.5)*dp : x;
+        R fk = R(0);
+        const int fine = function(pk, fk) ? 1 : 0;
+        y = quad_bcast<0>(fk);
+        f0 = quad_bcast<1>(fk);
+        f1 = quad_bcast<2>(fk);
+        ok = (quad_bcast<0>(fine) & quad_bcast<1>(fine) & quad_bcast<2>(fine)) != 0;
+      }
+      else
 #pragma unroll Shape<R>::unroll
       for (int k = 0; k < nev; ++k) {
         const R pk = k == 0 ? x : (T::fd_one_sided ? x + dp : (k == 1 ? x - R(0.5)*dp : x + R(0.5)*dp));
@@ -1512,17 +1540,24 @@ struct FluxCounters {
  * nested c2p, after which the outer U and F are dead; only the primitive states are
  * kept (to rebuild the flux side at the end and for the HLLC fallback, which averages
  * the normal field exactly as here, riemann_hllc-rmhd.cpp:60).
- * FAST = true (the FP32 sweeps; FP64 has riemann_hlld_lean) is the common path alone: the nested c2p from the average state and the
- * first Newton attempt from EstimateSolution(0), or with a small normal field the flux at
- * EstimateSolution(1). Anything else (an invalid state, the c2p cascade, attempts 2 and
+ * FAST = true (the FP32 sweeps; FP64 has riemann_hlld_lean) is the common path alone: the
+ * nested c2p from the average state and the first Newton attempt from EstimateSolution(0), or
+ * with a small normal field the flux at EstimateSolution(1). Anything else (an invalid state, the c2p cascade, attempts 2 and
  * 3, the HLLC fallback) returns kHlldDefer without writing f; the caller hands the
  * interface to the full solver, which then takes the same steps up to that point and
- * gives the same result. */
+ * gives the same result.
+ * GROUP = true runs the attempt ladder of one interface on 16 lanes (a row of the wave) that
+ * hold the same states: each quad takes one attempt (the fourth repeats the third), each lane
+ * of a quad one of the three residual evaluations of its Newton steps. The first attempt in
+ * the reference's order that succeeded supplies the flux, so the result is the serial one; f
+ * and the counters are returned in the lane for which `lead` is set. The ladder is a serial
+ * chain (up to 3 x 16 x 3 evaluations of some 250 dependent instructions, 50-70 us), and a
+ * handful of interfaces that need it would hold the stage that long. */
 constexpr int kHlldDefer = 100;   // common path: the interface needs the full solver
 
-template <typename R, int DIM, bool FAST = false>
+template <typename R, int DIM, bool FAST = false, bool GROUP = false>
 __device__ __forceinline__ int riemann_hlld(const R *pl, const R *pr, R *f, R gamma, double pfloor, R &lam,
-                                            FluxCounters &cnt)
+                                            FluxCounters &cnt, bool *lead = nullptr)
 {
   using T = Tol<R>;
   using Pm = Perm<DIM>;
@@ -1670,6 +1705,23 @@ __device__ __forceinline__ int riemann_hlld(const R *pl, const R *pr, R *f, R ga
       }
       if (!success) return kHlldDefer;
     }
+    if constexpr (GROUP) {
+      const int row = (int)(threadIdx.x & 15);
+      const int attempt = row < 12 ? row >> 2 : 2;
+      R p_star = attempt == 0 ? est0 : R(0);
+      if (small_bn || attempt == 1) p_star = estimate1();
+      int it = 0;
+      success = small_bn ? e.flux(p_star, Pl, Pr, gamma, Fx)
+                         : e.template newton<true>(p_star, it) && e.flux(p_star, Pl, Pr, gamma, Fx);
+      const unsigned m = (unsigned)(__ballot(success) >> (threadIdx.x & 48)) & 0xfffu;
+      const int taken = m ? (__ffs((int)m) - 1) >> 2 : 2;       // the ladder's last attempt
+      *lead = row == 4 * taken;
+      success = m != 0u;
+      // the lead's own iterations and those of the attempts before its own
+      const int i0 = __shfl(it, 0, 16), i1 = __shfl(it, 4, 16), i2 = __shfl(it, 8, 16);
+      cnt.newton_iters += taken == 0 ? i0 : taken == 1 ? i0 + i1 : i0 + i1 + i2;
+    }
+    else
 #pragma unroll Shape<R>::unroll
     for (int attempt = 0; attempt < (FAST ? 0 : 3) && !success; ++attempt) {
       R p_star;

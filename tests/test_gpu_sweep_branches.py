@@ -110,3 +110,45 @@ def test_single_zone(gpu, riemann):
     for _ in range(2):
         assert ctx.advance(0.1)[0] == 0
     assert np.abs(ctx.download() - P).max() < 1e-14
+
+
+@pytest.mark.parametrize("n", [8, 38])
+def test_full_solver_queue(gpu, oracle_lib, n):
+    """Rough states, whose interfaces leave the common path in number: few enough that the full
+    solver gives each 16 lanes (n = 8), and more than 4096 in a launch, one lane each (n = 38).
+    The HLLD counts and the state after one small step against the oracle, held to 4x its own
+    spread under 1-ulp noise (the attempt ladder flips there) or the plain tolerances."""
+    rng = np.random.default_rng(n)
+    N = (n, n, n)
+    P = np.empty((n + 6,) * 3 + (8,))
+    it = (slice(3, -3),) * 3
+    r = rng.uniform(-1, 1, N + (8,))
+    P[it + (0,)] = np.exp(1.5 * r[..., 0])
+    P[it + (1,)] = np.exp(2.0 * r[..., 1])
+    P[it + (slice(2, 5),)] = 0.5 * r[..., 2:5]
+    P[it + (slice(5, 8),)] = 2.0 * r[..., 5:8]
+    P = synchronize(P, 3)
+    kw = dict(N=N, extrap="plm", riemann="hlld", advance="single")
+
+    def step(P0):
+        so = oracle_lib.solver(Setup(**kw))
+        Q = P0.copy()
+        e, st = so.advance(Q, 1e-3 / n)
+        return e, st.hlld_success, st.hlld_failure, Q
+
+    e0, ok0, fail0, Q0 = step(P)
+    L1 = lambda Q: np.abs(Q - Q0).sum(axis=(0, 1, 2)) / np.abs(Q0).sum(axis=(0, 1, 2))  # noqa: E731
+    ok_tol, tol = 2.0, np.full(8, 1e-10)
+    for _ in range(8):
+        e, ok, fail, Q = step(P * (1 + 2.3e-16 * rng.choice([-1, 0, 1], size=P.shape)))
+        ok_tol = max(ok_tol, 4 * abs(ok - ok0))
+        tol = np.maximum(tol, 4 * L1(Q))
+    assert e0 == 0 and fail0 > (100 if n == 8 else 6000)
+    ctx = gpu.Context(gpu.make_config(**kw))
+    ctx.upload(P)
+    eg, st = ctx.advance(1e-3 / n)
+    assert eg == 0
+    assert (st.fp64_redo <= 4096) == (n == 8)
+    assert st.hlld_success + st.hlld_failure == ok0 + fail0
+    assert abs(st.hlld_success - ok0) <= ok_tol
+    assert (L1(ctx.download()) <= tol).all()
