@@ -1591,7 +1591,7 @@ __global__ __launch_bounds__(kBlock, MODE == C2P_NET ? 3 : 4) void k_p2c_c2p(con
  * result does not change from run to run. */
 constexpr int kMeasSums = 28, kMeasExt = 5, kMeasQ = kMeasSums + kMeasExt, kMeasBlocks = 1024;
 constexpr int kCoolBlocks = 1024;      // grid of k_cool and k_power (grid-stride), rows of their partial sums
-constexpr int kOuMaxK1 = 6;            // (2 k1 + 1)^3 modes x 48 B of amplitudes in LDS
+constexpr int kOuMaxK1 = 6;            // the sampling kernels' largest k1
 
 struct MeasureUnits { double ErgPerCC, GramsPerCC, mp, kb, K2MeV; };
 
@@ -1781,40 +1781,88 @@ __device__ __forceinline__ double2 cmul(double2 a, double2 b)
 }
 
 /* DrivingProcedure::ResampleField (Mara/driving.cpp:44-85): the field at every zone centre,
- * ghosts included, F(x) = Re sum_m F_m exp(i k_m . x), summed from the last mode to the
- * first as the reference's valarray expression is. exp(i k . x) is the product of per-axis
- * factors exp(2 pi i n x) from tables (ex, ey, ez: 2 k1 + 1 per zone index), which differs
- * from the exponential of the summed phase by round-off. The amplitudes (3 numk complex
- * numbers, axis-major) are staged in LDS. */
-__global__ __launch_bounds__(kBlock) void k_ou_sample(const double2 *__restrict__ ex, const double2 *__restrict__ ey,
-                                                      const double2 *__restrict__ ez, const double2 *__restrict__ amp,
-                                                      int k1, GridDesc g, double *__restrict__ Fd)
+ * ghosts included, F(x) = Re sum_m F_m exp(i k_m . x). exp(i k . x) is the product of per-axis
+ * factors exp(2 pi i n x), so the sum over the (2 k1 + 1)^3 modes is taken one axis at a time:
+ *   k_ou_phases   the factors at every zone index of each axis
+ *   k_ou_sum_z    G[q][a][b][k] = sum_c F_abc e_c(k), one per z index
+ *   k_ou_sum_y    H[q][a][j][k] = sum_b e_b(j) G[q][a][b][k], one per (y, z) column
+ *   k_ou_sum_x    F[q](i, j, k) = Re sum_a e_a(i) H[q][a][j][k]
+ * A zone then costs 3 (2 k1 + 1) complex multiply-adds instead of 3 (2 k1 + 1)^3, and writing
+ * the field is what bounds it: at k1 = 3 and 128^3 (2.4 M zones with ghosts) 685 us by the sum
+ * over the modes at every zone, 21 + 7 us and two short launches so (2.7 TB/s written). Modes are added from the last to the first along each axis, as
+ * the reference's valarray expression adds them; fewer additions and factors enter a value
+ * than in the full sum, so it rounds no worse. */
+__global__ __launch_bounds__(kBlock) void k_ou_phases(double2 *__restrict__ tab, GridDesc g, double x0, double x1,
+                                                      double x2, double d0, double d1, double d2, int k1)
 {
-  extern __shared__ double2 sh_amp[];
-  const int nk = 2 * k1 + 1, numk = nk * nk * nk;
-  for (int t = threadIdx.x; t < 3 * numk; t += blockDim.x) sh_amp[t] = amp[t];
-  __syncthreads();
-  const long z = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (z >= g.T) return;
-  const long k = z % g.n[2], j = (z / g.n[2]) % g.n[1], i = z / ((long)g.n[1] * g.n[2]);
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-  for (int a = nk - 1; a >= 0; --a) {
-    const double2 X = ex[i * nk + a];
-    for (int b = nk - 1; b >= 0; --b) {
-      const double2 xy = cmul(X, ey[j * nk + b]);
-      for (int c = nk - 1; c >= 0; --c) {
-        const double2 e = cmul(xy, ez[k * nk + c]);
-        const int m = (a * nk + b) * nk + c;
-        const double2 fx = sh_amp[m], fy = sh_amp[numk + m], fz = sh_amp[2 * numk + m];
-        s0 += fx.x * e.x - fx.y * e.y;
-        s1 += fy.x * e.x - fy.y * e.y;
-        s2 += fz.x * e.x - fz.y * e.y;
-      }
+  const int nk = 2 * k1 + 1;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (g.n[0] + g.n[1] + g.n[2]) * nk) return;
+  int i = t / nk;
+  const int a = t % nk;
+  const int d = i < g.n[0] ? 0 : i < g.n[0] + g.n[1] ? 1 : 2;
+  i -= d == 0 ? 0 : d == 1 ? g.n[0] : g.n[0] + g.n[1];
+  // x_at (Mara/simple-cart.hpp:42-44)
+  const double x = (d == 0 ? x0 : d == 1 ? x1 : x2) + (d == 0 ? d0 : d == 1 ? d1 : d2) * (i - g.Ng + 0.5);
+  double sn, cs;
+  sincos((2 * M_PI * (a - k1)) * x, &sn, &cs);
+  tab[t] = make_double2(cs, sn);
+}
+
+__device__ __forceinline__ void cfma(double2 &s, double2 a, double2 b)
+{
+  s.x += a.x * b.x - a.y * b.y;
+  s.y += a.x * b.y + a.y * b.x;
+}
+
+template <int NK>
+__global__ __launch_bounds__(kBlock) void k_ou_sum_z(const double2 *__restrict__ ez, const double2 *__restrict__ amp,
+                                                     int n2, double2 *__restrict__ G)
+{
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;       // (q, a, b, k)
+  if (t >= 3 * NK * NK * n2) return;
+  const int k = t % n2, qab = t / n2;
+  double2 s = make_double2(0.0, 0.0);
+#pragma unroll
+  for (int c = NK - 1; c >= 0; --c) cfma(s, ez[k * NK + c], amp[qab * NK + c]);
+  G[t] = s;
+}
+
+template <int NK>
+__global__ __launch_bounds__(kBlock) void k_ou_sum_y(const double2 *__restrict__ ey, const double2 *__restrict__ G,
+                                                     int n1, int n2, double2 *__restrict__ H)
+{
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;   // (q, a, j, k)
+  if (t >= (long)3 * NK * n1 * n2) return;
+  const int k = (int)(t % n2), j = (int)((t / n2) % n1), qa = (int)(t / ((long)n1 * n2));
+  double2 s = make_double2(0.0, 0.0);
+#pragma unroll
+  for (int b = NK - 1; b >= 0; --b) cfma(s, ey[j * NK + b], G[(qa * NK + b) * n2 + k]);
+  H[t] = s;
+}
+
+/* blockIdx.y takes kOuPlanes consecutive i: a thread keeps its column's sums and adds them up
+ * with each plane's factors, which are uniform */
+constexpr int kOuPlanes = 16;
+template <int NK>
+__global__ __launch_bounds__(kBlock) void k_ou_sum_x(const double2 *__restrict__ ex, const double2 *__restrict__ H,
+                                                     GridDesc g, double *__restrict__ Fd)
+{
+  const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;   // (j, k)
+  if (r >= g.sx) return;
+  const int i0 = blockIdx.y * kOuPlanes, i1 = min(i0 + kOuPlanes, g.n[0]);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    double2 h[NK];
+#pragma unroll
+    for (int a = 0; a < NK; ++a) h[a] = H[(q * NK + a) * g.sx + r];
+    for (int i = i0; i < i1; ++i) {
+      double s = 0.0;
+#pragma unroll
+      for (int a = NK - 1; a >= 0; --a) s += ex[i * NK + a].x * h[a].x - ex[i * NK + a].y * h[a].y;
+      Fd[q * g.T + i * g.sx + r] = s;
     }
   }
-  Fd[z] = s0;
-  Fd[g.T + z] = s1;
-  Fd[2 * g.T + z] = s2;
 }
 
 /* The field at n arbitrary points (xyz, 3 per point): the per-axis factors are formed per
@@ -2141,6 +2189,8 @@ struct maragpu_ctx {
   double *ctuU = nullptr, *ctuP = nullptr;
   // driving (DrivingProcedure): the field sampled at every zone, 3 planes of T doubles
   double *Fdrive = nullptr;
+  void *ou = nullptr;                // the sampling's workspace and its size
+  size_t ou_cap = 0;
   // cooling (CoolingModuleT4 / E4): kind 0 none, 1 T4, 2 E4; per-block partials of the
   // energy removed and, after them, its running total since the last read
   int cool_kind = 0;
@@ -2383,6 +2433,7 @@ int maragpu_destroy(maragpu_ctx *c)
   hipFree(c->ctuU);
   hipFree(c->ctuP);
   hipFree(c->Fdrive);
+  hipFree(c->ou);
   hipFree(c->dcool);
   for (auto &e : c->ev) if (e) hipEventDestroy(e);
   if (c->stream) hipStreamDestroy(c->stream);
@@ -2757,39 +2808,59 @@ int maragpu_measure_noalloc(maragpu_ctx *c, const double *units, maragpu_measure
   return measure_into(c, units, out, g_measure_scratch[c->device]);
 }
 
+}  // extern "C"
+
 namespace {
-/* per-axis tables exp(2 pi i n x) at the zone centres x_at (Mara/simple-cart.hpp:42-44) for
- * n = -k1..k1, and the amplitudes (axis-major), on the device */
-int ou_tables(const maragpu_host::OuField &f, const GridDesc &g, const maragpu_config &cfg, DevBuf &tab,
-              DevBuf &amp)
+/* the field's samples at every zone into c->Fdrive, with c->ou as workspace: the factors, the
+ * amplitudes (axis-major, as the modes are held), G and H */
+template <int NK> size_t ou_bytes(const GridDesc &g)
 {
-  const int nk = 2 * f.k1 + 1;
-  std::vector<double2> h;
-  for (int d = 0; d < 3; ++d) {
-    const double dx = (cfg.x1[d] - cfg.x0[d]) / cfg.N[d];
-    for (int i = 0; i < g.n[d]; ++i) {
-      const double x = cfg.x0[d] + dx * (i - g.Ng + 0.5);
-      for (int a = 0; a < nk; ++a) {
-        const double ph = (2 * M_PI * (a - f.k1)) * x;
-        h.push_back(make_double2(std::cos(ph), std::sin(ph)));
-      }
-    }
+  return sizeof(double2) * ((size_t)(g.n[0] + g.n[1] + g.n[2]) * NK + (size_t)3 * NK * NK * NK +
+                            (size_t)3 * NK * NK * g.n[2] + (size_t)3 * NK * g.sx);
+}
+
+template <int NK> int ou_sample(maragpu_ctx *c, const maragpu_host::OuField &f)
+{
+  const GridDesc &g = c->g;
+  const maragpu_config &cfg = c->cfg;
+  const size_t bytes = ou_bytes<NK>(g);
+  if (c->ou_cap < bytes) {
+    hipFree(c->ou);
+    c->ou = nullptr;
+    c->ou_cap = 0;
+    if (hipMalloc(&c->ou, bytes) != hipSuccess) { c->ou = nullptr; return MARAGPU_E_NOMEM; }
+    c->ou_cap = bytes;
   }
-  std::vector<double2> ha(3 * (size_t)f.numk);
-  for (size_t q = 0; q < ha.size(); ++q) ha[q] = make_double2(f.F[2 * q], f.F[2 * q + 1]);
-  if (dalloc(tab, h.size() * sizeof(double2)) || dalloc(amp, ha.size() * sizeof(double2))) return MARAGPU_E_NOMEM;
-  HIP_CHECK(hipMemcpy(tab.p, h.data(), h.size() * sizeof(double2), hipMemcpyHostToDevice));
-  HIP_CHECK(hipMemcpy(amp.p, ha.data(), ha.size() * sizeof(double2), hipMemcpyHostToDevice));
+  const int ntab = (g.n[0] + g.n[1] + g.n[2]) * NK;
+  double2 *tab = static_cast<double2 *>(c->ou), *amp = tab + ntab, *G = amp + 3 * NK * NK * NK,
+          *H = G + (size_t)3 * NK * NK * g.n[2];
+  double dx[3];
+  for (int d = 0; d < 3; ++d) dx[d] = (cfg.x1[d] - cfg.x0[d]) / cfg.N[d];
+  HIP_CHECK(hipMemcpyAsync(amp, f.F.data(), (size_t)3 * NK * NK * NK * sizeof(double2), hipMemcpyHostToDevice, c->stream));
+  k_ou_phases<<<nblocks(ntab), kBlock, 0, c->stream>>>(tab, g, cfg.x0[0], cfg.x0[1], cfg.x0[2], dx[0], dx[1], dx[2],
+                                                       (NK - 1) / 2);
+  const double2 *ey = tab + (size_t)g.n[0] * NK, *ez = ey + (size_t)g.n[1] * NK;
+  k_ou_sum_z<NK><<<nblocks((long)3 * NK * NK * g.n[2]), kBlock, 0, c->stream>>>(ez, amp, g.n[2], G);
+  k_ou_sum_y<NK><<<nblocks(3 * NK * g.sx), kBlock, 0, c->stream>>>(ey, G, g.n[1], g.n[2], H);
+  const dim3 nb(nblocks(g.sx), (unsigned)((g.n[0] + kOuPlanes - 1) / kOuPlanes));
+  k_ou_sum_x<NK><<<nb, kBlock, 0, c->stream>>>(tab, H, g, c->Fdrive);
+  HIP_CHECK(hipGetLastError());
+  HIP_CHECK(hipStreamSynchronize(c->stream));
   return MARAGPU_OK;
 }
 }  // namespace
+
+extern "C" {
 
 int maragpu_set_driving(maragpu_ctx *c, const maragpu_ou_field *field)
 {
   if (!c) return MARAGPU_E_INVALID;
   if (!field) {
     hipFree(c->Fdrive);
+    hipFree(c->ou);
     c->Fdrive = nullptr;
+    c->ou = nullptr;
+    c->ou_cap = 0;
     return MARAGPU_OK;
   }
   const maragpu_host::OuField &f = *maragpu_ou_field_modes(field);
@@ -2799,15 +2870,15 @@ int maragpu_set_driving(maragpu_ctx *c, const maragpu_ou_field *field)
     c->Fdrive = nullptr;
     return MARAGPU_E_NOMEM;
   }
-  DevBuf tab, amp;
-  if (int rc = ou_tables(f, g, c->cfg, tab, amp)) return rc;
-  const int nk = 2 * f.k1 + 1;
-  const double2 *t = tab.get<double2>();
-  k_ou_sample<<<nblocks(g.T), kBlock, 3 * f.numk * sizeof(double2), c->stream>>>(
-      t, t + (size_t)g.n[0] * nk, t + (size_t)(g.n[0] + g.n[1]) * nk, amp.get<double2>(), f.k1, g, c->Fdrive);
-  HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipStreamSynchronize(c->stream));
-  return MARAGPU_OK;
+  switch (f.k1) {
+  case 0: return ou_sample<1>(c, f);
+  case 1: return ou_sample<3>(c, f);
+  case 2: return ou_sample<5>(c, f);
+  case 3: return ou_sample<7>(c, f);
+  case 4: return ou_sample<9>(c, f);
+  case 5: return ou_sample<11>(c, f);
+  default: return ou_sample<13>(c, f);
+  }
 }
 
 int maragpu_driving_power(maragpu_ctx *c, double *power)

@@ -116,3 +116,29 @@ def test_driving_verbs_like_drvtrb(gpu, oracle_lib):
     rate = Mara.cooling_rate(0.5)
     assert abs(rate - removed_o / 0.5) <= 1e-11 * abs(removed_o / 0.5)
     Mara.close()
+
+
+def test_sampling_every_k1(gpu):
+    """set_driving's axis-by-axis sums for each size of field it takes (k1 = 0..6, one context,
+    so the workspace grows and shrinks), on an offset domain with three different sizes, and
+    kb_ou_sample's direct sum at the same points: mean |F|^2 over all zones, ghosts included, to
+    1e-12 (both sum (2 k1 + 1)^3 products in FP64), and the driven velocities to 1e-13."""
+    N, Ng, x0, x1 = (5, 18, 9), 3, (-0.3, 0.1, 0.0), (0.7, 2.1, 1.5)
+    x = [x0[d] + (x1[d] - x0[d]) / N[d] * (np.arange(N[d] + 2 * Ng) - Ng + 0.5) for d in range(3)]
+    xyz = np.stack(np.meshgrid(*x, indexing="ij"), axis=-1).reshape(-1, 3)
+    ctx = gpu.Context(gpu.make_config(N=N, Ng=Ng, x0=x0, x1=x1, extrap="plm", riemann="hll", advance="single"))
+    P = np.tile(np.array([1.0, 1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0]), tuple(n + 2 * Ng for n in N) + (1,))
+    for k1 in (6, 0, 1, 2, 3, 4, 5):
+        field = gpu.OuField.create(0.3, 1.0, k1, 40 + k1)
+        field.advance(0.2)
+        F = field.sample(xyz)
+        ctx.upload(P)
+        ctx.set_driving(field)
+        power = (F ** 2).sum(axis=1).mean()
+        assert abs(ctx.driving_power() - power) <= 1e-12 * max(power, 1e-300)
+        assert ctx.advance(1e-2)[0] == 0
+        # at rest, u = F dt exactly: v = u / sqrt(1 + u^2)
+        u = F * 1e-2
+        v = u / np.sqrt(1.0 + (u ** 2).sum(axis=1, keepdims=True))
+        got = ctx.download()[..., 2:5].reshape(-1, 3)
+        assert np.abs(got - v).max() <= 1e-13 * max(np.abs(v).max(), 1e-3)
