@@ -40,9 +40,12 @@
 #include "mlp_device.hpp"
 #include "eigensystem_device.hpp"
 #include "ou_field.hpp"
+#include "host_copy.hpp"
 #include "../../include/maragpu.h"
 
 using namespace maragpu;
+using maragpu_host::copy_to_device;
+using maragpu_host::copy_to_host;
 
 namespace {
 
@@ -2349,10 +2352,11 @@ int maragpu_create(const maragpu_config *cfg, maragpu_ctx **out)
   maragpu_ctx *c = new (std::nothrow) maragpu_ctx;
   if (!c) return MARAGPU_E_NOMEM;
   c->device = dev;
+  maragpu_host::staging_retain(dev);
   c->cfg = *cfg;
   c->g = make_grid(*cfg);
-  if (c->g.T >= (1L << 32)) { delete c; return MARAGPU_E_INVALID; }   // 32-bit queue slots
-  if (hipStreamCreate(&c->stream) != hipSuccess) { delete c; return MARAGPU_E_HIP; }
+  if (c->g.T >= (1L << 32)) { maragpu_host::staging_release(dev); delete c; return MARAGPU_E_INVALID; }   // 32-bit queue slots
+  if (hipStreamCreate(&c->stream) != hipSuccess) { maragpu_host::staging_release(dev); delete c; return MARAGPU_E_HIP; }
   const size_t nd = 8 * (size_t)c->g.T;
   const size_t fbytes = nd * (cfg->precision == MARAGPU_MIXED ? sizeof(float) : sizeof(double));
   if (hipMalloc(&c->Pc, nd * sizeof(double)) != hipSuccess) return fail_free(c);
@@ -2437,6 +2441,7 @@ int maragpu_destroy(maragpu_ctx *c)
   hipFree(c->dcool);
   for (auto &e : c->ev) if (e) hipEventDestroy(e);
   if (c->stream) hipStreamDestroy(c->stream);
+  maragpu_host::staging_release(c->device);
   delete c;
   return MARAGPU_OK;
 }
@@ -2445,7 +2450,7 @@ int maragpu_upload_prim(maragpu_ctx *c, const double *P, size_t n)
 {
   if (!c || !P) return MARAGPU_E_INVALID;
   if (n != 8 * (size_t)c->g.T) return MARAGPU_E_SIZE;
-  HIP_CHECK(hipMemcpyAsync(c->U0, P, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  HIP_CHECK(copy_to_device(c->device, c->stream, c->U0, P, n * sizeof(double)));
   k_aos_to_soa<<<nblocks(c->g.T), kBlock, 0, c->stream>>>(c->U0, c->Pc, c->g.T);
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipStreamSynchronize(c->stream));
@@ -2459,8 +2464,7 @@ int maragpu_download_prim(maragpu_ctx *c, double *P, size_t n)
   if (n != 8 * (size_t)c->g.T) return MARAGPU_E_SIZE;
   k_soa_to_aos<<<nblocks(c->g.T), kBlock, 0, c->stream>>>(c->Pc, c->U0, c->g.T);
   HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipMemcpyAsync(P, c->U0, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIP_CHECK(hipStreamSynchronize(c->stream));
+  HIP_CHECK(copy_to_host(c->device, c->stream, P, c->U0, n * sizeof(double)));
   return MARAGPU_OK;
 }
 
@@ -2480,8 +2484,7 @@ int maragpu_download_field(maragpu_ctx *c, int q, double *out, size_t n)
   // U0 (8 T doubles) is staging outside an advance
   k_field_out<<<nblocks(ni), kBlock, 0, c->stream>>>(c->Pc + (size_t)q * g.T, c->U0, g);
   HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipMemcpyAsync(out, c->U0, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIP_CHECK(hipStreamSynchronize(c->stream));
+  HIP_CHECK(copy_to_host(c->device, c->stream, out, c->U0, n * sizeof(double)));
   return MARAGPU_OK;
 }
 
@@ -2491,7 +2494,7 @@ int maragpu_upload_field(maragpu_ctx *c, int q, const double *in, size_t n)
   const GridDesc &g = c->g;
   const long ni = (long)g.N[0] * g.N[1] * g.N[2];
   if (n != (size_t)ni) return MARAGPU_E_SIZE;
-  HIP_CHECK(hipMemcpyAsync(c->U0, in, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  HIP_CHECK(copy_to_device(c->device, c->stream, c->U0, in, n * sizeof(double)));
   k_field_in<<<nblocks(ni), kBlock, 0, c->stream>>>(c->U0, c->Pc + (size_t)q * g.T, g);
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipStreamSynchronize(c->stream));
