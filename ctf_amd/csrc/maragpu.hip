@@ -16,9 +16,10 @@
  *                     c2p pass, its result written to the zone and its periodic ghost
  *                     images (replaces Synchronize + per-zone c2p)
  * then per RK stage:
- *   k_flux<DIM> x 3   per interface over the reference's flat sweep range
- *                     (Mara/plm-split.cpp:48): reconstruct 8 fields, Riemann solve,
- *                     PCM retry, max |lambda| (for HLLD: k_flux_hlld_fast + k_flux_redo)
+ *   k_flux_fast       per interface of the three axes over the reference's flat sweep ranges
+ *                     (Mara/plm-split.cpp:48): reconstruct 8 fields, Riemann solve, max
+ *                     |lambda|; k_flux_redo does those that leave the common path (PCM retry,
+ *                     the rare branches of HLLD)
  *   k_update_c2p      per interior zone: constrained-transport EMF averages
  *                     (Mara/rmhd.cpp:293-337), flux divergence (plm-split.cpp:117-119) and
  *                     the RK stage combination (Mara/runge-kutta.hpp), all in FP64, then
@@ -50,15 +51,21 @@ using maragpu_host::copy_to_host;
 namespace {
 
 constexpr int kBlock = 256;
-// block size of k_flux_hlld_fast (it ends without a block barrier): FP64 in one-wave blocks
+// block size of k_flux_fast (it ends without a block barrier): FP64 in one-wave blocks
 // (1.55 ms for the slowest 256^3 sweep, 1.67 with 4-wave blocks), FP32 in blocks of 4
 // (8-wave blocks: 16.1 against 14.6 ms of sweeps per step; 2-wave blocks: 14.5)
 template <typename R> constexpr int kFluxBlock = sizeof(R) == 4 ? 256 : 64;
-// occupancy targets of k_flux_hlld_fast (waves per SIMD), measured at 256^3 WENO5/HLLD:
+// occupancy targets of k_flux_fast (waves per SIMD), measured at 256^3 WENO5/HLLD:
 // FP64 at 3 (166 VGPRs, no scratch: 1.48-1.55 ms a sweep, against 1.92-2.23 at 4, which
 // spills), FP32 at 5 (92 VGPRs; at 4 waves 9 % slower)
 constexpr int kFastFluxWaves64 = 3;
+// FP64 HLL and HLLC at 4 (118 VGPRs)
+constexpr int kFastHllWaves64 = 4;
 constexpr int kFastFluxWaves32 = 5;
+template <typename R, int SOLVER> constexpr int fast_flux_waves()
+{
+  return sizeof(R) == 4 ? kFastFluxWaves32 : SOLVER == RIEMANN_HLLD ? kFastFluxWaves64 : kFastHllWaves64;
+}
 // grid of the redo kernels (a grid-stride loop over the queue): one block per CU, all that their
 // registers let be resident
 constexpr int kRedoBlocks = 256;
@@ -87,7 +94,7 @@ struct DevStats {
 
 /* Interfaces of the HLLD sweeps handed to the full FP64 solver (k_flux_redo) before the
  * update reads the fluxes: in the mixed form those whose FP32 HLLD solve failed, in the
- * plain form those outside the common path of the lean sweep (k_flux_hlld_fast). One list
+ * plain form those outside the common path of the lean sweep (k_flux_fast). One list
  * per axis. */
 struct RedoQueue {
   unsigned int *count;     // device counters, one per axis; cleared before the sweeps (clear_queue)
@@ -537,25 +544,26 @@ __device__ __forceinline__ int interface_flux(const double *__restrict__ P, long
   return err;
 }
 
-/* The common path of an HLLD interface, the flux written to its planes: reconstruction and
- * riemann_hlld_lean in FP64, riemann_hlld in FAST mode in FP32. Returns kHlldDefer where the
- * full solver is needed. */
-template <typename R>
+/* The common path of an interface, the flux written to its planes: reconstruction and the lean
+ * solvers in FP64, riemann_hlld in FAST mode in FP32. Returns kHlldDefer where the full solver
+ * is needed. */
+template <typename R, int SOLVER>
 __device__ __forceinline__ int interface_flux_fast(const double *__restrict__ P, R *__restrict__ Fout, long T, long S,
                                                    int axis, long z, int recon, const PhysParams &pp, R &lam,
                                                    FluxCounters &fc)
 {
   R ql[8], qr[8];
   reconstruct_states<R, sizeof(R) == 8>(P, T, S, axis, z, recon, pp, ql, qr);
-  if constexpr (sizeof(R) == 8)
-    return riemann_hlld_lean<1>(ql, qr, pp, lam, fc,
-                                [&](int q, double f) { Fout[axis_plane(q, axis) * T + z] = f; });
+  auto store = [&](int q, R f) { Fout[axis_plane(q, axis) * T + z] = f; };
+  if constexpr (sizeof(R) == 8 && SOLVER == RIEMANN_HLLD) return riemann_hlld_lean<1>(ql, qr, pp, lam, fc, store);
+  else if constexpr (sizeof(R) == 8) return riemann_hllx_lean<SOLVER>(ql, qr, pp, lam, store);
   else {
+    static_assert(SOLVER == RIEMANN_HLLD, "FP32: the HLLD sweep");
     R F[8];
     const int rc = riemann_hlld<R, 1, true>(ql, qr, F, (R)pp.gamma, pp.pfloor, lam, fc);
     if (rc == 0) {
 #pragma unroll
-      for (int q = 0; q < 8; ++q) Fout[axis_plane(q, axis) * T + z] = F[q];
+      for (int q = 0; q < 8; ++q) store(q, F[q]);
     }
     return rc;
   }
@@ -710,14 +718,14 @@ __device__ __forceinline__ bool update_zone_index(const GridDesc &g, long &t)
   return r < plane;
 }
 
-/* HLL and HLLC sweeps of a stage: one thread per interface, all three axes in one launch.
- * Occupancy targets (waves per SIMD): FP32 at 3, FP64 at 2 even where 256 registers spill
- * (the spill traffic costs less than the latency that a single wave cannot hide). */
-template <typename R, typename FT, int SOLVER>
-__global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 3 : 2) void k_flux(const double *__restrict__ P, FluxPlanes<FT> Fo,
-                                                                        GridDesc g, SweepGrid sg, int recon,
-                                                                        PhysParams pp, DevStats *st)
+/* The mixed form's HLL and HLLC sweeps of a stage: one thread per interface, all three axes in
+ * one launch, with the full FP32 solver and the retry (FP64 has k_flux_fast). */
+template <int SOLVER>
+__global__ __launch_bounds__(kBlock, 3) void k_flux32(const double *__restrict__ P, FluxPlanes<float> Fo, GridDesc g,
+                                                      SweepGrid sg, int recon, PhysParams pp, DevStats *st)
 {
+  using R = float;
+  using FT = float;
   const long T = g.T;
   int axis;
   long z = 0;
@@ -742,15 +750,15 @@ __global__ __launch_bounds__(kBlock, sizeof(R) == 4 ? 3 : 2) void k_flux(const d
   block_add<2>(cnt, dst);
 }
 
-/* HLLD sweeps of a stage, common path only (interface_flux_fast): interfaces that need
- * the c2p cascade, a later Newton attempt, the HLLC fallback or the retry are queued for
- * k_flux_redo, which computes them with the full FP64 solver. In the plain form that is the
+/* The sweeps of a stage, common path only (interface_flux_fast): interfaces that need the
+ * retry or, in HLLD, the c2p cascade, a later Newton attempt or the HLLC fallback, are queued
+ * for k_flux_redo, which computes them with the full FP64 solver. In the plain form that is the
  * result the full sweep gives; in the mixed form (R = float) the rare branches run in FP64
  * instead of FP32. Leaving them out of this kernel lowers its register peak. The queue holds
  * every interface of a sweep, so it cannot overflow. */
-template <typename R>
-__global__ __launch_bounds__(kFluxBlock<R>, sizeof(R) == 4 ? kFastFluxWaves32 : kFastFluxWaves64)
-void k_flux_hlld_fast(const double *__restrict__ P, FluxPlanes<R> Fo, GridDesc g, SweepGrid sg, int recon,
+template <typename R, int SOLVER>
+__global__ __launch_bounds__(kFluxBlock<R>, (fast_flux_waves<R, SOLVER>()))
+void k_flux_fast(const double *__restrict__ P, FluxPlanes<R> Fo, GridDesc g, SweepGrid sg, int recon,
                       PhysParams pp, RedoQueue rq)
 {
   int axis;
@@ -762,8 +770,8 @@ void k_flux_hlld_fast(const double *__restrict__ P, FluxPlanes<R> Fo, GridDesc g
   if (has) {
     R lam = R(0);
     FluxCounters fc = {0, 0, 0, 0};
-    defer = interface_flux_fast<R>(P, Fo.f[axis], g.T, axis_stride(g, axis), axis, z, recon, pp, lam, fc) != 0;
-    if (!defer) {
+    defer = interface_flux_fast<R, SOLVER>(P, Fo.f[axis], g.T, axis_stride(g, axis), axis, z, recon, pp, lam, fc) != 0;
+    if (!defer && SOLVER == RIEMANN_HLLD) {
       cnt[0] = 1;
       cnt[1] = (unsigned long long)fc.c2p_iters;
       cnt[2] = (unsigned long long)fc.newton_iters;
@@ -826,8 +834,8 @@ __global__ __launch_bounds__(kBlock) void k_flux_redo(const double *__restrict__
     cnt[5] += (unsigned long long)fc.newton_iters;
     cnt[6] += 1;
   };
-  if (n * 16 <= nthreads)
-    for (unsigned long k = tid >> 4; k < n; k += nthreads >> 4) redo(k, std::true_type());
+  if (SOLVER == RIEMANN_HLLD && n * 16 <= nthreads)
+    for (unsigned long k = tid >> 4; k < n; k += nthreads >> 4) redo(k, std::integral_constant<bool, SOLVER == RIEMANN_HLLD>());
   else
     for (unsigned long k = (tid & 63) * (nthreads >> 6) + (tid >> 6); k < n; k += nthreads) redo(k, std::false_type());
   block_max_lambda(lam_out, &st->lam_bits);
@@ -1026,47 +1034,12 @@ __device__ __forceinline__ void ctu_face_states(const double *__restrict__ P, co
 struct FaceStates { const double *p[3]; };
 
 /* Godunov fluxes of the half-slope states over the faces z | z+S, z in [begin, T - sx), of the
- * three axes in one launch, with the full solver (HLL, HLLC; HLLD through the redo). An
- * unphysical state counts a failure and leaves the flux unwritten. A solver error also leaves
- * it: then the flux is what the reference's array holds there, zero in step 2 (fresh arrays)
- * and the step-2 flux in step 4 (`keep`). */
+ * three axes in one launch, on the common path (riemann_hlld_lean, riemann_hllx_lean): a face
+ * that leaves it is queued for k_ctu_faces_redo. An unphysical state counts a failure and
+ * leaves the flux unwritten. The queue holds every face of an axis, so it cannot overflow.
+ * Blocks and occupancy as k_flux_fast. */
 template <int SOLVER>
-__global__ __launch_bounds__(kBlock, 2) void k_ctu_faces(const double *__restrict__ P, FaceStates Ps, FluxPlanes<double> Fo,
-                                                         GridDesc g, SweepGrid sg, PhysParams pp, int keep, DevStats *st,
-                                                         unsigned long long *fail)
-{
-  const long T = g.T;
-  int axis;
-  long z = 0;
-  const bool has = sweep_interface(g, sg, axis, z);
-  double lam_out = 0.0;
-  unsigned long long cnt[1] = {0};
-  if (has) {
-    double pl[8], pr[8];
-    ctu_face_states(P, Ps.p[axis], g, axis, z, pp.theta, pl, pr);
-    if (check_prim(pl) || check_prim(pr)) cnt[0] = 1;
-    else {
-      double *__restrict__ F = Fo.f[axis];
-      double f[8], lam = 0.0;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) f[q] = keep ? F[axis_plane(q, axis) * T + z] : 0.0;
-      FluxCounters fc = {0, 0, 0, 0};
-      riemann_dispatch<double, 1>(SOLVER, pl, pr, f, pp.gamma, pp.pfloor, lam, fc);
-#pragma unroll
-      for (int q = 0; q < 8; ++q) F[axis_plane(q, axis) * T + z] = f[q];
-      lam_out = lam;
-    }
-  }
-  block_max_lambda(lam_out, &st->lam_bits);
-  unsigned long long *const dst[1] = { fail };
-  block_add<1>(cnt, dst);
-}
-
-/* The HLLD faces on the common path (riemann_hlld_lean): a face that needs the c2p cascade, a
- * later Newton attempt or the HLLC fallback is queued for k_ctu_faces_redo. The queue holds
- * every face of an axis, so it cannot overflow. Grid, blocks and occupancy as
- * k_flux_hlld_fast<double>. */
-__global__ __launch_bounds__(kFluxBlock<double>, kFastFluxWaves64)
+__global__ __launch_bounds__(kFluxBlock<double>, (fast_flux_waves<double, SOLVER>()))
 void k_ctu_faces_fast(const double *__restrict__ P, FaceStates Ps, FluxPlanes<double> Fo, GridDesc g, SweepGrid sg,
                       PhysParams pp, RedoQueue rq)
 {
@@ -1085,9 +1058,10 @@ void k_ctu_faces_fast(const double *__restrict__ P, FaceStates Ps, FluxPlanes<do
       double *__restrict__ F = Fo.f[axis];
       double lam = 0.0;
       FluxCounters fc = {0, 0, 0, 0};
-      defer = riemann_hlld_lean<1>(pl, pr, pp, lam, fc,
-                                   [&](int q, double f) { F[axis_plane(q, axis) * T + z] = f; }) != 0;
-      if (!defer) {
+      auto store = [&](int q, double f) { F[axis_plane(q, axis) * T + z] = f; };
+      if constexpr (SOLVER == RIEMANN_HLLD) defer = riemann_hlld_lean<1>(pl, pr, pp, lam, fc, store) != 0;
+      else defer = riemann_hllx_lean<SOLVER>(pl, pr, pp, lam, store) != 0;
+      if (!defer && SOLVER == RIEMANN_HLLD) {
         cnt[1] = 1;
         cnt[2] = (unsigned long long)fc.c2p_iters;
         cnt[3] = (unsigned long long)fc.newton_iters;
@@ -1099,10 +1073,12 @@ void k_ctu_faces_fast(const double *__restrict__ P, FaceStates Ps, FluxPlanes<do
   sweep_counters_wave(lam_out, cnt[1] != 0, (unsigned)cnt[2], (unsigned)cnt[3], cnt[0] != 0, rq.part);
 }
 
-/* The queued faces of k_ctu_faces_fast by the full HLLD method (attempt ladder, HLLC
- * fallback), as k_flux_redo does it for the sweeps. Their states passed the physical check in
- * the fast pass. A face whose fast waves both lie on one side may hold that side's flux
- * already; the solver then never fails there, so `keep` finds the flux it needs. */
+/* The queued faces of k_ctu_faces_fast by the full solver, as k_flux_redo does it for the
+ * sweeps. Their states passed the physical check in the fast pass. A solver error leaves the
+ * flux: it is then what the reference's array holds there, zero in step 2 (fresh arrays) and
+ * the step-2 flux in step 4 (`keep`). A face whose fast waves both lie on one side may hold
+ * that side's flux already; the solver then never fails there. */
+template <int SOLVER>
 __global__ __launch_bounds__(kBlock) void k_ctu_faces_redo(const double *__restrict__ P, FaceStates Ps,
                                                            FluxPlanes<double> Fo, GridDesc g, PhysParams pp, int keep,
                                                            DevStats *st, unsigned long long *fail, RedoQueue rq,
@@ -1132,7 +1108,7 @@ __global__ __launch_bounds__(kBlock) void k_ctu_faces_redo(const double *__restr
 #pragma unroll
     for (int q = 0; q < 8; ++q) f[q] = keep ? F[axis_plane(q, axis) * T + z] : 0.0;
     FluxCounters fc = {0, 0, 0, 0};
-    riemann_hlld<double, 1>(pl, pr, f, pp.gamma, pp.pfloor, lam, fc);
+    riemann_dispatch<double, 1>(SOLVER, pl, pr, f, pp.gamma, pp.pfloor, lam, fc);
 #pragma unroll
     for (int q = 0; q < 8; ++q) F[axis_plane(q, axis) * T + z] = f[q];
     lam_out = fmax(lam_out, lam);
@@ -2180,7 +2156,7 @@ struct maragpu_ctx {
   float2 *start = nullptr;
   // the c2p passes' per-wave counters (one slot per wave of a pass)
   uint4 *c2p_part = nullptr;
-  // HLLD: the interfaces of the sweeps or face passes left to the full solver
+  // the interfaces of the sweeps or face passes left to the full solver
   RedoQueue redo = {};
   // weno-split: U with its ghost images, and the zone fluxes (8 planes) and speeds (1 plane)
   // of the current sweep in the flux precision
@@ -2239,29 +2215,50 @@ GridDesc make_grid(const maragpu_config &c)
   return g;
 }
 
-/* the three axis sweeps of a stage: HLLD on the common path and, for what it queued (in the
- * mixed form the FP32 HLLD failures, in the plain form whatever left the common path), the
- * full FP64 solver; HLL and HLLC by the full kernel */
+/* the three axis sweeps of a stage on the common path and, for what it queued (in the mixed
+ * form the FP32 HLLD failures, in the plain form whatever left the common path), the full
+ * FP64 solver; the mixed form's HLL and HLLC by the full FP32 kernel */
+template <typename R, int SOLVER>
+void launch_flux_fast(maragpu_ctx *c, const PhysParams &pp, const FluxPlanes<R> &F)
+{
+  const SweepGrid sg = sweep_grid(c->g, kFluxBlock<R>);
+  const unsigned nb = sg.first[3];
+  if (!nb) return;
+  k_flux_fast<R, SOLVER><<<nb, kFluxBlock<R>, 0, c->stream>>>(c->Pw, F, c->g, sg, c->cfg.recon, pp, c->redo);
+  k_flux_redo<R, SOLVER><<<kRedoBlocks, kBlock, 0, c->stream>>>(c->Pw, F, c->g, c->cfg.recon, pp, c->dstats, c->redo,
+                                                               nb * (kFluxBlock<R> / 64));
+}
+
 template <typename R>
 void launch_flux(maragpu_ctx *c, const PhysParams &pp)
 {
   FluxPlanes<R> F;
   for (int d = 0; d < 3; ++d) F.f[d] = static_cast<R *>(c->F[d]);
-  if (c->cfg.riemann == MARAGPU_HLLD) {
-    const SweepGrid sg = sweep_grid(c->g, kFluxBlock<R>);
-    const unsigned nb = sg.first[3];
-    if (!nb) return;
-    k_flux_hlld_fast<R><<<nb, kFluxBlock<R>, 0, c->stream>>>(c->Pw, F, c->g, sg, c->cfg.recon, pp, c->redo);
-    k_flux_redo<R, RIEMANN_HLLD><<<kRedoBlocks, kBlock, 0, c->stream>>>(c->Pw, F, c->g, c->cfg.recon, pp, c->dstats,
-                                                                       c->redo, nb * (kFluxBlock<R> / 64));
-    return;
+  if (c->cfg.riemann == MARAGPU_HLLD) return launch_flux_fast<R, RIEMANN_HLLD>(c, pp, F);
+  if constexpr (sizeof(R) == 8) {
+    if (c->cfg.riemann == MARAGPU_HLL) launch_flux_fast<R, RIEMANN_HLL>(c, pp, F);
+    else launch_flux_fast<R, RIEMANN_HLLC>(c, pp, F);
   }
-  const SweepGrid sg = sweep_grid(c->g, kBlock);
-  if (!sg.first[3]) return;
-  if (c->cfg.riemann == MARAGPU_HLL)
-    k_flux<R, R, RIEMANN_HLL><<<sg.first[3], kBlock, 0, c->stream>>>(c->Pw, F, c->g, sg, c->cfg.recon, pp, c->dstats);
-  else
-    k_flux<R, R, RIEMANN_HLLC><<<sg.first[3], kBlock, 0, c->stream>>>(c->Pw, F, c->g, sg, c->cfg.recon, pp, c->dstats);
+  else {
+    const SweepGrid sg = sweep_grid(c->g, kBlock);
+    if (!sg.first[3]) return;
+    if (c->cfg.riemann == MARAGPU_HLL)
+      k_flux32<RIEMANN_HLL><<<sg.first[3], kBlock, 0, c->stream>>>(c->Pw, F, c->g, sg, c->cfg.recon, pp, c->dstats);
+    else
+      k_flux32<RIEMANN_HLLC><<<sg.first[3], kBlock, 0, c->stream>>>(c->Pw, F, c->g, sg, c->cfg.recon, pp, c->dstats);
+  }
+}
+
+/* the faces of a plm-muscl pass, likewise */
+template <int SOLVER>
+void launch_faces(maragpu_ctx *c, const PhysParams &pp, const FaceStates &Ps, const FluxPlanes<double> &F, long begin,
+                  int keep, unsigned long long *fail)
+{
+  const SweepGrid sg = face_grid(c->g, begin, kFluxBlock<double>);
+  const unsigned nb = sg.first[3];
+  if (!nb) return;
+  k_ctu_faces_fast<SOLVER><<<nb, kFluxBlock<double>, 0, c->stream>>>(c->Pw, Ps, F, c->g, sg, pp, c->redo);
+  k_ctu_faces_redo<SOLVER><<<kRedoBlocks, kBlock, 0, c->stream>>>(c->Pw, Ps, F, c->g, pp, keep, c->dstats, fail, c->redo, nb);
 }
 
 /* weno-split sweep along DIM: zone fluxes and speeds, then the split interface fluxes */
@@ -2389,7 +2386,7 @@ int maragpu_create(const maragpu_config *cfg, maragpu_ctx **out)
         hipMalloc(&c->ctuP, 3 * nd * sizeof(double)) != hipSuccess)
       return fail_free(c);
   }
-  if (cfg->riemann == MARAGPU_HLLD && cfg->godunov != MARAGPU_WENO_SPLIT) {
+  if (cfg->godunov != MARAGPU_WENO_SPLIT && (cfg->riemann == MARAGPU_HLLD || cfg->precision == MARAGPU_FP64)) {
     // a slot for every interface of a sweep or face pass (4 bytes a slot: half a state plane
     // for an axis), and per-wave counters of the three sweeps
     RedoQueue &q = c->redo;
@@ -2567,24 +2564,10 @@ int maragpu_advance(maragpu_ctx *c, double dt, maragpu_stats *stats)
     double *Ux = c->ctuU, *Uy = c->ctuU + nd, *Uz = c->ctuU + 2 * nd;
     double *Px = c->ctuP, *Py = c->ctuP + nd, *Pz = c->ctuP + 2 * nd;
     unsigned long long *fl = c->dstats->ctu_failed[s];
-    // the faces of the three axes over [begin, T - sx): HLLD on the common path and its queue,
-    // HLL and HLLC by the full kernel
-    auto faces = [&](FaceStates Ps, long begin, int keep, unsigned long long *f) {
-      if (c->redo.z) {
-        const SweepGrid sg = face_grid(g, begin, kFluxBlock<double>);
-        const unsigned nb = sg.first[3];
-        if (!nb) return;
-        k_ctu_faces_fast<<<nb, kFluxBlock<double>, 0, c->stream>>>(c->Pw, Ps, F, g, sg, pp, c->redo);
-        k_ctu_faces_redo<<<kRedoBlocks, kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, pp, keep, c->dstats, f, c->redo, nb);
-        return;
-      }
-      const SweepGrid sg = face_grid(g, begin, kBlock);
-      const unsigned nb = sg.first[3];
-      if (!nb) return;
-      if (c->cfg.riemann == MARAGPU_HLL)
-        k_ctu_faces<RIEMANN_HLL><<<nb, kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, sg, pp, keep, c->dstats, f);
-      else
-        k_ctu_faces<RIEMANN_HLLC><<<nb, kBlock, 0, c->stream>>>(c->Pw, Ps, F, g, sg, pp, keep, c->dstats, f);
+    auto faces = [&](const FaceStates &Ps, long begin, int keep, unsigned long long *f) {
+      if (c->cfg.riemann == MARAGPU_HLLD) launch_faces<RIEMANN_HLLD>(c, pp, Ps, F, begin, keep, f);
+      else if (c->cfg.riemann == MARAGPU_HLL) launch_faces<RIEMANN_HLL>(c, pp, Ps, F, begin, keep, f);
+      else launch_faces<RIEMANN_HLLC>(c, pp, Ps, F, begin, keep, f);
     };
     faces(FaceStates{ { c->Pw, c->Pw, c->Pw } }, 0, 0, fl + 0);
     k_ctu_predict<<<nblocks(T - sxz), kBlock, 0, c->stream>>>(c->Pw, c->Uw, F.f[0], F.f[1], F.f[2], Ux, Uy, Uz, g, pp, dt,

@@ -1,4 +1,4 @@
-"""The FP64 HLLD sweep where its common path branches, against the oracle: both fast waves on
+"""The FP64 sweeps where their common path branches, against the oracle: both fast waves on
 one side of the interface (the flux of that side, in either direction), the reconstruction
 methods it dispatches on, and grids whose sweeps end inside a block.
 
@@ -16,14 +16,16 @@ from oracle.oracle import Setup, synchronize
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("extrap,IS,flow,N", [
-    ("weno5", "js96", (0.95, 0.0, 0.0), (13, 18, 11)),
-    ("weno5", "js96", (0.0, -0.9, 0.3), (9, 14, 22)),
-    ("weno5", "sz10", (0.2, 0.1, 0.93), (12, 10, 19)),
-    ("plm", "js96", (-0.93, 0.2, 0.0), (17, 8, 15)),
-    ("pcm", "js96", (0.0, 0.0, -0.95), (10, 11, 33)),
+@pytest.mark.parametrize("extrap,IS,flow,N,riemann", [
+    ("weno5", "js96", (0.95, 0.0, 0.0), (13, 18, 11), "hlld"),
+    ("weno5", "js96", (0.0, -0.9, 0.3), (9, 14, 22), "hlld"),
+    ("weno5", "sz10", (0.2, 0.1, 0.93), (12, 10, 19), "hlld"),
+    ("plm", "js96", (-0.93, 0.2, 0.0), (17, 8, 15), "hlld"),
+    ("pcm", "js96", (0.0, 0.0, -0.95), (10, 11, 33), "hlld"),
+    ("plm", "js96", (0.0, 0.93, 0.1), (11, 9, 13), "hll"),
+    ("weno5", "js96", (-0.9, 0.0, 0.3), (14, 9, 16), "hllc"),
 ])
-def test_supersonic_sweeps(gpu, oracle_lib, extrap, IS, flow, N):
+def test_supersonic_sweeps(gpu, oracle_lib, extrap, IS, flow, N, riemann):
     rng = np.random.default_rng(sum(N))
     x = [2 * np.pi * (np.arange(n) + 0.5) / n for n in N]
     X, Y, Z = np.meshgrid(*x, indexing="ij")
@@ -36,7 +38,8 @@ def test_supersonic_sweeps(gpu, oracle_lib, extrap, IS, flow, N):
         P[it + (2 + d,)] = flow[d] + 0.01 * wave[2 + d]
         P[it + (5 + d,)] = (0.2, 0.15, 0.25)[d] + 0.02 * wave[5 + d]
     P = synchronize(P, 3)
-    s = Setup(N=N, extrap=extrap, IS=IS, riemann="hlld", advance="rk2")
+    s = Setup(N=N, extrap=extrap, IS=IS, riemann=riemann, advance="rk2")
+
     def march(P0):
         so = oracle_lib.solver(s)
         Po, dt, out = P0.copy(), 0.0, []
@@ -56,7 +59,7 @@ def test_supersonic_sweeps(gpu, oracle_lib, extrap, IS, flow, N):
         lam_tol = np.maximum(lam_tol, [4 * abs(a[2] - b[2]) / b[2] for a, b in zip(noisy, ref)])
         L1_tol, max_tol = np.maximum(L1_tol, 4 * L1(Pn)), np.maximum(max_tol, 4 * worst(Pn))
 
-    ctx = gpu.Context(gpu.make_config(N=N, extrap=extrap, IS=IS, riemann="hlld", advance="rk2"))
+    ctx = gpu.Context(gpu.make_config(N=N, extrap=extrap, IS=IS, riemann=riemann, advance="rk2"))
     ctx.upload(P)
     for (eo, ok, lam, dt), tol in zip(ref, lam_tol):
         eg, stg = ctx.advance(dt)
@@ -152,3 +155,33 @@ def test_full_solver_queue(gpu, oracle_lib, n):
     assert st.hlld_success + st.hlld_failure == ok0 + fail0
     assert abs(st.hlld_success - ok0) <= ok_tol
     assert (L1(ctx.download()) <= tol).all()
+
+
+@pytest.mark.parametrize("riemann", ["hll", "hllc"])
+def test_retry_queue_hll(gpu, oracle_lib, riemann):
+    """A zone next to the light cone, whose neighbours' reconstructed states pass it: those
+    interfaces go to the full solver, which retries with the zone-centred states, in the HLL and
+    HLLC sweeps too. Counts as the oracle's, the state as in test_supersonic_sweeps (one small
+    step, so nothing has time to grow)."""
+    N = (9, 8, 12)
+    rng = np.random.default_rng(3)
+    P = np.empty(tuple(n + 6 for n in N) + (8,))
+    it = (slice(3, -3),) * 3
+    P[it] = [1.0, 1.0, 0.5, 0.1, 0.0, 0.2, 0.3, 0.1]
+    P[it + (slice(2, 5),)] += 0.3 * rng.uniform(-1, 1, N + (3,))
+    P[7, 6, 8, 2:5] = (0.99, 0.1, 0.05)
+    P[6, 6, 8, 2:5] = (0.8, 0.1, 0.05)
+    P[8, 6, 8, 2:5] = (0.9, 0.4, 0.05)
+    P = synchronize(P, 3)
+    kw = dict(N=N, extrap="weno5", riemann=riemann, advance="single")
+    so = oracle_lib.solver(Setup(**kw))
+    Po = P.copy()
+    eo, sto = so.advance(Po, 1e-4)
+    ctx = gpu.Context(gpu.make_config(**kw))
+    ctx.upload(P)
+    eg, stg = ctx.advance(1e-4)
+    assert eo == eg == 0 and sto.riemann_retries > 0
+    assert stg.riemann_retries == sto.riemann_retries == stg.fp64_redo
+    assert stg.riemann_failures == sto.riemann_failures
+    Pg = ctx.download()
+    assert (np.abs(Pg - Po).sum(axis=(0, 1, 2)) / np.abs(Po).sum(axis=(0, 1, 2))).max() < 1e-10
