@@ -1015,6 +1015,23 @@ __device__ __forceinline__ void weno5_js_pair(double vm2, double vm1, double v0,
   qr = side(Tc, tc + 2.0*gc, Td, gc + gd, Te, te - 2.0*gd, tc, td, te);
 }
 
+/* The finite-difference WENO5 flux reconstruction (WENO5_FD_C2R of weno.c:30-38, 97-154, with
+ * the Jiang-Shu weights) at the face between c and d from the values a..e upwind of it; the
+ * mirrored C2L form is the same function of the mirrored values. In differences as
+ * weno5_js_pair: (c + d)/2 plus multiples of the second differences. */
+__device__ __forceinline__ double weno5_js_fd(double a, double b, double c, double d, double e)
+{
+  const double gb = c - b, gc = d - c;
+  const double t2 = gb - (b - a), t1 = gc - gb, t0 = (e - d) - gc;
+  const double u2 = t2 + 2.0*gb, u1 = gb + gc, u0 = t0 - 2.0*gc;
+  const double k = 13./3., e4 = 4e-6;
+  const double B0 = u0*u0 + ((k*t0)*t0 + e4), B1 = u1*u1 + ((k*t1)*t1 + e4), B2 = u2*u2 + ((k*t2)*t2 + e4);
+  const double a0 = B0*B0, a1 = B1*B1, a2 = B2*B2;
+  const double w0 = 3.0*(a1*a2), w1 = 6.0*(a0*a2), w2 = a0*a1;
+  const double num = w0*t0 + w1*t1 + w2*(3.0*t1 - 2.0*t2);
+  return (c + 0.5*gc) - (1./6.)*(num*rcp_normal(w0 + w1 + w2));
+}
+
 /* The plane of field q of a state held in the frame whose first axis is `axis` (0, 1, 2):
  * (rho, p, v1, v2, v3, B1, B2, B3), or a conserved state or flux in that order. Uniform over
  * a launch's block, so it costs scalar instructions only, and one copy of the sweep's code
@@ -1847,6 +1864,41 @@ struct FastSide {
     return true;
   }
 };
+
+/* FluxAndEigenvalues of a zone, in the frame whose first axis is the normal, with the conserved
+ * state u given (weno-split's): the flux f and the fastest speed max(|a+|, |a-|) */
+__device__ __forceinline__ double zone_flux_lean(const double *u, const double *P, double *f, const PhysParams &pp)
+{
+  const double V2 = P[vx]*P[vx] + P[vy]*P[vy] + P[vz]*P[vz];
+  const double B2 = P[Bx]*P[Bx] + P[By]*P[By] + P[Bz]*P[Bz];
+  const double Bv = P[Bx]*P[vx] + P[By]*P[vy] + P[Bz]*P[vz];
+  const double om = 1.0 - V2;
+  const double W = rsqrt_normal(om), iW = om*W, W2 = W*W;
+  const double b0 = W*Bv;
+  const double b2 = (B2 + b0*b0)*om;
+  const double bx = P[Bx]*iW + b0*P[vx], by = P[By]*iW + b0*P[vy], bz = P[Bz]*iW + b0*P[vz];
+  const double rhoh = P[rho] + pp.g1*P[pre];
+  const double pt = P[pre] + 0.5*b2;
+  const double v = P[vx], BiW = P[Bx]*iW;
+  f[ddd] = u[ddd]*v;
+  f[tau] = u[tau]*v - b0*BiW + pt*v;
+  f[Sx] = u[Sx]*v - bx*BiW + pt;
+  f[Sy] = u[Sy]*v - by*BiW;
+  f[Sz] = u[Sz]*v - bz*BiW;
+  f[Bx] = 0.0;
+  f[By] = v*P[By] - P[vy]*P[Bx];
+  f[Bz] = v*P[Bz] - P[vz]*P[Bx];
+  const double ics2 = rhoh*pp.igamma*rcp_normal(P[pre]);
+  const double K = rhoh*(ics2 - 1.0)*(W2*W2);
+  const double L = -(rhoh + b2*ics2)*W2;
+  const double v2 = v*v, v3 = v*v2, v4 = v*v3;
+  double ep, em;
+  int nr;
+  quartic_extremes_lean(K - L - b0*b0, -4.0*K*v + L*v*2.0 + 2.0*b0*bx, 6.0*K*v2 + L*(1.0 - v2) + b0*b0 - bx*bx,
+                        -4.0*K*v3 - L*v*2.0 - 2.0*b0*bx, K*v4 + L*v2 + bx*bx, ep, em, nr);
+  const double a = dfabs(ep), b = dfabs(em);
+  return a > 1.0 || b > 1.0 ? 1.0 : (a > b ? a : b);
+}
 
 /* The flux of a lean solver, (D, E = tau + D, S, B) in the axis's frame, to `store` */
 template <int DIM, typename Store>

@@ -185,3 +185,32 @@ def test_retry_queue_hll(gpu, oracle_lib, riemann):
     assert stg.riemann_failures == sto.riemann_failures
     Pg = ctx.download()
     assert (np.abs(Pg - Po).sum(axis=(0, 1, 2)) / np.abs(Po).sum(axis=(0, 1, 2))).max() < 1e-10
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("N,Ng,IS", [((3, 5, 4), 3, "js96"), ((58, 4, 59), 3, "js96"), ((6, 60, 118), 4, "sz10"),
+                                     ((65, 7, 5), 3, "b08")])
+def test_weno_split_tiles(gpu, oracle_lib, N, Ng, IS, precision):
+    """The component-wise weno-split kernel at the edges of its tiles: one tile of interfaces
+    along an axis (up to 59), one more, two full ones, lines that fill no block, more ghost zones
+    than the stencil needs, the other smoothness indicators. Two steps against the oracle,
+    plain-form tolerances (mixed: L1 1e-6, its bound against FP64)."""
+    rng = np.random.default_rng(sum(N))
+    P = np.empty(tuple(n + 2 * Ng for n in N) + (8,))
+    it = (slice(Ng, -Ng),) * 3
+    P[it] = [1.0, 0.6, 0.1, -0.05, 0.08, 0.3, 0.2, 0.4]
+    P[it] *= 1.0 + 0.02 * rng.uniform(-1, 1, tuple(N) + (8,))
+    P = synchronize(P, Ng)
+    kw = dict(N=N, Ng=Ng, godunov="weno-split", extrap="weno5", IS=IS, advance="rk2")
+    so = oracle_lib.solver(Setup(**kw))
+    ctx = gpu.Context(gpu.make_config(precision=precision, **kw))
+    ctx.upload(P)
+    Po, dt = P.copy(), 0.1 / max(N)
+    for _ in range(2):
+        eo, sto = so.advance(Po, dt)
+        eg, stg = ctx.advance(dt)
+        assert eo == eg == 0
+        assert abs(stg.max_lambda - sto.max_lambda) <= (1e-12 if precision == "fp64" else 1e-5) * sto.max_lambda
+    Pg = ctx.download()
+    L1 = np.abs(Pg - Po).sum(axis=(0, 1, 2)) / np.abs(Po).sum(axis=(0, 1, 2))
+    assert L1.max() < (1e-10 if precision == "fp64" else 1e-6)
