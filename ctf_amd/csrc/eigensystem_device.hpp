@@ -1,6 +1,7 @@
 /* Characteristic eigensystem of the RMHD flux Jacobian, FP64, one state per group of 8 lanes.
  *
- * Used by the weno-split sweep to project the split fluxes into characteristic fields
+ * Used by the weno-split sweep (which has a shorter way for simple spectra, simple_projection
+ * below) to project the split fluxes into characteristic fields
  * (WenoSplit::intercell_flux_sweep, Mara/weno-split.cpp:163-207, which calls
  * FluidEquations::Eigensystem; the reference's RMHD fluid leaves that function empty,
  * Mara/hydro.hpp:146-147). The construction:
@@ -20,6 +21,7 @@
 #pragma once
 
 #include "rmhd_device.hpp"
+#include "mlp_device.hpp"     // wave_lds_sync
 
 namespace maragpu {
 namespace eig {
@@ -537,6 +539,331 @@ __device__ __forceinline__ int rmhd_eigensystem(const double *P, int lane, doubl
 #pragma unroll
   for (int k = 0; k < 8; ++k) lam[k] = ev[k];
   return 0;
+}
+
+/* --------------------------------------------------------------------------
+ * The projection of a state with a simple spectrum, for the sweep
+ *
+ * The same eigenvectors (up to sign) as rmhd_eigensystem forms, where all eigenvalues are at
+ * least 1e-7 apart: there each has one eigenvector, and the flux equations give most of it in
+ * closed form. In the frame whose first axis n is the normal, with x = (drho, dp, dv, dB) and
+ * (F' - lam U') x = 0, F' and U' the derivatives of flux and conserved state:
+ *   dv = (vn - lam) y and dBn = vn b with b = 1 for lam = 0 and b = 0 otherwise;
+ *   the rows of the tangential field:  dB_k = Bn y_k - B_k y_n + v_k b;
+ *   the row of D:                      drho = -rho (y_n + W^2 (vn - lam) v.y);
+ *   the rows of E = tau + D and S:     4 equations for (dp, y): the null vector for lam != 0,
+ *                                      an inhomogeneous system for lam = 0.
+ * No step divides by a gap of the spectrum, so nothing is lost as lam approaches vn. The
+ * entropy wave (lam = vn) is drho alone. A 4x4 elimination per lane replaces the 8x8 one, no
+ * M^-1 is formed, and matrices change hands through LDS instead of lane exchanges and selects:
+ *   lane k computes column k of U' and F' and, with eigenvalue k, eigenvector k;
+ *   R = U' x, transposed through LDS, is inverted by Gauss-Jordan elimination with lane = row:
+ *   partial pivoting picks a lane, so no row is moved, and the pivot row is broadcast.
+ * A quarter of the instructions of rmhd_eigensystem, and 98 VGPRs where it takes 235. What this
+ * cannot do (a cluster of eigenvalues, an elimination that breaks down, a projection that
+ * fails the acceptance bounds) is left to it.
+ * ------------------------------------------------------------------------ */
+constexpr int kGroupPad = 66;            // doubles of a group's 8x8 matrix in LDS (bank offset between groups)
+struct FastLds {
+  double a[8 * kGroupPad], r[8 * kGroupPad];   // one wave: 8 groups
+};
+
+__device__ __forceinline__ double quartic_newton_lean(double K, double L, double b0, double bi, double v, double x)
+{
+  for (int it = 0; it < 60; ++it) {
+    const double y = x - v, y2 = y*y, c = b0*x - bi, q1 = L*y2 + c*c, om = (1.0 - x)*(1.0 + x);
+    const double Q = K*y2*y2 + om*q1;
+    const double dQ = 4.0*K*y2*y - 2.0*x*q1 + om*(2.0*L*y + 2.0*b0*c);
+    const double step = Q*rcp(dQ);
+    const double xn = x - step;
+    if (!(fabs(xn) <= 1.0)) break;
+    x = xn;
+    if (!(fabs(step) > 1e-15)) break;
+  }
+  return x;
+}
+
+/* One step of the 4x4 complete-pivot elimination (rhs carried along; colp: nibble c is the
+ * unknown now in column c) */
+template <int K>
+__device__ __forceinline__ bool elim4_step(double (&a)[4][4], double (&rhs)[4], unsigned &colp)
+{
+  double best = -1.0;
+  int at = 5 * K;
+#pragma unroll
+  for (int r = K; r < 4; ++r)
+#pragma unroll
+    for (int c = K; c < 4; ++c) {
+      const double v = fabs(a[r][c]);
+      if (v > best) { best = v; at = 4 * r + c; }
+    }
+  const int pr = at >> 2, pc = at & 3;
+#pragma unroll
+  for (int c = K; c < 5; ++c) {                 // rows K <-> pr
+    const double ak = opaque(c < 4 ? a[K][c < 4 ? c : 3] : rhs[K]);
+    double ap = ak;
+#pragma unroll
+    for (int r = K + 1; r < 4; ++r) {
+      const double cur = opaque(c < 4 ? a[r][c < 4 ? c : 3] : rhs[r]);
+      ap = (pr == r) ? cur : ap;
+      const double now = (pr == r) ? ak : cur;
+      if (c < 4) a[r][c < 4 ? c : 3] = now;
+      else rhs[r] = now;
+    }
+    if (c < 4) a[K][c < 4 ? c : 3] = ap;
+    else rhs[K] = ap;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {                 // columns K <-> pc
+    const double ak = opaque(a[r][K]);
+    double ap = ak;
+#pragma unroll
+    for (int c = K + 1; c < 4; ++c) {
+      const double cur = opaque(a[r][c]);
+      ap = (pc == c) ? cur : ap;
+      a[r][c] = (pc == c) ? ak : cur;
+    }
+    a[r][K] = ap;
+  }
+  const unsigned nk = (colp >> (4 * K)) & 15u, np = (colp >> (4 * pc)) & 15u;
+  colp = (colp & ~((15u << (4 * K)) | (15u << (4 * pc)))) | (np << (4 * K)) | (nk << (4 * pc));
+  const double ip = rcp_normal(a[K][K]);
+#pragma unroll
+  for (int r = K + 1; r < 4; ++r) {
+    const double f = a[r][K] * ip;
+#pragma unroll
+    for (int c = K + 1; c < 4; ++c) a[r][c] -= f * a[K][c];
+    rhs[r] -= f * rhs[K];
+  }
+  return best > 0.0;
+}
+
+/* Lrow, Rrow (row `lane` of L and R) of the state P in the axis's frame, or false where
+ * rmhd_eigensystem has to be asked. All lanes of the wave call it together; `valid` = false
+ * for a group without an interface. */
+__device__ __forceinline__ bool simple_projection(FastLds &lds, const double *P, int lane, bool valid, double gamma,
+                                                  double (&Lrow)[8], double (&Rrow)[8])
+{
+  const double g1 = gamma * rcp(gamma - 1.0);
+  const double V2 = P[vx]*P[vx] + P[vy]*P[vy] + P[vz]*P[vz];
+  const double B2 = P[Bx]*P[Bx] + P[By]*P[By] + P[Bz]*P[Bz];
+  const double Bv = P[Bx]*P[vx] + P[By]*P[vy] + P[Bz]*P[vz];
+  const double om = 1.0 - V2;
+  const double W = rsqrt_normal(om), iW = om*W, W2 = W*W;
+  const double b0 = W*Bv, bb = B2 + b0*b0, b2 = bb*om;
+  const double rhoh = P[rho] + g1*P[pre];
+  const double vn = P[vx], Bn = P[Bx];
+  double lam;                                   // eigenvalue number `lane`
+  {
+    const double bi = Bn*iW + b0*vn;
+    const double irh = rcp(rhoh), ics2 = rhoh*rcp(gamma*P[pre]), cs2 = gamma*P[pre]*irh;
+    const double K = rhoh*(ics2 - 1.0)*(W2*W2), L = -(rhoh + b2*ics2)*W2;
+    const double e = sqrt_lean(rhoh + b2);
+    const double s = (lane & 1) ? -e : e;
+    const double alfven = (bi + s*W*vn)*rcp(b0 + s*W);
+    const double ca2 = b2*rcp(rhoh + b2);
+    const double w2 = cs2 + ca2 - cs2*ca2;
+    const double den = rcp(1.0 - V2*w2);
+    const double rt = sqrt_lean(w2*om*(1.0 - V2*w2 - vn*vn*(1.0 - w2)));
+    // even lanes take the roots from above, odd lanes from below
+    const double start = (lane & 1) ? fmax((vn*(1.0 - w2) - rt)*den - 1e-12, -1.0)
+                                    : fmin((vn*(1.0 - w2) + rt)*den + 1e-12, 1.0);
+    const double fast = quartic_newton_lean(K, L, b0, bi, vn, start);
+    const double other = xchg<kDppXor1>(fast);
+    const double A4 = K - L - b0*b0;
+    const double A3 = -4.0*K*vn + L*vn*2.0 + 2.0*b0*bi;
+    const double A2 = 6.0*K*vn*vn + L*(1.0 - vn*vn) + b0*b0 - bi*bi;
+    const double c1 = A3 + A4*(fast + other);
+    const double c0 = A2 + c1*(fast + other) - A4*(fast*other);
+    const double sq = sqrt_lean(fmax(c1*c1 - 4.0*A4*c0, 0.0));
+    const double slow = quartic_newton_lean(K, L, b0, bi, vn, ((lane & 1) ? -c1 - sq : sq - c1)*rcp(2.0*A4));
+    lam = lane < 2 ? (lane == 0 ? 0.0 : vn) : lane < 4 ? alfven : lane < 6 ? fast : slow;
+    // a simple spectrum: the smallest distance between two eigenvalues, each lane against the
+    // other seven
+    double gap = 1.0;
+#pragma unroll
+    for (int d = 1; d < 8; ++d) gap = fmin(gap, fabs(lam - bc(lam, (lane + d) & 7)));
+    // NaN anywhere leaves some difference NaN: !(>=) would miss it through fmin, so test lam
+    const int bad = !(gap >= 1e-7) || !(fabs(lam) <= 1.0) || !valid ? 1 : 0;
+    if (imax(bad)) return false;
+  }
+  const int base = (int)((threadIdx.x & 63) >> 3) * kGroupPad;
+  double *A = lds.a + base, *Rm = lds.r + base;
+  {
+    // column `lane` of U' (rows E, S) and F' (rows S; that of E is U' of S_n), explicitly
+    // differentiated along P[lane]
+    const double wt = rhoh + b2, wW2 = wt*W2;
+    double dv[3], dB[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      dv[k] = lane == 2 + k ? 1.0 : 0.0;
+      dB[k] = lane == 5 + k ? 1.0 : 0.0;
+    }
+    const double dp = lane == 1 ? 1.0 : 0.0;
+    const double vdv = P[vx]*dv[0] + P[vy]*dv[1] + P[vz]*dv[2];
+    const double dW = W*W2*vdv;
+    const double db0 = dW*Bv + W*(P[Bx]*dv[0] + P[By]*dv[1] + P[Bz]*dv[2] + P[vx]*dB[0] + P[vy]*dB[1] + P[vz]*dB[2]);
+    const double db2 = 2.0*((P[Bx]*dB[0] + P[By]*dB[1] + P[Bz]*dB[2] + b0*db0)*om - bb*vdv);
+    const double dw = (lane == 0 ? 1.0 : 0.0) + g1*dp + db2;
+    const double dpt = dp + 0.5*db2;
+    const double dwW2 = dw*W2 + 2.0*wt*W*dW;
+    const double diW = -W*vdv;
+    const double BniW = Bn*iW, dBniW = dB[0]*iW + Bn*diW;
+    double *col = A + 8 * lane;
+    col[0] = dwW2 - dpt - 2.0*b0*db0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const double b = P[Bx + k]*iW + b0*P[vx + k];
+      const double db = dB[k]*iW + P[Bx + k]*diW + db0*P[vx + k] + b0*dv[k];
+      const double S = wW2*P[vx + k] - b0*b;
+      const double dS = dwW2*P[vx + k] + wW2*dv[k] - db0*b - b0*db;
+      col[1 + k] = dS;
+      col[4 + k] = dS*vn + S*dv[0] - db*BniW - b*dBniW + (k == 0 ? dpt : 0.0);
+    }
+  }
+  wave_lds_sync();
+  const double c = vn - lam, beta = lane == 0 ? 1.0 : 0.0;
+  double Rc[8];
+  {
+    double a[4][4], rhs[4];
+    // G = F' - lam U', rows E, S: column k of it from lane k's entries
+    auto G = [&](int k, double (&g)[4]) {
+      const double *q = A + 8 * k;
+      g[0] = q[1] - lam*q[0];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) g[1 + i] = q[4 + i] - lam*q[1 + i];
+    };
+    double g[4], gr[4];
+    G(rho, gr);
+    G(pre, g);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) a[r][0] = g[r];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      G(vx + k, g);
+      const double dr = -P[rho]*(W2*c*P[vx + k] + (k == 0 ? 1.0 : 0.0));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) a[r][1 + k] = c*g[r] + dr*gr[r];
+    }
+    G(Bx, g);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) rhs[r] = vn*g[r];
+#pragma unroll
+    for (int k = 1; k < 3; ++k) {
+      G(Bx + k, g);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        a[r][1] -= P[Bx + k]*g[r];
+        a[r][1 + k] += Bn*g[r];
+        rhs[r] += P[vx + k]*g[r];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) rhs[r] *= beta;
+    unsigned colp = 0x3210u;
+    bool ok = elim4_step<0>(a, rhs, colp);
+    ok = elim4_step<1>(a, rhs, colp) && ok;
+    ok = elim4_step<2>(a, rhs, colp) && ok;
+    double t[4];
+    t[3] = lane == 0 ? -rhs[3]*rcp(a[3][3]) : 1.0;
+    t[2] = -(rhs[2] + a[2][3]*t[3])*rcp(a[2][2]);
+    t[1] = -(rhs[1] + a[1][2]*t[2] + a[1][3]*t[3])*rcp(a[1][1]);
+    t[0] = -(rhs[0] + a[0][1]*t[1] + a[0][2]*t[2] + a[0][3]*t[3])*rcp(a[0][0]);
+    double y[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      y[u] = t[0];
+#pragma unroll
+      for (int q = 1; q < 4; ++q) y[u] = ((colp >> (4 * q)) & 15u) == (unsigned)u ? t[q] : y[u];
+    }
+    double x[8];
+    const double vy_ = P[vx]*y[1] + P[vy]*y[2] + P[vz]*y[3];
+    x[rho] = -P[rho]*(y[1] + W2*c*vy_);
+    x[pre] = y[0];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) x[vx + k] = c*y[1 + k];
+    x[Bx] = vn*beta;
+    x[By] = Bn*y[2] - P[By]*y[1] + P[vy]*beta;
+    x[Bz] = Bn*y[3] - P[Bz]*y[1] + P[vz]*beta;
+    if (lane == 1) {                            // the entropy wave
+      ok = true;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) x[k] = k == rho ? 1.0 : 0.0;
+    }
+    const double D = W*x[rho] + P[rho]*W*W2*(P[vx]*x[vx] + P[vy]*x[vy] + P[vz]*x[vz]);
+    double E = 0.0, S0 = 0.0, S1 = 0.0, S2 = 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const double *q = A + 8 * k;
+      E += q[0]*x[k];
+      S0 += q[1]*x[k];
+      S1 += q[2]*x[k];
+      S2 += q[3]*x[k];
+    }
+    Rc[ddd] = D;
+    Rc[tau] = E - D;
+    Rc[Sx] = S0; Rc[Sy] = S1; Rc[Sz] = S2;
+    Rc[Bx] = x[Bx]; Rc[By] = x[By]; Rc[Bz] = x[Bz];
+    double m = 0.0;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) m = fmax(m, fabs(Rc[r]));
+    const double im = rcp(m);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) Rm[8 * r + lane] = Rc[r]*im;
+    if (imax(!ok || !(m > 0.0) || !(im > 0.0) ? 1 : 0)) return false;
+  }
+  wave_lds_sync();
+  // R^-1: this lane has row `lane`; step k eliminates column k with the unused row of largest
+  // |a[k]|, in place (column k then holds the inverse's). perm: 3 bits per step, the row taken.
+  double a[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) a[j] = Rm[8 * lane + j];
+  unsigned perm = 0u;
+  int mine = -1;
+  bool fine = true;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const double mag = mine < 0 ? fabs(a[k]) : -1.0;
+    const double best = vmax(mag);
+    const unsigned long long eq = __ballot(mag == best);
+    const int p = __ffs((int)((unsigned)(eq >> (threadIdx.x & 56)) & 0xffu)) - 1;
+    fine = fine && best > 0.0;
+    perm |= (unsigned)(p & 7) << (3 * k);
+    const bool me = p == lane;
+    if (me) mine = k;
+    double row[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) row[j] = bc(a[j], p);
+    const double ip = rcp(row[k]);
+    const double f = me ? -ip : a[k]*ip;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j == k) continue;
+      const double cur = me ? 0.0 : a[j];
+      a[j] = cur - f*row[j];
+    }
+    a[k] = -f;
+  }
+  if (imax(!fine || mine < 0 ? 1 : 0)) return false;
+  // row `mine` of the inverse, its columns in the order of the rows taken
+#pragma unroll
+  for (int j = 0; j < 8; ++j) A[8 * mine + ((perm >> (3 * j)) & 7u)] = a[j];
+  wave_lds_sync();
+  double lmax = 0.0, err = 0.0, LR[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    Lrow[j] = A[8 * lane + j];
+    Rrow[j] = Rm[8 * lane + j];
+    lmax = fmax(lmax, fabs(Lrow[j]));
+    LR[j] = lane == j ? -1.0 : 0.0;
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) LR[j] += Lrow[k]*Rm[8 * k + j];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) err = fmax(err, fabs(LR[j]));
+  return !imax(!(lmax < 1e8) || !(err < 1e-8) ? 1 : 0);
 }
 
 /* rows of the identity projection */

@@ -848,28 +848,39 @@ __global__ __launch_bounds__(kBlock) void k_flux_redo(const double *__restrict__
 /* --------------------------------------------------------------------------
  * weno-split (WenoSplit, Mara/weno-split.cpp) with local Lax-Friedrichs flux splitting.
  * ------------------------------------------------------------------------ */
-/* Per zone, for the sweep along DIM: the physical flux F and the fastest speed
- * A = max(|a+|, |a-|) (drive_single_sweep, Mara/weno-split.cpp:224-236), over every zone;
+/* Per zone, for the characteristic sweep along `axis`: the physical flux F and the fastest
+ * speed A = max(|a+|, |a-|) (drive_single_sweep, Mara/weno-split.cpp:224-236), over every zone;
  * MaxLambda is their maximum. Uw holds U with its ghost images (as Uglb after ConsToPrim). */
-template <typename R, int DIM>
+template <typename R>
+__device__ __forceinline__ R zone_flux(const R *u, const R *p, R *f, const PhysParams &pp)
+{
+  if constexpr (sizeof(R) == 8) return zone_flux_lean(u, p, f, pp);
+  else {
+    R ap, am;
+    flux_and_eigenvalues<R, 1>(u, p, f, ap, am, (R)pp.gamma);
+    return (dfabs(ap) > dfabs(am)) ? dfabs(ap) : dfabs(am);
+  }
+}
+
+template <typename R>
 __global__ __launch_bounds__(kBlock) void k_zone_flux(const double *__restrict__ Uw, const double *__restrict__ P,
-                                                      R *__restrict__ FZ, R *__restrict__ AZ, GridDesc g,
+                                                      R *__restrict__ FZ, R *__restrict__ AZ, GridDesc g, int axis,
                                                       PhysParams pp, DevStats *st)
 {
   const long z = (long)blockIdx.x * blockDim.x + threadIdx.x;
   const long T = g.T;
   double lam_out = 0.0;
   if (z < T) {
-    R u[8], p[8], f[8], ap, am;
+    R u[8], p[8], f[8];
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      u[q] = (R)Uw[q * T + z];
-      p[q] = (R)P[q * T + z];
+      const long o = axis_plane(q, axis) * T + z;
+      u[q] = (R)Uw[o];
+      p[q] = (R)P[o];
     }
-    flux_and_eigenvalues<R, DIM>(u, p, f, ap, am, (R)pp.gamma);
-    const R a = (dfabs(ap) > dfabs(am)) ? dfabs(ap) : dfabs(am);
+    const R a = zone_flux<R>(u, p, f, pp);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) FZ[q * T + z] = f[q];
+    for (int q = 0; q < 8; ++q) FZ[axis_plane(q, axis) * T + z] = f[q];
     AZ[z] = a;
     lam_out = (double)a;
   }
@@ -947,12 +958,7 @@ __global__ __launch_bounds__(kWsLines * kWsRows) void k_weno_split(const double 
       u[q] = (R)Uw[o];
       p[q] = (R)P[o];
     }
-    if constexpr (sizeof(R) == 8) A = zone_flux_lean(u, p, f, pp);
-    else {
-      R ap, am;
-      flux_and_eigenvalues<R, 1>(u, p, f, ap, am, (R)pp.gamma);
-      A = (dfabs(ap) > dfabs(am)) ? dfabs(ap) : dfabs(am);
-    }
+    A = zone_flux<R>(u, p, f, pp);
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
       u[q] *= R(0.5);
@@ -1009,54 +1015,26 @@ __global__ __launch_bounds__(kWsLines * kWsRows) void k_weno_split(const double 
   }
 }
 
-/* The same sweep with the RMHD characteristic projection (eigen = RMHD): the eigensystem
- * of the averaged primitive state 0.5 (P_z + P_z+S) in FP64 (L and R; the identity where
- * it is rejected), the 6-zone split fluxes projected with L, the finite-difference WENO5
- * of every characteristic field, and the projection of their sum back with R
- * (Mara/weno-split.cpp:176-203, the eigensystem call at :181). In the mixed form (R =
- * float) only the zone fluxes and speeds are FP32.
- * Eight lanes share one interface (eig::g8): lane q holds row q of L and R, projects and
- * reconstructs characteristic field q, and writes flux component q. */
-template <typename R, int DIM>
-__global__ __launch_bounds__(kBlock) void k_flux_weno_split_char(const double *__restrict__ Uw,
-                                                                 const double *__restrict__ P,
-                                                                 const R *__restrict__ FZ, const R *__restrict__ AZ,
-                                                                 R *__restrict__ Fout, GridDesc g, PhysParams pp,
-                                                                 DevStats *st)
+/* The characteristic flux of interface z | z+S by the group of 8 lanes that holds L and R:
+ * lane q projects and reconstructs characteristic field q and writes flux component q (in the
+ * axis's frame). With ml the largest A over the 6-zone stencil, the split fluxes are projected
+ * with L, every characteristic field reconstructed by the finite-difference WENO5, and the sum
+ * projected back with R (Mara/weno-split.cpp:176-203). The projections and reconstructions
+ * stay in FP64 also in the mixed form (R = float has FP32 zone fluxes and speeds only): the
+ * characteristic fields carry large parts that cancel on the way back through R, so their
+ * rounding is multiplied by the condition number of R. */
+template <typename R>
+__device__ __forceinline__ void char_flux(const double *__restrict__ Uw, const R *__restrict__ FZ,
+                                          const R *__restrict__ AZ, R *__restrict__ Fout, long T, long S, int axis,
+                                          long z, int lane, const double (&Lrow)[8], const double (&Rrow)[8],
+                                          const PhysParams &pp)
 {
-#pragma clang fp contract(off)
-  const long c0 = DIM == 1 ? g.N[0] + 1 : g.n[0];
-  const long c1 = DIM == 2 ? g.N[1] + 1 : g.n[1];
-  const long c2 = DIM == 3 ? g.N[2] + 1 : g.n[2];
-  const long t = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 3;     // alike in the 8 lanes
-  const int lane = (int)(threadIdx.x & 7);
-  if (t >= c0 * c1 * c2) return;
-  const long k = t % c2 + (DIM == 3 ? g.Ng - 1 : 0);
-  const long j = (t / c2) % c1 + (DIM == 2 ? g.Ng - 1 : 0);
-  const long i = t / (c2 * c1) + (DIM == 1 ? g.Ng - 1 : 0);
-  const long T = g.T;
-  const long S = DIM == 1 ? g.sx : DIM == 2 ? g.sy : g.sz;
-  const long z = (i * g.n[1] + j) * g.n[2] + k;
-
-  double Lrow[8], Rrow[8], lam[8];
-  {
-    double Ph[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) Ph[q] = 0.5 * (P[q * T + z] + P[q * T + z + S]);
-    if (eig::g8::rmhd_eigensystem<DIM>(Ph, lane, Lrow, Rrow, lam, pp.gamma) != 0) {
-      eig::g8::identity_rows(lane, Lrow, Rrow, lam);
-      if (lane == 0) atomicAdd(&st->eig_identity, 1ull);
-    }
-  }
   R mlr = AZ[z - 2 * S];
 #pragma unroll
   for (int m = -1; m <= 3; ++m) {
     const R a = AZ[z + m * S];
     mlr = a > mlr ? a : mlr;
   }
-  // the projections and the reconstructions stay in FP64 also in the mixed form: the
-  // characteristic fields carry large parts that cancel on the way back through R, so
-  // their rounding is multiplied by the condition number of R
   const double ml = (double)mlr;
   double fp[6], fm[6];
 #pragma unroll
@@ -1065,19 +1043,96 @@ __global__ __launch_bounds__(kBlock) void k_flux_weno_split_char(const double *_
     double a = 0.0, b = 0.0;
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      const double F = (double)FZ[c * T + zm], U = Uw[c * T + zm];
-      a += Lrow[c] * (0.5 * (F + ml * U));
-      b += Lrow[c] * (0.5 * (F - ml * U));
+      const long o = axis_plane(c, axis) * T + zm;
+      const double F = 0.5 * (double)FZ[o], U = 0.5 * ml * Uw[o];
+      a += Lrow[c] * (F + U);
+      b += Lrow[c] * (F - U);
     }
     fp[m] = a;
     fm[m] = b;
   }
-  const double f = weno5<double, true, true>(fp[0], fp[1], fp[2], fp[3], fp[4], pp.IS, pp.sz10A) +
-                   weno5<double, false, true>(fm[1], fm[2], fm[3], fm[4], fm[5], pp.IS, pp.sz10A);
+  double f;
+  if (pp.IS == IS_JS96) f = weno5_js_fd(fp[0], fp[1], fp[2], fp[3], fp[4]) + weno5_js_fd(fm[5], fm[4], fm[3], fm[2], fm[1]);
+  else
+    f = weno5<double, true, true>(fp[0], fp[1], fp[2], fp[3], fp[4], pp.IS, pp.sz10A) +
+        weno5<double, false, true>(fm[1], fm[2], fm[3], fm[4], fm[5], pp.IS, pp.sz10A);
   double a = 0.0;
 #pragma unroll
   for (int c = 0; c < 8; ++c) a += Rrow[c] * eig::g8::bc(f, c);
-  Fout[lane * T + z] = (R)a;
+  Fout[axis_plane(lane, axis) * T + z] = (R)a;
+}
+
+/* The sweep along `axis` with the RMHD characteristic projection (eigen = RMHD), over the
+ * interfaces whose index along the axis lies in [Ng-1, N+Ng-1], on every transverse line: the
+ * eigensystem of the averaged primitive state 0.5 (P_z + P_z+S) in FP64 (the eigensystem call at
+ * Mara/weno-split.cpp:181), eight lanes to an interface. States with a simple spectrum are done
+ * here (eig::g8::simple_projection); the others are queued for k_flux_weno_split_char_redo.
+ * At 48x56x44, FP64: 146 us a sweep (2 500 VALU instructions per wave of 8 interfaces, half of
+ * the time their issue and the rest the latency of LDS and loads at 98 VGPRs and 34 KB of LDS a
+ * block, 4 waves per SIMD), and 4-60 us for the queue; 512 us with the general eigensystem for
+ * every interface (10 100 instructions, 235 VGPRs, 2 waves). */
+template <typename R>
+__global__ __launch_bounds__(kBlock, 3) void k_flux_weno_split_char(const double *__restrict__ Uw,
+                                                                    const double *__restrict__ P,
+                                                                    const R *__restrict__ FZ, const R *__restrict__ AZ,
+                                                                    R *__restrict__ Fout, GridDesc g, int axis,
+                                                                    PhysParams pp, RedoQueue rq)
+{
+  __shared__ __align__(16) eig::g8::FastLds lds[kBlock / 64];
+  const long c0 = axis == 0 ? g.N[0] + 1 : g.n[0];
+  const long c1 = axis == 1 ? g.N[1] + 1 : g.n[1];
+  const long c2 = axis == 2 ? g.N[2] + 1 : g.n[2];
+  long t = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 3;           // alike in the 8 lanes
+  const int lane = (int)(threadIdx.x & 7);
+  const bool valid = t < c0 * c1 * c2;
+  if (!valid) t = 0;
+  const long k = t % c2 + (axis == 2 ? g.Ng - 1 : 0);
+  const long j = (t / c2) % c1 + (axis == 1 ? g.Ng - 1 : 0);
+  const long i = t / (c2 * c1) + (axis == 0 ? g.Ng - 1 : 0);
+  const long T = g.T, S = axis_stride(g, axis);
+  const long z = (i * g.n[1] + j) * g.n[2] + k;
+  double Lrow[8], Rrow[8];
+  bool done;
+  {
+    double Ph[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const double *v = P + axis_plane(q, axis) * T + z;
+      Ph[q] = 0.5 * (v[0] + v[S]);
+    }
+    done = eig::g8::simple_projection(lds[threadIdx.x >> 6], Ph, lane, valid, pp.gamma, Lrow, Rrow);
+  }
+  if (done && valid) char_flux<R>(Uw, FZ, AZ, Fout, T, S, axis, z, lane, Lrow, Rrow, pp);
+  queue_push(rq, axis, valid && !done && lane == 0, z);
+}
+
+/* The queued interfaces, with the general eigensystem (eig::g8::rmhd_eigensystem; the identity
+ * where it is rejected); a loop over the queue's count, eight lanes to an interface. */
+template <typename R>
+__global__ __launch_bounds__(kBlock) void k_flux_weno_split_char_redo(const double *__restrict__ Uw,
+                                                                      const double *__restrict__ P,
+                                                                      const R *__restrict__ FZ,
+                                                                      const R *__restrict__ AZ, R *__restrict__ Fout,
+                                                                      GridDesc g, int axis, PhysParams pp, DevStats *st,
+                                                                      RedoQueue rq)
+{
+  const long T = g.T, S = axis_stride(g, axis);
+  const int lane = (int)(threadIdx.x & 7);
+  const unsigned n = min(rq.count[axis], rq.cap);
+  for (unsigned e = (blockIdx.x * blockDim.x + threadIdx.x) >> 3; e < n; e += (gridDim.x * blockDim.x) >> 3) {
+    const long z = (long)rq.z[(size_t)axis * rq.cap + e];
+    double Lrow[8], Rrow[8], lam[8], Ph[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const double *v = P + axis_plane(q, axis) * T + z;
+      Ph[q] = 0.5 * (v[0] + v[S]);
+    }
+    if (eig::g8::rmhd_eigensystem<1>(Ph, lane, Lrow, Rrow, lam, pp.gamma) != 0) {
+      eig::g8::identity_rows(lane, Lrow, Rrow, lam);
+      if (lane == 0) atomicAdd(&st->eig_identity, 1ull);
+    }
+    char_flux<R>(Uw, FZ, AZ, Fout, T, S, axis, z, lane, Lrow, Rrow, pp);
+  }
 }
 
 /* --------------------------------------------------------------------------
@@ -2243,7 +2298,8 @@ struct maragpu_ctx {
   float2 *start = nullptr;
   // the c2p passes' per-wave counters (one slot per wave of a pass)
   uint4 *c2p_part = nullptr;
-  // the interfaces of the sweeps or face passes left to the full solver
+  // the interfaces of the sweeps or face passes left to the full solver (weno-split, eigen =
+  // RMHD: to the general eigensystem)
   RedoQueue redo = {};
   // weno-split: U with its ghost images, and with the characteristic projection the zone fluxes
   // (8 planes) and speeds (1 plane) of the current sweep in the flux precision
@@ -2366,10 +2422,12 @@ void launch_weno_split(maragpu_ctx *c, const PhysParams &pp)
   }
   R *FZ = static_cast<R *>(c->FZ);
   R *AZ = FZ + 8 * g.T;
-  k_zone_flux<R, DIM><<<nblocks(g.T), kBlock, 0, c->stream>>>(c->Uw, c->Pw, FZ, AZ, g, pp, c->dstats);
+  k_zone_flux<R><<<nblocks(g.T), kBlock, 0, c->stream>>>(c->Uw, c->Pw, FZ, AZ, g, DIM - 1, pp, c->dstats);
   const long cnt = (long)(DIM == 1 ? g.N[0] + 1 : g.n[0]) * (DIM == 2 ? g.N[1] + 1 : g.n[1]) *
                    (DIM == 3 ? g.N[2] + 1 : g.n[2]);
-  k_flux_weno_split_char<R, DIM><<<nblocks(8 * cnt), kBlock, 0, c->stream>>>(c->Uw, c->Pw, FZ, AZ, F, g, pp, c->dstats);
+  k_flux_weno_split_char<R><<<nblocks(8 * cnt), kBlock, 0, c->stream>>>(c->Uw, c->Pw, FZ, AZ, F, g, DIM - 1, pp, c->redo);
+  k_flux_weno_split_char_redo<R><<<std::min(nblocks(8 * cnt), 2048u), kBlock, 0, c->stream>>>(
+      c->Uw, c->Pw, FZ, AZ, F, g, DIM - 1, pp, c->dstats, c->redo);
 }
 
 /* Per-block partials of the measure table for maragpu_measure_noalloc, in a file-scope
@@ -2479,13 +2537,15 @@ int maragpu_create(const maragpu_config *cfg, maragpu_ctx **out)
         hipMalloc(&c->ctuP, 3 * nd * sizeof(double)) != hipSuccess)
       return fail_free(c);
   }
-  if (cfg->godunov != MARAGPU_WENO_SPLIT && (cfg->riemann == MARAGPU_HLLD || cfg->precision == MARAGPU_FP64)) {
+  if (cfg->godunov == MARAGPU_WENO_SPLIT ? cfg->eigen == MARAGPU_EIG_RMHD
+                                         : cfg->riemann == MARAGPU_HLLD || cfg->precision == MARAGPU_FP64) {
     // a slot for every interface of a sweep or face pass (4 bytes a slot: half a state plane
     // for an axis), and per-wave counters of the three sweeps
     RedoQueue &q = c->redo;
     q.cap = (unsigned int)c->g.T;
     unsigned waves;
-    if (cfg->godunov == MARAGPU_PLM_MUSCL) waves = face_grid(c->g, 0, kFluxBlock<double>).first[3];
+    if (cfg->godunov == MARAGPU_WENO_SPLIT) waves = 0;       // its queue has no counters
+    else if (cfg->godunov == MARAGPU_PLM_MUSCL) waves = face_grid(c->g, 0, kFluxBlock<double>).first[3];
     else if (cfg->precision == MARAGPU_MIXED) waves = sweep_grid(c->g, kFluxBlock<float>).first[3] * (kFluxBlock<float> / 64);
     else waves = sweep_grid(c->g, kFluxBlock<double>).first[3];
     static_assert(kFluxBlock<double> == 64, "one wave per FP64 block");
