@@ -115,6 +115,7 @@ struct GridDesc {
   long T;                  // zones including ghosts
   long sx, sy, sz;         // zone strides
   double dx, dy, dz, min_dx;
+  double rdx, rdy, rdz;    // 1/dx, 1/dy, 1/dz, rounded (div_by)
 };
 
 #define HIP_CHECK(expr)                                                            \
@@ -280,13 +281,23 @@ __global__ void k_soa_to_aos(const double *__restrict__ soa, double *__restrict_
   for (int q = 0; q < 8; ++q) aos[8 * z + q] = soa[q * T + z];
 }
 
+/* The indices, in the grid with ghosts, of interior zone t (flat (i, j, k) order). 32-bit
+ * divisions: a zone takes over 300 bytes of device memory, so their number stays below 2^31,
+ * and the 64-bit ones cost over a hundred instructions each. */
+__device__ __forceinline__ void interior_zone(const GridDesc &g, long t, int &i, int &j, int &k)
+{
+  const unsigned u = (unsigned)t, n1 = (unsigned)g.N[1], n2 = (unsigned)g.N[2];
+  const unsigned ij = u / n2, a = ij / n1;
+  k = (int)(u - ij * n2) + g.Ng;
+  j = (int)(ij - a * n1) + g.Ng;
+  i = (int)a + g.Ng;
+}
+
 __device__ __forceinline__ long interior_zone(const GridDesc &g, long t)
 {
-  const long nzk = g.N[2], nyk = g.N[1];
-  const long k = t % nzk;
-  const long j = (t / nzk) % nyk;
-  const long i = t / (nzk * nyk);
-  return ((i + g.Ng) * g.n[1] + (j + g.Ng)) * g.n[2] + (k + g.Ng);
+  int i, j, k;
+  interior_zone(g, t, i, j, k);
+  return ((long)i * g.n[1] + j) * g.n[2] + k;
 }
 
 /* one field's interior, (i, j, k) order with k fastest, out of / into its SoA plane: the
@@ -303,9 +314,8 @@ __global__ void k_field_in(const double *__restrict__ in, double *__restrict__ p
 {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long)g.N[0] * g.N[1] * g.N[2]) return;
-  const int k = (int)(t % g.N[2]) + g.Ng;
-  const int j = (int)((t / g.N[2]) % g.N[1]) + g.Ng;
-  const int i = (int)(t / ((long)g.N[2] * g.N[1])) + g.Ng;
+  int i, j, k;
+  interior_zone(g, t, i, j, k);
   const double v = in[t];
   int li[3], lj[3], lk[3];
   int ni = 0, nj = 0, nk = 0;
@@ -690,9 +700,9 @@ inline unsigned update_blocks(const int *N)
   return (unsigned)(N[0] * ((plane + kBlock - 1) / kBlock));
 }
 
-/* The calling thread's interior zone t (flat (i, j, k) order, 0 <= t < N0 N1 N2); false
- * where it has none (the last tile of a plane). */
-__device__ __forceinline__ bool update_zone_index(const GridDesc &g, long &t)
+/* The calling thread's interior zone t (flat (i, j, k) order, 0 <= t < N0 N1 N2) and its
+ * indices in the grid with ghosts; false where it has none (the last tile of a plane). */
+__device__ __forceinline__ bool update_zone_index(const GridDesc &g, long &t, int &i, int &j, int &k)
 {
   const unsigned nb = gridDim.x, b = blockIdx.x;
   const unsigned q = nb >> 3;
@@ -714,6 +724,10 @@ __device__ __forceinline__ bool update_zone_index(const GridDesc &g, long &t)
     tile = full * C + rem % width;
   }
   const unsigned r = tile * kBlock + threadIdx.x;
+  const unsigned jr = r / (unsigned)g.N[2];
+  i = (int)a + g.Ng;
+  j = (int)jr + g.Ng;
+  k = (int)(r - jr * (unsigned)g.N[2]) + g.Ng;
   t = (long)a * plane + r;
   return r < plane;
 }
@@ -1392,6 +1406,18 @@ constexpr bool stage_reads_u(int kind)
   return kind == ST_RK2_FINAL || kind == ST_RK3_2 || kind == ST_RK3_3;
 }
 
+/* a/d as the division rounds it, from r = 1/d rounded: the first correction brings the
+ * quotient within one unit in the last place, and from there a correction with the exact
+ * residual and a correctly rounded reciprocal gives the rounded quotient (Markstein 1990;
+ * quotients above the subnormal range). 5 operations where the compiler's division, which
+ * has its own reciprocal and scaling, takes 11. */
+__device__ __forceinline__ double div_by(double a, double d, double r)
+{
+  double q = a*r;
+  q = __builtin_fma(__builtin_fma(-q, d, a), r, q);
+  return __builtin_fma(__builtin_fma(-q, d, a), r, q);
+}
+
 template <typename FT>
 __device__ __forceinline__ double ld(const FT *__restrict__ a, long i) { return (double)a[i]; }
 
@@ -1449,7 +1475,8 @@ __device__ __forceinline__ void update_zone(const FT *__restrict__ Fx, const FT 
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
     // Mara/plm-split.cpp:117-119
-    const double L = -(F0[q]-F1[q])/g.dx - (G0[q]-G1[q])/g.dy - (H0[q]-H1[q])/g.dz;
+    const double L = -div_by(F0[q]-F1[q], g.dx, g.rdx) - div_by(G0[q]-G1[q], g.dy, g.rdy) -
+                     div_by(H0[q]-H1[q], g.dz, g.rdz);
     const long m = q * T + z;
     const double u0 = U0[m];
     double un;
@@ -1569,7 +1596,11 @@ enum { C2P_CASCADE = 0, C2P_NET = 1, C2P_STORED = 2 };
  * (not the first pass): CT, the flux divergence and the RK combination, then the new U
  * from registers into the inversion (the plain cascade, or from the zone's stored start
  * with the cascade as fallback). With Uw (weno-split, plm-muscl) U's ghost images are
- * written too. */
+ * written too.
+ * Bound by HBM: 6.75 GB at 256^3 in FP64 (the fluxes once, U0, U and P), 1.72 ms, 80 % of a
+ * copy's rate. With the compiler's divisions by dx, dy, dz and 64-bit index divisions the
+ * arithmetic reached into that time: 1.83 ms. 3 waves per SIMD: with 4 the zone's loads no
+ * longer fit in registers (2.73 ms); 2 gain 2 % here and lose what small grids overlap. */
 template <typename FT, int MODE>
 __global__ __launch_bounds__(kBlock, 3) void k_update_c2p(
     const FT *__restrict__ Fx, const FT *__restrict__ Fy, const FT *__restrict__ Fz,
@@ -1585,14 +1616,11 @@ __global__ __launch_bounds__(kBlock, 3) void k_update_c2p(
   unsigned long long cnt[NC] = {};
   {
     long t = 0;
-    const bool valid = update_zone_index(g, t);
     int i = 0, j = 0, k = 0;
+    const bool valid = update_zone_index(g, t, i, j, k);
     long z = 0;
     double u[8], p[8];
     if (valid) {
-      k = (int)(t % g.N[2]) + g.Ng;
-      j = (int)((t / g.N[2]) % g.N[1]) + g.Ng;
-      i = (int)(t / ((long)g.N[2] * g.N[1])) + g.Ng;
       z = ((long)i * g.n[1] + j) * g.n[2] + k;
       update_zone<FT>(Fx, Fy, Fz, U0, U, A, g, z, dt, kind, write_u != 0, u);
     }
@@ -1659,9 +1687,7 @@ __global__ __launch_bounds__(kBlock, MODE == C2P_NET ? 3 : 4) void k_p2c_c2p(con
     int i = 0, j = 0, k = 0;
     double u[8], p[8];
     if (valid) {
-      k = (int)(t % g.N[2]) + g.Ng;
-      j = (int)((t / g.N[2]) % g.N[1]) + g.Ng;
-      i = (int)(t / ((long)g.N[2] * g.N[1])) + g.Ng;
+      interior_zone(g, t, i, j, k);
       const long z = ((long)i * g.n[1] + j) * g.n[2] + k;
 #pragma unroll
       for (int q = 0; q < 8; ++q) p[q] = Pc[q * T + z];
@@ -2355,6 +2381,9 @@ GridDesc make_grid(const maragpu_config &c)
   g.dy = (lx1[1] - lx0[1]) / (g.n[1] - 2 * c.Ng);
   g.dz = (lx1[2] - lx0[2]) / (g.n[2] - 2 * c.Ng);
   g.min_dx = min_dx;
+  g.rdx = 1.0 / g.dx;
+  g.rdy = 1.0 / g.dy;
+  g.rdz = 1.0 / g.dz;
   return g;
 }
 
