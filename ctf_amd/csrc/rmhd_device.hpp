@@ -44,11 +44,14 @@ template <> struct Tol<double> {
   // common path (riemann_hlld_lean): Newton steps of the p* solve (the reference's); the last
   // one, from a residual within newton_ftol, reuses the derivative of the one before where
   // it moves p by at most reuse_step, relatively; step tolerance and cap of the nested c2p,
-  // whose result only starts the p* solve
+  // whose result only starts the p* solve. Where the Alfven speeds differ by less than
+  // weak_delK (a weak normal field) the solve ends early, below small_delK, or wanders: its
+  // result depends on the path, and the full solver takes the reference's path.
   static constexpr int newton_fast_max_it = 15;
   static constexpr double reuse_step = 1e-11;
   static constexpr double nested_step = 1e-6;
   static constexpr int nested_max_it = 16;
+  static constexpr double weak_delK = 1e-6;
   static constexpr double fd_dp = 1e-8;          // HlldEquation48::Jacobian, :313
   static constexpr bool fd_relative = false;
   static constexpr bool fd_one_sided = false;    // the reference's centred difference
@@ -2215,7 +2218,8 @@ __device__ __forceinline__ int riemann_hlld_lean(const double *pl, const double 
       if (mode == RESIDUAL) {
         const double ay = dfabs(y);
         const double dx = Gd*y;
-        if (have && ay <= T::newton_ftol && ay <= 0.05*dfabs(y0) && dfabs(dx) <= T::reuse_step*dfabs(p)) {
+        if (have && it < T::newton_fast_max_it && ay <= T::newton_ftol && ay <= 0.05*dfabs(y0) &&
+            dfabs(dx) <= T::reuse_step*dfabs(p)) {
           p -= dx;
           pe = p;
           mode = SOLUTION;
@@ -2244,6 +2248,7 @@ __device__ __forceinline__ int riemann_hlld_lean(const double *pl, const double 
     }
     cnt.newton_iters += it;
     p = pe;
+    if (!small_bn && dfabs(delK) < T::weak_delK) return kHlldDefer;
   }
 
   // ReconstructSolution, :417-538, for s = 0
