@@ -1597,12 +1597,13 @@ enum { C2P_CASCADE = 0, C2P_NET = 1, C2P_STORED = 2 };
  * from registers into the inversion (the plain cascade, or from the zone's stored start
  * with the cascade as fallback). With Uw (weno-split, plm-muscl) U's ghost images are
  * written too.
- * Bound by HBM: 6.75 GB at 256^3 in FP64 (the fluxes once, U0, U and P), 1.72 ms, 80 % of a
+ * Bound by HBM: 6.75 GB at 256^3 in FP64 (the fluxes once, U0, U and P), 1.68 ms, 82 % of a
  * copy's rate. With the compiler's divisions by dx, dy, dz and 64-bit index divisions the
- * arithmetic reached into that time: 1.83 ms. 3 waves per SIMD: with 4 the zone's loads no
- * longer fit in registers (2.73 ms); 2 gain 2 % here and lose what small grids overlap. */
+ * arithmetic reached into that time: 1.83 ms. Waves per SIMD in FP64: 2 (1.68 ms; 126.5 us
+ * at 96^3) rather than 3 (1.72 ms; 128 us), where 12 B per lane go to scratch; with 4 the
+ * zone's loads no longer fit in registers (2.73 ms). */
 template <typename FT, int MODE>
-__global__ __launch_bounds__(kBlock, 3) void k_update_c2p(
+__global__ __launch_bounds__(kBlock, (sizeof(FT) == 8 ? 2 : 3)) void k_update_c2p(
     const FT *__restrict__ Fx, const FT *__restrict__ Fy, const FT *__restrict__ Fz,
     const double *__restrict__ U0, double *__restrict__ U, double *__restrict__ A, double *__restrict__ P,
     GridDesc g, double dt, int kind, int write_u, double gamma, double pfloor, int ereset, double preset,
