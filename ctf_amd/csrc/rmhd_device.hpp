@@ -1868,6 +1868,32 @@ struct FastSide {
   }
 };
 
+/* The flux of a physical state (v < 1), in the frame whose first axis is the normal, as in
+ * FastSide; the energy's without the rest mass, its terms as the reference sums them */
+__device__ __forceinline__ void side_flux_lean(const double *P, double g1, double *F)
+{
+  const double V2 = P[vx]*P[vx] + P[vy]*P[vy] + P[vz]*P[vz];
+  const double B2 = P[Bx]*P[Bx] + P[By]*P[By] + P[Bz]*P[Bz];
+  const double Bv = P[Bx]*P[vx] + P[By]*P[vy] + P[Bz]*P[vz];
+  const double om = 1.0 - V2;
+  const double W = rsqrt_normal(om), iW = om*W, W2 = W*W;
+  const double b0 = W*Bv;
+  const double b2 = (B2 + b0*b0)*om;
+  const double bx = P[Bx]*iW + b0*P[vx], by = P[By]*iW + b0*P[vy], bz = P[Bz]*iW + b0*P[vz];
+  const double wW2 = (P[rho] + g1*P[pre] + b2)*W2;
+  const double pt = P[pre] + 0.5*b2;
+  const double D = P[rho]*W;
+  const double v = P[vx], BiW = P[Bx]*iW;
+  F[ddd] = D*v;
+  F[tau] = (wW2 - pt - b0*b0 - D)*v - b0*BiW + pt*v;
+  F[Sx] = (wW2*P[vx] - b0*bx)*v - bx*BiW + pt;
+  F[Sy] = (wW2*P[vy] - b0*by)*v - by*BiW;
+  F[Sz] = (wW2*P[vz] - b0*bz)*v - bz*BiW;
+  F[Bx] = 0.0;
+  F[By] = v*P[By] - P[vy]*P[Bx];
+  F[Bz] = v*P[Bz] - P[vz]*P[Bx];
+}
+
 /* FluxAndEigenvalues of a zone, in the frame whose first axis is the normal, with the conserved
  * state u given (weno-split's): the flux f and the fastest speed max(|a+|, |a-|) */
 __device__ __forceinline__ double zone_flux_lean(const double *u, const double *P, double *f, const PhysParams &pp)
