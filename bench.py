@@ -69,14 +69,15 @@ def sweep_flops(w, fc=None):
     return (nif[0] * fpi["x"] + nif[1] * fpi["y"] + nif[2] * fpi["z"]) / 3.0
 
 
-def sweep_hw_ops(w):
-    """Hardware FP32 operations of one FP32 sweep launch (mean over the axes): the count per
-    interface measured at 256^3 times the interfaces of the sweep; None without the file."""
+def sweep_hw_ops(w, fp32):
+    """Hardware FP32 (mixed form) or FP64 operations of one axis's sweep (mean over the axes):
+    the count per interface measured at 256^3 times the interfaces; None without the file, and
+    in FP64 for another flow than c2's (the number of Newton steps depends on it)."""
     path = os.path.join(ROOT, "profiles", "sweep_ops_c2_256.json")
-    if not os.path.exists(path):
+    if not os.path.exists(path) or not (fp32 or w.name == "c2"):
         return None
     with open(path) as f:
-        per = json.load(f)["fp32_ops_per_interface"]
+        per = json.load(f)["fp32_ops_per_interface" if fp32 else "fp64_ops_per_interface"]
     return per * sum(interfaces_per_sweep(w)) / 3.0
 
 
@@ -118,23 +119,23 @@ def form_roofline(w, r, form):
     f_sweep = sweep_flops(w, fc)
     t_sweep = r["flux_ms_per_launch"] * 1e-3
     peak = FP32_PEAK_TFLOPS if fp32 else FP64_PEAK_TFLOPS
-    # The FP64 sweep is priced by the oracle's count along its path. The FP32 sweep accepts
-    # the HLLD start without a Newton step at most interfaces, so that count would credit it
-    # with work it skips: it is priced by the hardware FP32 operations it issues per
-    # interface (rocprofv3 SQ counters at 256^3, profiles/sweep_ops_c2_256.json).
-    hw = sweep_hw_ops(w) if fp32 else None
+    # The sweeps leave out operations of the reference's order whose result is already known
+    # (and the FP32 one most Newton steps), so the oracle's count would credit them with work
+    # they skip: they are priced by the hardware operations they issue per interface
+    # (rocprofv3 SQ counters at 256^3, profiles/sweep_ops_c2_256.json).
+    hw = sweep_hw_ops(w, fp32)
     f_priced = hw if hw is not None else f_sweep
     ach = f_priced / t_sweep / 1e12
-    sweep = {"kernel": f"k_flux_hlld_fast<{'float' if fp32 else 'double'}> + k_flux_redo (one axis sweep)",
+    sweep = {"kernel": f"k_flux_fast<{'float' if fp32 else 'double'}> + k_flux_redo (a third of the launch: one axis)",
              "bound": "valu", "achieved": ach, "peak": peak, "unit": "TFLOP/s", "frac": ach / peak,
              "flops_per_launch": f_priced, "avg_launch_ms": r["flux_ms_per_launch"],
-             "flops_source": ("hardware FP32 operations per interface (FMA = 2) x interfaces, "
+             "flops_source": (f"hardware FP{32 if fp32 else 64} operations per interface (FMA = 2) x interfaces, "
                               "profiles/sweep_ops_c2_256.json" if hw is not None else
                               "oracle count along the device's path (tests/golden/flops_*.json device_path)"),
              "bytes_per_launch": nif * (64 + (32 if fp32 else 64)),
              "hbm_GBs": nif * (64 + (32 if fp32 else 64)) / t_sweep / 1e9}
+    sweep["oracle_flops_per_launch"] = f_sweep
     if fp32:
-        sweep["oracle_flops_per_launch"] = f_sweep
         sweep["peak_without_packed_fp32"] = FP32_UNPACKED_TFLOPS
         sweep["frac_without_packed_fp32"] = ach / FP32_UNPACKED_TFLOPS
     chained = form != "plain"
@@ -547,15 +548,19 @@ def main():
     forms_out, plain = forms_record(w, forms, args.steps, args.warmup, acc_steps, args.model)
 
     fc = flop_counts(w)
-    flops_per_launch = sweep_flops(w, fc)
+    hw = sweep_hw_ops(w, False)
+    flops_per_launch = hw if hw is not None else sweep_flops(w, fc)
     avg_flux_s = plain["flux_ms_per_launch"] * 1e-3
     achieved = flops_per_launch / avg_flux_s / 1e12
     roofline = {"bound": "valu", "achieved": achieved, "peak": FP64_PEAK_TFLOPS,
                 "unit": "TFLOP/s", "frac": achieved / FP64_PEAK_TFLOPS,
-                "kernel": "k_flux_hlld_fast<double> + k_flux_redo (one axis sweep, WENO5/HLLD)",
+                "kernel": "k_flux_fast<double> + k_flux_redo (a third of the launch: one axis, WENO5/HLLD)",
                 "flops_per_launch": flops_per_launch,
-                "flops_source": "oracle count along the device's path (nested c2p from the average state), "
-                                "tests/golden/flops_%s.json" % w.name,
+                "flops_source": ("hardware FP64 operations per interface (FMA = 2) x interfaces, "
+                                 "profiles/sweep_ops_c2_256.json" if hw is not None else
+                                 "oracle count along the device's path (nested c2p from the average state), "
+                                 "tests/golden/flops_%s.json" % w.name),
+                "oracle_flops_per_launch": sweep_flops(w, fc),
                 "avg_launch_ms": plain["flux_ms_per_launch"],
                 "traffic": None}
     tr = traffic_record(w)

@@ -2009,7 +2009,7 @@ __global__ __launch_bounds__(kBlock) void k_ou_sum_x(const double2 *__restrict__
 }
 
 /* The field at n arbitrary points (xyz, 3 per point): the per-axis factors are formed per
- * point (nk <= 13 per axis), then summed as in k_ou_sample */
+ * point (nk <= 13 per axis), then summed as the sampling does */
 __global__ __launch_bounds__(kBlock) void kb_ou_sample(long n, const double *__restrict__ xyz,
                                                        const double2 *__restrict__ amp, int k1, double *__restrict__ F)
 {
