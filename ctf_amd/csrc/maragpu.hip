@@ -1033,7 +1033,10 @@ __global__ __launch_bounds__(kWsLines * kWsRows) void k_weno_split(const double 
  * lane q projects and reconstructs characteristic field q and writes flux component q (in the
  * axis's frame). With ml the largest A over the 6-zone stencil, the split fluxes are projected
  * with L, every characteristic field reconstructed by the finite-difference WENO5, and the sum
- * projected back with R (Mara/weno-split.cpp:176-203). The projections and reconstructions
+ * projected back with R (Mara/weno-split.cpp:176-203). Lane c loads and splits component c of the
+ * six zones and the lanes exchange them through LDS (Fp, Fm: the group's 48 values each): with
+ * every lane loading every component the sweep took 146 us at 48x56x44 in FP64 and 16.5 ms at
+ * 256^3, with the exchange 103 us and 10.7 ms. The projections and reconstructions
  * stay in FP64 also in the mixed form (R = float has FP32 zone fluxes and speeds only): the
  * characteristic fields carry large parts that cancel on the way back through R, so their
  * rounding is multiplied by the condition number of R. */
@@ -1041,7 +1044,7 @@ template <typename R>
 __device__ __forceinline__ void char_flux(const double *__restrict__ Uw, const R *__restrict__ FZ,
                                           const R *__restrict__ AZ, R *__restrict__ Fout, long T, long S, int axis,
                                           long z, int lane, const double (&Lrow)[8], const double (&Rrow)[8],
-                                          const PhysParams &pp)
+                                          double *Fp, double *Fm, const PhysParams &pp)
 {
   R mlr = AZ[z - 2 * S];
 #pragma unroll
@@ -1050,17 +1053,23 @@ __device__ __forceinline__ void char_flux(const double *__restrict__ Uw, const R
     mlr = a > mlr ? a : mlr;
   }
   const double ml = (double)mlr;
+  wave_lds_sync();                 // the group is done with what was there
+  const long o = axis_plane(lane, axis) * T + z;
+#pragma unroll
+  for (int m = 0; m < 6; ++m) {
+    const double F = 0.5 * (double)FZ[o + (m - 2) * S], U = 0.5 * ml * Uw[o + (m - 2) * S];
+    Fp[8 * m + lane] = F + U;
+    Fm[8 * m + lane] = F - U;
+  }
+  wave_lds_sync();
   double fp[6], fm[6];
 #pragma unroll
   for (int m = 0; m < 6; ++m) {
-    const long zm = z + (m - 2) * S;
     double a = 0.0, b = 0.0;
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      const long o = axis_plane(c, axis) * T + zm;
-      const double F = 0.5 * (double)FZ[o], U = 0.5 * ml * Uw[o];
-      a += Lrow[c] * (F + U);
-      b += Lrow[c] * (F - U);
+      a += Lrow[c] * Fp[8 * m + c];
+      b += Lrow[c] * Fm[8 * m + c];
     }
     fp[m] = a;
     fm[m] = b;
@@ -1081,10 +1090,10 @@ __device__ __forceinline__ void char_flux(const double *__restrict__ Uw, const R
  * eigensystem of the averaged primitive state 0.5 (P_z + P_z+S) in FP64 (the eigensystem call at
  * Mara/weno-split.cpp:181), eight lanes to an interface. States with a simple spectrum are done
  * here (eig::g8::simple_projection); the others are queued for k_flux_weno_split_char_redo.
- * At 48x56x44, FP64: 146 us a sweep (2 500 VALU instructions per wave of 8 interfaces, half of
- * the time their issue and the rest the latency of LDS and loads at 98 VGPRs and 34 KB of LDS a
- * block, 4 waves per SIMD), and 4-60 us for the queue; 512 us with the general eigensystem for
- * every interface (10 100 instructions, 235 VGPRs, 2 waves). */
+ * At 48x56x44, FP64: 103 us a sweep (2 280 VALU instructions per wave of 8 interfaces, 76 % of the
+ * time their issue at 256^3, 34 KB of LDS a block, 4 waves per SIMD), and 4-60 us for the queue;
+ * 512 us with the general eigensystem for every interface (10 100 instructions, 235 VGPRs, 2
+ * waves). */
 template <typename R>
 __global__ __launch_bounds__(kBlock, 3) void k_flux_weno_split_char(const double *__restrict__ Uw,
                                                                     const double *__restrict__ P,
@@ -1096,13 +1105,14 @@ __global__ __launch_bounds__(kBlock, 3) void k_flux_weno_split_char(const double
   const long c0 = axis == 0 ? g.N[0] + 1 : g.n[0];
   const long c1 = axis == 1 ? g.N[1] + 1 : g.n[1];
   const long c2 = axis == 2 ? g.N[2] + 1 : g.n[2];
-  long t = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 3;           // alike in the 8 lanes
+  const long t = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 3;     // alike in the 8 lanes
   const int lane = (int)(threadIdx.x & 7);
   const bool valid = t < c0 * c1 * c2;
-  if (!valid) t = 0;
-  const long k = t % c2 + (axis == 2 ? g.Ng - 1 : 0);
-  const long j = (t / c2) % c1 + (axis == 1 ? g.Ng - 1 : 0);
-  const long i = t / (c2 * c1) + (axis == 0 ? g.Ng - 1 : 0);
+  const unsigned u = valid ? (unsigned)t : 0u, n1 = (unsigned)c1, n2 = (unsigned)c2;   // 32-bit: interior_zone
+  const unsigned ij = u / n2, a = ij / n1;
+  const long k = (long)(u - ij * n2) + (axis == 2 ? g.Ng - 1 : 0);
+  const long j = (long)(ij - a * n1) + (axis == 1 ? g.Ng - 1 : 0);
+  const long i = (long)a + (axis == 0 ? g.Ng - 1 : 0);
   const long T = g.T, S = axis_stride(g, axis);
   const long z = (i * g.n[1] + j) * g.n[2] + k;
   double Lrow[8], Rrow[8];
@@ -1116,7 +1126,11 @@ __global__ __launch_bounds__(kBlock, 3) void k_flux_weno_split_char(const double
     }
     done = eig::g8::simple_projection(lds[threadIdx.x >> 6], Ph, lane, valid, pp.gamma, Lrow, Rrow);
   }
-  if (done && valid) char_flux<R>(Uw, FZ, AZ, Fout, T, S, axis, z, lane, Lrow, Rrow, pp);
+  if (done && valid) {
+    const int base = (int)((threadIdx.x & 63) >> 3) * eig::g8::kGroupPad;
+    char_flux<R>(Uw, FZ, AZ, Fout, T, S, axis, z, lane, Lrow, Rrow, lds[threadIdx.x >> 6].a + base,
+                 lds[threadIdx.x >> 6].r + base, pp);
+  }
   queue_push(rq, axis, valid && !done && lane == 0, z);
 }
 
@@ -1130,8 +1144,10 @@ __global__ __launch_bounds__(kBlock) void k_flux_weno_split_char_redo(const doub
                                                                       GridDesc g, int axis, PhysParams pp, DevStats *st,
                                                                       RedoQueue rq)
 {
+  __shared__ __align__(16) double split[kBlock / 8][2 * 48 + 4];     // the pad staggers the groups' banks
   const long T = g.T, S = axis_stride(g, axis);
   const int lane = (int)(threadIdx.x & 7);
+  double *const Fp = split[threadIdx.x >> 3];
   const unsigned n = min(rq.count[axis], rq.cap);
   for (unsigned e = (blockIdx.x * blockDim.x + threadIdx.x) >> 3; e < n; e += (gridDim.x * blockDim.x) >> 3) {
     const long z = (long)rq.z[(size_t)axis * rq.cap + e];
@@ -1145,7 +1161,7 @@ __global__ __launch_bounds__(kBlock) void k_flux_weno_split_char_redo(const doub
       eig::g8::identity_rows(lane, Lrow, Rrow, lam);
       if (lane == 0) atomicAdd(&st->eig_identity, 1ull);
     }
-    char_flux<R>(Uw, FZ, AZ, Fout, T, S, axis, z, lane, Lrow, Rrow, pp);
+    char_flux<R>(Uw, FZ, AZ, Fout, T, S, axis, z, lane, Lrow, Rrow, Fp, Fp + 48, pp);
   }
 }
 
