@@ -2135,7 +2135,8 @@ __device__ __forceinline__ int riemann_hlld_lean(const double *pl, const double 
     L.set(sl, am);
     Rt.set(sr, ap);
     // both fast waves on one side: the flux is that side's own, stored now so that its state
-    // need not be kept (the solve below still decides whether HLLD is counted a success)
+    // need not be kept (the solve below still decides whether HLLD is counted a success, and,
+    // with both on the left, whether an inner wave lies on the right all the same)
     supersonic = 0.0 <= am || !(0.0 <= ap);
     if (supersonic) {
       const bool l = 0.0 <= am;
@@ -2307,9 +2308,10 @@ __device__ __forceinline__ int riemann_hlld_lean(const double *pl, const double 
     if (!((wR > p) && (vR[0] < Rt.lam + TOL) && (cR0 < lmaR + TOL))) return kHlldDefer;
     if (dfabs(cR0 - cL0) > T::contact) return kHlldDefer;
   }
-  if (!supersonic) {
-    // the first region of the reference's chain (:518-524) whose upper speed bounds s = 0;
-    // left of the contact up to region 2
+  // the first region of the reference's chain (:518-524) whose upper speed bounds s = 0; left of
+  // the contact up to region 2. The right fast wave is asked last, and nothing orders it
+  // against the right Alfven wave, so ap < 0 alone does not make the flux the right state's.
+  if (!supersonic || (!(0.0 <= L.lam) && (0.0 <= KL[0] || 0.0 <= cR0 || 0.0 <= KR[0]))) {
     const bool left = 0.0 <= KL[0] || 0.0 <= cR0;
     const bool outer = left ? 0.0 <= KL[0] : !(0.0 <= KR[0]);   // between the fast and the Alfven wave
     const double lam = left ? L.lam : Rt.lam;

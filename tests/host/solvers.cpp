@@ -1,0 +1,47 @@
+/* The FP64 Riemann solvers of rmhd_device.hpp at n interfaces normal to x, on the host: the
+ * sweeps' common path (lean) and the full solver. rc: 0, an error, or kHlldDefer = 100 where
+ * the common path hands the interface to the full solver (its flux is then not final). */
+#include "rmhd_device.hpp"
+
+using namespace maragpu;
+
+extern "C" {
+
+void lean(int solver, long n, const double *pl, const double *pr, double gamma, double pfloor, double *f, int *rc,
+          double *lam, int *steps)
+{
+  PhysParams pp = {};
+  pp.gamma = gamma;
+  pp.pfloor = pfloor;
+  pp.g1 = gamma / (gamma - 1.0);
+  pp.gamf = (gamma - 1.0) / gamma;
+  pp.igamma = 1.0 / gamma;
+#pragma omp parallel for
+  for (long i = 0; i < n; ++i) {
+    const double *l = pl + 8 * i, *r = pr + 8 * i;
+    FluxCounters fc = {0, 0, 0, 0};
+    auto store = [&](int q, double v) { f[8 * i + q] = v; };
+    lam[i] = 0.0;
+    rc[i] = solver == RIEMANN_HLLD ? riemann_hlld_lean<1>(l, r, pp, lam[i], fc, store)
+          : solver == RIEMANN_HLLC ? riemann_hllx_lean<RIEMANN_HLLC>(l, r, pp, lam[i], store)
+                                   : riemann_hllx_lean<RIEMANN_HLL>(l, r, pp, lam[i], store);
+    steps[i] = fc.newton_iters;
+  }
+}
+
+void full(int solver, long n, const double *pl, const double *pr, double gamma, double pfloor, double *f, int *rc,
+          double *lam, int *steps)
+{
+#pragma omp parallel for
+  for (long i = 0; i < n; ++i) {
+    const double *l = pl + 8 * i, *r = pr + 8 * i;
+    FluxCounters fc = {0, 0, 0, 0};
+    lam[i] = 0.0;
+    rc[i] = solver == RIEMANN_HLLD ? riemann_hlld<double, 1>(l, r, f + 8 * i, gamma, pfloor, lam[i], fc)
+          : solver == RIEMANN_HLLC ? riemann_hllc<double, 1>(l, r, f + 8 * i, gamma, lam[i])
+                                   : riemann_hll<double, 1>(l, r, f + 8 * i, gamma, lam[i]);
+    steps[i] = fc.newton_iters;
+  }
+}
+
+}

@@ -1,0 +1,75 @@
+"""The FP64 sweeps' common path (riemann_hlld_lean, riemann_hllx_lean) against the full solver
+it replaces and against the oracle, interface by interface. rmhd_device.hpp is compiled for
+the host with stand-ins for the hardware approximations (tests/host)."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HLL, HLLC, HLLD = 0, 1, 2
+DEFER = 100
+DOUBLES, INTS = ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int)
+
+
+class Solvers:
+    def __init__(self, path):
+        self.lib = ctypes.CDLL(path)
+
+    def __call__(self, which, solver, PL, PR, gamma=4.0 / 3.0, pfloor=0.0):
+        """Flux, return code, fastest speed and p* steps of n interfaces normal to x."""
+        PL, PR = np.ascontiguousarray(PL, dtype=float), np.ascontiguousarray(PR, dtype=float)
+        n = len(PL)
+        F, lam, rc, steps = np.zeros((n, 8)), np.zeros(n), np.zeros(n, np.int32), np.zeros(n, np.int32)
+        getattr(self.lib, which)(ctypes.c_int(solver), ctypes.c_long(n), PL.ctypes.data_as(DOUBLES),
+                                 PR.ctypes.data_as(DOUBLES), ctypes.c_double(gamma), ctypes.c_double(pfloor),
+                                 F.ctypes.data_as(DOUBLES), rc.ctypes.data_as(INTS), lam.ctypes.data_as(DOUBLES),
+                                 steps.ctypes.data_as(INTS))
+        return F, rc, lam, steps
+
+
+@pytest.fixture(scope="module")
+def solvers(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("host") / "solvers.so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-mfma", "-ffp-contract=fast", "-fopenmp", "-w", "-shared", "-fPIC",
+                    "-I", os.path.join(ROOT, "tests", "host"), "-I", os.path.join(ROOT, "ctf_amd", "csrc"),
+                    "-o", out, os.path.join(ROOT, "tests", "host", "solvers.cpp")], check=True)
+    return Solvers(out)
+
+
+# interfaces whose right fast wave moves left while the right Alfven wave moves right
+TRANS_FAST = [
+    ([6.2163, 0.46995, -0.2378, -0.7187, -0.473, 2.0485, 0.7083, -1.1451],
+     [8.0491, 0.24608, -0.55881, -0.41229, -0.21378, 2.0485, 1.3851, -0.22483]),
+    ([1.0805, 0.28644, -0.54631, 0.59338, -0.31491, 1.6803, 0.13063, -1.4054],
+     [1.1193, 0.1588, -0.65694, 0.10161, -0.53991, 1.6803, -0.89298, 0.2466]),
+    ([0.88341, 0.044542, -0.44481, 0.66776, -0.22813, -0.82136, 0.11297, 0.32027],
+     [0.34259, 0.023266, -0.66294, 0.21559, -0.52903, -0.82136, 0.48395, -0.17018]),
+    ([1.8798, 0.37374, -0.50156, 0.52429, 0.048764, -0.84443, 0.44374, 0.26674],
+     [1.0173, 0.17073, -0.40034, -0.11127, 0.5813, -0.84443, 0.080919, 0.052828]),
+    ([0.60645, 0.058776, -0.74339, -0.34436, -0.26366, 1.0373, -0.44309, 0.87441],
+     [0.3555, 0.030151, -0.75145, -0.36283, 0.20616, 1.0373, 0.18288, -0.027719]),
+    ([1.0031, 0.33669, -0.53523, -0.57094, 0.30507, -1.9073, 0.75086, -0.075821],
+     [0.8959, 0.1353, -0.79157, -0.26121, 0.22481, -1.9073, -0.10198, 0.063667]),
+    ([0.37575, 0.053587, -0.55838, -0.35888, -0.63519, 1.291, -0.17125, -0.28025],
+     [0.41098, 0.028817, -0.6138, -0.018785, -0.65501, 1.291, -0.21529, 0.046615]),
+]
+
+
+def test_trans_fast_fan(solvers, oracle_lib):
+    """HLLD accepts fans whose right fast wave lies left of the right Alfven wave; the wave chain
+    asks for the contact and the Alfven waves before the right fast wave
+    (Mara/riemann_hlld-rmhd.cpp:518-524), so s = 0 between them takes the state there and not
+    the right state. The flux of every interface that the common path keeps against the full
+    solver and the oracle, 1e-10 of its largest component."""
+    PL, PR = (np.array(side) for side in zip(*TRANS_FAST))
+    F, rc, _, _ = solvers("lean", HLLD, PL, PR)
+    G, full_rc, _, _ = solvers("full", HLLD, PL, PR)
+    O = np.array([oracle_lib.riemann("hlld", l[None], r[None], 1, 4.0 / 3.0)[0][0] for l, r in zip(PL, PR)])
+    assert (full_rc == 0).all() and np.isin(rc, (0, DEFER)).all()
+    scale = np.abs(G).max(axis=1, keepdims=True)
+    assert (np.abs(G - O) <= 1e-10 * scale).all()
+    keep = rc == 0
+    assert (np.abs(F - G)[keep] <= 1e-10 * scale[keep]).all()
