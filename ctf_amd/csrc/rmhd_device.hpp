@@ -41,13 +41,21 @@ template <> struct Tol<double> {
   static constexpr bool nested_c2p_from_average = true;
   static constexpr bool nested_c2p_fp32 = false;  // that attempt in FP64
   static constexpr double newton_ftol = 1e-12;   // NewtonRaphesonSolver(15, 1e-12), riemann_hlld-rmhd.cpp:220
-  // common path (riemann_hlld_lean): Newton steps of the p* solve (the reference's); the last
-  // one, from a residual within newton_ftol, reuses the derivative of the one before where
-  // it moves p by at most reuse_step, relatively; step tolerance and cap of the nested c2p,
-  // whose result only starts the p* solve. Where the Alfven speeds differ by less than
-  // weak_delK (a weak normal field) the solve ends early, below small_delK, or wanders: its
-  // result depends on the path, and the full solver takes the reference's path.
-  static constexpr int newton_fast_max_it = 15;
+  // common path (riemann_hlld_lean). The last Newton step of the p* solve, from a residual within
+  // newton_ftol, reuses the derivative of the one before where it moves p by at most
+  // reuse_step, relatively; step tolerance and cap of the nested c2p, whose result only starts
+  // the p* solve. Handed to the full solver, because there the result depends on the path that
+  // the solve takes, and the full solver takes the reference's:
+  //   - solves of lean_max_it steps and more, of the reference's 15 (2 in 1 000 of random
+  //     states; 1 in 100 of those with 14 steps ended at another root);
+  //   - solves whose residual has a round-off near newton_ftol. One ulp of p moves it by
+  //     2.2e-16 |p dy/dp|, so with |p dy/dp| > steep the reference's solve ends by chance, and
+  //     often not at all (p* of 10 and more, field-dominated states): of 829 random interfaces
+  //     decided otherwise than by the full solver 820 are above steep, of the rest 1 in 80;
+  //   - Alfven speeds that differ by less than weak_delK (a weak normal field): the solve ends
+  //     early, below small_delK, or wanders.
+  static constexpr int lean_max_it = 9;
+  static constexpr double steep = 27.0;
   static constexpr double reuse_step = 1e-11;
   static constexpr double nested_step = 1e-6;
   static constexpr int nested_max_it = 16;
@@ -2245,7 +2253,7 @@ __device__ __forceinline__ int riemann_hlld_lean(const double *pl, const double 
       if (mode == RESIDUAL) {
         const double ay = dfabs(y);
         const double dx = Gd*y;
-        if (have && it < T::newton_fast_max_it && ay <= T::newton_ftol && ay <= 0.05*dfabs(y0) &&
+        if (have && it < T::lean_max_it && ay <= T::newton_ftol && ay <= 0.05*dfabs(y0) &&
             dfabs(dx) <= T::reuse_step*dfabs(p)) {
           p -= dx;
           pe = p;
@@ -2263,7 +2271,7 @@ __device__ __forceinline__ int riemann_hlld_lean(const double *pl, const double 
         const double last = eps;
         eps = dfabs(y0);
         worse += (eps > last);
-        if (worse >= 10 || it == T::newton_fast_max_it || is_nan(eps)) { cnt.newton_iters += it; return kHlldDefer; }
+        if (worse >= 10 || it == T::lean_max_it || is_nan(eps)) { cnt.newton_iters += it; return kHlldDefer; }
         mode = SOLUTION;
         if (eps > T::newton_ftol) {
           ++it;
@@ -2275,7 +2283,7 @@ __device__ __forceinline__ int riemann_hlld_lean(const double *pl, const double 
     }
     cnt.newton_iters += it;
     p = pe;
-    if (!small_bn && dfabs(delK) < T::weak_delK) return kHlldDefer;
+    if (!small_bn && (dfabs(delK) < T::weak_delK || dfabs(p) > T::steep*dfabs(Gd))) return kHlldDefer;
   }
 
   // ReconstructSolution, :417-538, for s = 0

@@ -73,3 +73,48 @@ def test_trans_fast_fan(solvers, oracle_lib):
     assert (np.abs(G - O) <= 1e-10 * scale).all()
     keep = rc == 0
     assert (np.abs(F - G)[keep] <= 1e-10 * scale[keep]).all()
+
+
+def random_interfaces(rng, n, jump, W, beta):
+    """Interfaces with jumps of the given size between states with Lorentz factors up to W and
+    fields of the order of beta (log-normal), the normal field continuous."""
+    P = np.empty((n, 8))
+    P[:, 0] = np.exp(rng.normal(0.0, 1.0, n))
+    P[:, 1] = P[:, 0] * np.exp(rng.normal(-0.5, 1.2, n))
+    e = rng.normal(size=(n, 3))
+    w = 1.0 + (W - 1.0) * rng.uniform(0, 1, n)
+    P[:, 2:5] = e / np.linalg.norm(e, axis=1)[:, None] * np.sqrt(1.0 - w ** -2.0)[:, None]
+    P[:, 5:8] = beta * rng.normal(size=(n, 3)) * np.exp(rng.normal(-0.5, 1.0, n))[:, None]
+    Q = P.copy()
+    Q[:, :2] *= np.exp(jump * rng.uniform(-1, 1, (n, 2)))
+    u = P[:, 2:5] * w[:, None] + jump * rng.uniform(-1, 1, (n, 3))
+    Q[:, 2:5] = u / np.sqrt(1.0 + (u * u).sum(axis=1))[:, None]
+    Q[:, 5:8] += jump * np.abs(P[:, 5:8]).max(axis=1)[:, None] * rng.uniform(-1, 1, (n, 3))
+    Q[:, 5] = P[:, 5]
+    return P, Q
+
+
+@pytest.mark.parametrize("solver", [HLLD, HLLC, HLL])
+@pytest.mark.parametrize("beta", [0.1, 1.0, 3.0])
+def test_kept_interfaces_have_the_full_solvers_flux(solvers, solver, beta):
+    """What the common path keeps is what the full solver decides, also where the full p* solve
+    is at the end of its reach (many steps, a residual whose round-off is near its tolerance)
+    and falls to another attempt or to HLLC. 600 000 random interfaces: at most one kept
+    interface in 100 000 off by more than 1e-9 of its flux (some are so ill-conditioned
+    that round-off does it). Without a rule for such solves 1 in 600 of the HLLD ones are at
+    beta = 3, and 1 in 7 000 at beta = 1."""
+    rng = np.random.default_rng(12)
+    kept = off = 0
+    for jump in (1e-3, 0.02, 0.1, 0.3, 1.0):
+        for W in (1.05, 1.5, 3.0):
+            PL, PR = random_interfaces(rng, 40000, jump, W, beta)
+            F, rc, _, _ = solvers("lean", solver, PL, PR)
+            G, full_rc, _, _ = solvers("full", solver, PL, PR)
+            assert np.isin(rc, (0, DEFER)).all()
+            keep = rc == 0
+            assert (full_rc[keep] == 0).all()
+            d = np.abs(F - G).max(axis=1) / np.abs(G).max(axis=1)
+            kept += keep.sum()
+            off += (keep & ~(d <= 1e-9)).sum()
+    assert kept > 400000
+    assert off <= 1e-5 * kept
