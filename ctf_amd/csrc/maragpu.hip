@@ -1249,7 +1249,8 @@ void k_ctu_faces_fast(const double *__restrict__ P, FaceStates Ps, FluxPlanes<do
  * sweeps. Their states passed the physical check in the fast pass. A solver error leaves the
  * flux: it is then what the reference's array holds there, zero in step 2 (fresh arrays) and
  * the step-2 flux in step 4 (`keep`). A face whose fast waves both lie on one side may hold
- * that side's flux already; the solver then never fails there. */
+ * that side's flux already; the solver then never fails there (FastSide::set hands on what
+ * prim_to_cons might refuse before any flux is stored). */
 template <int SOLVER>
 __global__ __launch_bounds__(kBlock) void k_ctu_faces_redo(const double *__restrict__ P, FaceStates Ps,
                                                            FluxPlanes<double> Fo, GridDesc g, PhysParams pp, int keep,

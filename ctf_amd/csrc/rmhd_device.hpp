@@ -1820,8 +1820,8 @@ __device__ __forceinline__ int riemann_hlld(const R *pl, const R *pr, R *f, R ga
  *     four evaluations of the fan per interface where centred differences take seven.
  * ------------------------------------------------------------------------- */
 /* One side of an interface in the x-normal frame: D, E = tau + D, S, the fluxes and the
- * fast speeds (Mara/rmhd.cpp:133-265). False for a state that prim_to_cons would refuse or
- * whose speeds need the general cubic. */
+ * fast speeds (Mara/rmhd.cpp:133-265). False for a state that prim_to_cons would or might
+ * refuse or whose speeds need the general cubic. */
 struct FastSide {
   double D, E, S[3], B[3];
   double FD, FS[3], FB2, FB3;      // the energy flux is S[0], the normal field's is zero
@@ -1842,8 +1842,10 @@ struct FastSide {
     const double pt = P[pre] + 0.5*b2;
     D = P[rho]*W;
     E = wW2 - pt - b0*b0;
-    // NaN in any primitive reaches E
-    if (!(D >= 0.0) || !(E - D >= 0.0)) return false;
+    // NaN in any primitive reaches E. Without density prim_to_cons, which divides by it, has no
+    // conserved state; and where tau = E - D is within round-off of zero its sign, formed
+    // there in another order, may be the other one
+    if (!(D > 0.0) || !(E - D >= 1e-14*E)) return false;
     S[0] = wW2*P[vx] - b0*bx;
     S[1] = wW2*P[vy] - b0*by;
     S[2] = wW2*P[vz] - b0*bz;
@@ -1888,9 +1890,11 @@ __device__ __forceinline__ void side_flux_lean(const double *P, double g1, doubl
   const double b0 = W*Bv;
   const double b2 = (B2 + b0*b0)*om;
   const double bx = P[Bx]*iW + b0*P[vx], by = P[By]*iW + b0*P[vy], bz = P[Bz]*iW + b0*P[vz];
-  const double wW2 = (P[rho] + g1*P[pre] + b2)*W2;
+  // no flux without density, as from the conserved state (prim_to_cons divides by it)
+  const double r = P[rho] == 0.0 ? NAN : P[rho];
+  const double wW2 = (r + g1*P[pre] + b2)*W2;
   const double pt = P[pre] + 0.5*b2;
-  const double D = P[rho]*W;
+  const double D = r*W;
   const double v = P[vx], BiW = P[Bx]*iW;
   F[ddd] = D*v;
   F[tau] = (wW2 - pt - b0*b0 - D)*v - b0*BiW + pt*v;

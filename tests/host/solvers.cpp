@@ -44,4 +44,16 @@ void full(int solver, long n, const double *pl, const double *pr, double gamma, 
   }
 }
 
+/* the predictor's flux of a physical state (plm-muscl) and the reference's, from its conserved state */
+void side_flux(long n, const double *p, double gamma, double *lean_f, double *full_f)
+{
+  for (long i = 0; i < n; ++i) {
+    const double *P = p + 8 * i;
+    side_flux_lean(P, gamma / (gamma - 1.0), lean_f + 8 * i);
+    double U[8], a, b;
+    prim_to_cons(P, U, gamma - 1.0);
+    flux_and_eigenvalues<double, 1, false>(U, P, full_f + 8 * i, a, b, gamma);
+  }
+}
+
 }
