@@ -526,7 +526,7 @@ __device__ __forceinline__ int interface_flux(const double *__restrict__ P, long
                                               int &retried, bool *lead = nullptr)
 {
   R ql[8], qr[8];
-  reconstruct_states<R, false>(P, T, S, axis, z, recon, pp, ql, qr);
+  reconstruct_states<R, false, false>(P, T, S, axis, z, recon, pp, ql, qr);
   int err = 1;
   retried = 0;
   // one call site: the reconstructed states, then the zone-centred states
@@ -563,7 +563,7 @@ __device__ __forceinline__ int interface_flux_fast(const double *__restrict__ P,
                                                    FluxCounters &fc)
 {
   R ql[8], qr[8];
-  reconstruct_states<R, sizeof(R) == 8>(P, T, S, axis, z, recon, pp, ql, qr);
+  reconstruct_states<R, sizeof(R) == 8, true>(P, T, S, axis, z, recon, pp, ql, qr);
   auto store = [&](int q, R f) { Fout[axis_plane(q, axis) * T + z] = f; };
   if constexpr (sizeof(R) == 8 && SOLVER == RIEMANN_HLLD) return riemann_hlld_lean<1>(ql, qr, pp, lam, fc, store);
   else if constexpr (sizeof(R) == 8) return riemann_hllx_lean<SOLVER>(ql, qr, pp, lam, store);
@@ -1174,7 +1174,7 @@ __global__ __launch_bounds__(kBlock) void k_flux_weno_split_char_redo(const doub
  * ------------------------------------------------------------------------ */
 /* the operator's own limited slope (plm_minmod with its theta, :22-31) of a field's plane Pq
  * along S at zone z, zero outside the flat range [sx, T - sx) where the reference computes
- * slopes; the minmod as in plm() */
+ * slopes */
 __device__ __forceinline__ double ctu_slope(const double *__restrict__ Pq, long T, long sxz, long z, long S, double theta)
 {
 #pragma clang fp contract(off)
@@ -1183,7 +1183,7 @@ __device__ __forceinline__ double ctu_slope(const double *__restrict__ Pq, long 
   const double a = theta * (u0 - ul);
   const double b = 0.5 * (ur - ul);
   const double c = theta * (ur - u0);
-  return fmax(fmin(fmin(a, b), c), 0.0) + fmin(fmax(fmax(a, b), c), 0.0);
+  return minmod(a, b, c);
 }
 
 /* the half-slope states, in the axis's frame, of face z | z+S along the axis: from P with its

@@ -56,4 +56,17 @@ void side_flux(long n, const double *p, double gamma, double *lean_f, double *fu
   }
 }
 
+/* plm at the face ahead of n values (behind, centre, ahead), in general and as the sweeps that
+ * hand on take it, in FP64 and FP32 */
+void plm_ahead(long n, const double *v, double theta, double *d, double *d_hand_on, float *f, float *f_hand_on)
+{
+  for (long i = 0; i < n; ++i) {
+    const double a = v[3 * i], b = v[3 * i + 1], c = v[3 * i + 2];
+    d[i] = plm<double>(a, b, c, 1.0, theta);
+    d_hand_on[i] = plm<double, true>(a, b, c, 1.0, theta);
+    f[i] = plm<float>((float)a, (float)b, (float)c, 1.0f, (float)theta);
+    f_hand_on[i] = plm<float, true>((float)a, (float)b, (float)c, 1.0f, (float)theta);
+  }
+}
+
 }

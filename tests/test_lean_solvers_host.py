@@ -37,6 +37,13 @@ class Solvers:
                            F.ctypes.data_as(DOUBLES), G.ctypes.data_as(DOUBLES))
         return F, G
 
+    def plm_ahead(self, V, theta):
+        V = np.ascontiguousarray(V, dtype=float)
+        out = [np.zeros(len(V), t) for t in (np.float64, np.float64, np.float32, np.float32)]
+        self.lib.plm_ahead(ctypes.c_long(len(V)), V.ctypes.data_as(DOUBLES), ctypes.c_double(theta),
+                           *(o.ctypes.data_as(ctypes.c_void_p) for o in out))
+        return out
+
 
 @pytest.fixture(scope="module")
 def solvers(tmp_path_factory):
@@ -165,3 +172,27 @@ def test_side_flux_without_density_is_not_a_number(solvers):
     PL, _ = random_interfaces(np.random.default_rng(3), 20000, 0.1, 1.5, 1.0)
     F, G = solvers.side_flux(PL)
     assert (np.abs(F - G).max(axis=1) <= 1e-13 * np.abs(G).max(axis=1)).all()
+
+
+@pytest.mark.parametrize("theta", [1.0, 1.5, 2.0])
+def test_plm_with_infinities_and_not_a_number(solvers, oracle_lib, theta):
+    """The limited state of every triple of ordinary, infinite and not-a-number values is the
+    oracle's (equal as numbers or both not a number; with an infinite centre both are infinite or
+    not a number, which no solver takes); the form for sweeps that hand such states on gives
+    the same or, where one of the three is not finite, not a number. FP32 likewise, by the same
+    values (all exact there)."""
+    x = [-np.inf, -2.0, -1.0, -0.25, 0.0, 0.5, 1.0, 2.0, np.inf, np.nan]
+    V = np.array(np.meshgrid(x, x, x, indexing="ij")).reshape(3, -1).T
+    V6 = np.zeros((len(V), 6))
+    V6[:, 1:4] = V
+    # the oracle takes 6 values v[-2..3]; PLM uses v[-1..1]
+    ref = oracle_lib.reconstruct(V6, "PLM_C2R", theta=theta)
+    finite = np.isfinite(V).all(axis=1)
+    for got, hand_on in zip(*[iter(solvers.plm_ahead(V, theta))] * 2):
+        some = ~np.isinf(V[:, 1])
+        assert np.array_equal(got[some].astype(float), ref[some], equal_nan=True)
+        assert not np.isfinite(got[~some]).any() and not np.isfinite(ref[~some]).any()
+        assert np.array_equal(hand_on[finite].astype(float), ref[finite])
+        assert (np.isnan(hand_on) | (hand_on.astype(float) == ref)).all()
+        # a value that is not a number never goes unseen
+        assert np.isnan(hand_on[np.isnan(V).any(axis=1)]).all()
