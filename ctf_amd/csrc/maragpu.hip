@@ -69,6 +69,9 @@ template <typename R, int SOLVER> constexpr int fast_flux_waves()
 // grid of the redo kernels (a grid-stride loop over the queue): one block per CU, all that their
 // registers let be resident
 constexpr int kRedoBlocks = 256;
+// the bulk kernels: a block per CU, 2 waves per SIMD (a grid that exits at once, the usual case,
+// costs a stage 3 us; with two blocks per CU 5 us)
+constexpr int kBulkBlocks = 256, kBulkBlock = 512;
 
 /* Device-side counters of one step; reduced per block, then atomically. */
 struct DevStats {
@@ -92,22 +95,58 @@ struct DevStats {
   unsigned long long ctu_failed[4][4]; // plm-muscl: failed checks per stage and abort point
 };
 
-/* Interfaces of the HLLD sweeps handed to the full FP64 solver (k_flux_redo) before the
- * update reads the fluxes: in the mixed form those whose FP32 HLLD solve failed, in the
- * plain form those outside the common path of the lean sweep (k_flux_fast). One list
- * per axis. */
+/* Interfaces handed on by the sweeps before the update reads the fluxes: to the full FP64 solver
+ * (k_flux_redo; in the mixed form those whose FP32 HLLD solve failed, in the plain form those
+ * outside the common path of the lean sweep, k_flux_fast), or to the general eigensystem
+ * (weno-split, eigen = RMHD).
+ * A set is eight lists, one per XCD: an atomic on a counter takes 8 ns when all waves of the
+ * chip meet on it (128^3, every interface handed on: 800 us of 1315 in k_flux_fast). Up to
+ * three sets: the sweeps' own, and what the bulk kernels leave of it; or, for the
+ * characteristic sweeps, one per axis. */
+constexpr int kQueueLists = 8, kQueueSets = 3;
+constexpr int kCountStride = 32;         // counters 128 B apart
 struct RedoQueue {
-  unsigned int *count;     // device counters, one per axis; cleared before the sweeps (clear_queue)
-  unsigned int cap;        // slots of an axis
-  unsigned int *z;         // device slots, cap per axis: interface index z (left zone; T < 2^32)
+  unsigned int *count;     // device counters; cleared before the sweeps (clear_queue)
+  unsigned int cap;        // slots of a list
+  unsigned int *z;         // device slots: axis << 30 | interface index z (left zone; T <= 2^30)
   uint4 *part;             // per wave of the sweeps: its counters, summed by the redo
+  __host__ __device__ RedoQueue set(int k) const
+  {
+    return { count + k * kQueueLists * kCountStride, cap, z + (size_t)k * kQueueLists * cap, part };
+  }
+};
+
+/* A longer queue than this goes through the bulk kernel first: 16 lanes for each interface of a
+ * shorter one fill the redo kernel's grid once. */
+constexpr unsigned kShortQueue = 4096;
+
+/* A set's entries counted through its lists. The counts are uniform: scalar loads. */
+struct QueueView {
+  unsigned n = 0, first[kQueueLists];
+  __device__ __forceinline__ explicit QueueView(const RedoQueue &rq)
+  {
+#pragma unroll
+    for (int l = 0; l < kQueueLists; ++l) {
+      first[l] = n;
+      n += min(rq.count[l * kCountStride], rq.cap);
+    }
+  }
+  __device__ __forceinline__ void entry(const RedoQueue &rq, unsigned k, int &axis, long &z) const
+  {
+    unsigned at = k;                     // 8 cap < 2^32
+#pragma unroll
+    for (int l = 1; l < kQueueLists; ++l) at = k >= first[l] ? (unsigned)l * rq.cap + (k - first[l]) : at;
+    const unsigned e = rq.z[at];
+    axis = (int)(e >> 30);
+    z = (long)(e & 0x3fffffffu);
+  }
 };
 
 /* The kernel before a stage's sweeps (the step start, or the previous stage's update) clears
  * the queue's counts: whoever read them has finished, and the sweeps follow in stream order. */
 __device__ __forceinline__ void clear_queue(unsigned int *count)
 {
-  if (count && blockIdx.x == 0 && threadIdx.x < 3) count[threadIdx.x] = 0u;
+  if (count && blockIdx.x == 0 && threadIdx.x < kQueueSets * kQueueLists) count[threadIdx.x * kCountStride] = 0u;
 }
 
 struct GridDesc {
@@ -236,12 +275,13 @@ __device__ __forceinline__ bool queue_push(const RedoQueue &rq, int axis, bool p
   const int lane = (int)(threadIdx.x & 63);
   const int leader = __ffsll((unsigned long long)m) - 1;
   unsigned int base = 0u;
-  if (lane == leader) base = atomicAdd(rq.count + axis, (unsigned int)__popcll(m));
+  const unsigned l = blockIdx.x & (kQueueLists - 1);       // the block's XCD
+  if (lane == leader) base = atomicAdd(rq.count + l * kCountStride, (unsigned int)__popcll(m));
   base = (unsigned int)__shfl((int)base, leader);
   if (!push) return true;
   const unsigned int k = base + (unsigned int)__popcll(m & ((1ull << lane) - 1ull));
   if (k >= rq.cap) return false;
-  rq.z[(size_t)axis * rq.cap + k] = (unsigned int)z;
+  rq.z[(size_t)l * rq.cap + k] = (unsigned int)axis << 30 | (unsigned int)z;
   return true;
 }
 
@@ -796,6 +836,56 @@ void k_flux_fast(const double *__restrict__ P, FluxPlanes<R> Fo, GridDesc g, Swe
   sweep_counters_wave(lam_out, cnt[0] != 0, (unsigned)cnt[1], (unsigned)cnt[2], false, rq.part);
 }
 
+/* A long queue of the FP64 HLLD sweeps (a weak normal field, below 1e-5, or a field that dominates
+ * takes most interfaces off the lean path): the full solver's steps up to its first attempt,
+ * riemann_hlld's FAST mode, which nearly all of them end with; the rest goes to the queue's
+ * second set for k_flux_redo. The full solver needs over 400 registers, one wave per SIMD;
+ * this part of it 2 waves. At 128^3 WENO5 with every interface handed on, a step takes 6.6 ms;
+ * 13.4 ms with the full solver alone and one counter for each axis's queue; 2.9 ms where none
+ * is. `states` gives an interface's two states. */
+template <typename States>
+__device__ __forceinline__ void bulk_pass(const RedoQueue &rq, const QueueView &view, const FluxPlanes<double> &Fo, long T,
+                                          const PhysParams &pp, DevStats *st, States states)
+{
+  double lam_out = 0.0;
+  unsigned int done_n = 0, c2p_n = 0, newton_n = 0;
+  const RedoQueue rest = rq.set(1);
+  for (unsigned k = blockIdx.x * blockDim.x + threadIdx.x; k < view.n; k += gridDim.x * blockDim.x) {
+    int axis;
+    long z;
+    view.entry(rq, k, axis, z);
+    double ql[8], qr[8], f[8], lam = 0.0;
+    FluxCounters fc = {0, 0, 0, 0};
+    states(axis, z, ql, qr);
+    const bool done = riemann_hlld<double, 1, true>(ql, qr, f, pp.gamma, pp.pfloor, lam, fc) == 0;
+    if (done) {
+      double *__restrict__ F = axis == 0 ? Fo.f[0] : axis == 1 ? Fo.f[1] : Fo.f[2];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) F[axis_plane(q, axis) * T + z] = f[q];
+      done_n += 1;
+      c2p_n += (unsigned)fc.c2p_iters;
+      newton_n += (unsigned)fc.newton_iters;
+    }
+    lam_out = fmax(lam_out, lam);
+    queue_push(rest, axis, !done, z);
+  }
+  block_max_lambda<kBulkBlock>(lam_out, &st->lam_bits);
+  const unsigned long long cnt[4] = { done_n, c2p_n, newton_n, done_n };
+  unsigned long long *const dst[4] = { &st->hlld_success, &st->hlld_c2p_iters, &st->hlld_newton_iters, &st->redo };
+  block_add<4, kBulkBlock>(cnt, dst);
+}
+
+__global__ __launch_bounds__(kBulkBlock, 2) void k_flux_bulk(const double *__restrict__ P, FluxPlanes<double> Fo,
+                                                             GridDesc g, int recon, PhysParams pp, DevStats *st,
+                                                             RedoQueue rq)
+{
+  const QueueView view(rq);
+  if (view.n <= kShortQueue) return;
+  bulk_pass(rq, view, Fo, g.T, pp, st, [&](int axis, long z, double *ql, double *qr) {
+    reconstruct_states<double, false, false>(P, g.T, axis_stride(g, axis), axis, z, recon, pp, ql, qr);
+  });
+}
+
 /* The queued interfaces of the sweeps, recomputed by the full FP64 method (reconstruction,
  * HLLD attempt ladder, HLLC fallback, retry) and written over the sweep's fluxes (FP32
  * in the mixed form, FP64 in the plain one). A grid-stride loop over each axis's list; the
@@ -805,6 +895,11 @@ __global__ __launch_bounds__(kBlock) void k_flux_redo(const double *__restrict__
                                                       int recon, PhysParams pp, DevStats *st, RedoQueue rq,
                                                       unsigned int nparts)
 {
+  QueueView view(rq);
+  if (SOLVER == RIEMANN_HLLD && sizeof(FT) == 8 && view.n > kShortQueue) {    // k_flux_bulk's rest
+    rq = rq.set(1);
+    view = QueueView(rq);
+  }
   double lam_out = 0.0;
   unsigned long long cnt[7] = {0, 0, 0, 0, 0, 0, 0};
   // the sweeps' per-wave counters (nparts waves)
@@ -816,18 +911,16 @@ __global__ __launch_bounds__(kBlock) void k_flux_redo(const double *__restrict__
     cnt[5] += (unsigned long long)(v.w & 0xffffu);
   }
   const long T = g.T;
-  // k counts through the three lists. Up to 4096 interfaces (16 lanes each fill the grid once)
-  // the kernel is bound by the latency of one interface's attempt ladder, and 16 lanes share
-  // an interface: 52 -> 29 us for the 8 a stage of a 64^3 step, 105 -> 39 us at 131x94x113.
-  // Above, one lane each, dealt out over the waves first, so that every SIMD has a few.
-  const unsigned int n0 = min(rq.count[0], rq.cap), n1 = min(rq.count[1], rq.cap), n2 = min(rq.count[2], rq.cap);
-  const unsigned long n = (unsigned long)n0 + n1 + n2;
+  // Up to kShortQueue interfaces the kernel is bound by the
+  // latency of one interface's attempt ladder, and 16 lanes share an interface: 52 -> 29 us
+  // for the 8 a stage of a 64^3 step, 105 -> 39 us at 131x94x113. Above, one lane each, dealt out over the waves first, so that every SIMD has a few.
+  const unsigned n = view.n;
   const unsigned tid = blockIdx.x * blockDim.x + threadIdx.x, nthreads = gridDim.x * blockDim.x;
-  auto redo = [&](unsigned long k, auto group) {
+  auto redo = [&](unsigned k, auto group) {
     constexpr bool GROUP = decltype(group)::value;
-    const int axis = k < n0 ? 0 : k < (unsigned long)n0 + n1 ? 1 : 2;
-    const unsigned long i = axis == 0 ? k : axis == 1 ? k - n0 : k - n0 - n1;
-    const long z = (long)rq.z[(size_t)axis * rq.cap + i];
+    int axis;
+    long z;
+    view.entry(rq, k, axis, z);
     double lam = 0.0;
     FluxCounters fc = {0, 0, 0, 0};
     double F[8];
@@ -848,10 +941,10 @@ __global__ __launch_bounds__(kBlock) void k_flux_redo(const double *__restrict__
     cnt[5] += (unsigned long long)fc.newton_iters;
     cnt[6] += 1;
   };
-  if (SOLVER == RIEMANN_HLLD && n * 16 <= nthreads)
-    for (unsigned long k = tid >> 4; k < n; k += nthreads >> 4) redo(k, std::integral_constant<bool, SOLVER == RIEMANN_HLLD>());
+  if (SOLVER == RIEMANN_HLLD && n <= kShortQueue)
+    for (unsigned k = tid >> 4; k < n; k += nthreads >> 4) redo(k, std::integral_constant<bool, SOLVER == RIEMANN_HLLD>());
   else
-    for (unsigned long k = (tid & 63) * (nthreads >> 6) + (tid >> 6); k < n; k += nthreads) redo(k, std::false_type());
+    for (unsigned k = (tid & 63) * (nthreads >> 6) + (tid >> 6); k < n; k += nthreads) redo(k, std::false_type());
   block_max_lambda(lam_out, &st->lam_bits);
   unsigned long long *const dst[7] = { &st->hlld_success, &st->hlld_failure, &st->retries,
                                        &st->failures, &st->hlld_c2p_iters, &st->hlld_newton_iters,
@@ -1131,7 +1224,7 @@ __global__ __launch_bounds__(kBlock, 3) void k_flux_weno_split_char(const double
     char_flux<R>(Uw, FZ, AZ, Fout, T, S, axis, z, lane, Lrow, Rrow, lds[threadIdx.x >> 6].a + base,
                  lds[threadIdx.x >> 6].r + base, pp);
   }
-  queue_push(rq, axis, valid && !done && lane == 0, z);
+  queue_push(rq.set(axis), axis, valid && !done && lane == 0, z);
 }
 
 /* The queued interfaces, with the general eigensystem (eig::g8::rmhd_eigensystem; the identity
@@ -1148,9 +1241,12 @@ __global__ __launch_bounds__(kBlock) void k_flux_weno_split_char_redo(const doub
   const long T = g.T, S = axis_stride(g, axis);
   const int lane = (int)(threadIdx.x & 7);
   double *const Fp = split[threadIdx.x >> 3];
-  const unsigned n = min(rq.count[axis], rq.cap);
-  for (unsigned e = (blockIdx.x * blockDim.x + threadIdx.x) >> 3; e < n; e += (gridDim.x * blockDim.x) >> 3) {
-    const long z = (long)rq.z[(size_t)axis * rq.cap + e];
+  rq = rq.set(axis);
+  const QueueView view(rq);
+  for (unsigned e = (blockIdx.x * blockDim.x + threadIdx.x) >> 3; e < view.n; e += (gridDim.x * blockDim.x) >> 3) {
+    long z;
+    int a;
+    view.entry(rq, e, a, z);
     double Lrow[8], Rrow[8], lam[8], Ph[8];
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
@@ -1245,6 +1341,17 @@ void k_ctu_faces_fast(const double *__restrict__ P, FaceStates Ps, FluxPlanes<do
   sweep_counters_wave(lam_out, cnt[1] != 0, (unsigned)cnt[2], (unsigned)cnt[3], cnt[0] != 0, rq.part);
 }
 
+__global__ __launch_bounds__(kBulkBlock, 2) void k_ctu_faces_bulk(const double *__restrict__ P, FaceStates Ps,
+                                                                  FluxPlanes<double> Fo, GridDesc g, PhysParams pp,
+                                                                  DevStats *st, RedoQueue rq)
+{
+  const QueueView view(rq);
+  if (view.n <= kShortQueue) return;
+  bulk_pass(rq, view, Fo, g.T, pp, st, [&](int axis, long z, double *pl, double *pr) {
+    ctu_face_states(P, axis == 0 ? Ps.p[0] : axis == 1 ? Ps.p[1] : Ps.p[2], g, axis, z, pp.theta, pl, pr);
+  });
+}
+
 /* The queued faces of k_ctu_faces_fast by the full solver, as k_flux_redo does it for the
  * sweeps. Their states passed the physical check in the fast pass. A solver error leaves the
  * flux: it is then what the reference's array holds there, zero in step 2 (fresh arrays) and
@@ -1257,6 +1364,11 @@ __global__ __launch_bounds__(kBlock) void k_ctu_faces_redo(const double *__restr
                                                            DevStats *st, unsigned long long *fail, RedoQueue rq,
                                                            unsigned int nparts)
 {
+  QueueView view(rq);
+  if (SOLVER == RIEMANN_HLLD && view.n > kShortQueue) {    // k_ctu_faces_bulk's rest
+    rq = rq.set(1);
+    view = QueueView(rq);
+  }
   const long T = g.T;
   double lam_out = 0.0;
   unsigned long long cnt[6] = {0, 0, 0, 0, 0, 0};
@@ -1269,12 +1381,10 @@ __global__ __launch_bounds__(kBlock) void k_ctu_faces_redo(const double *__restr
     cnt[3] += (unsigned long long)(v.w & 0xffffu);
     cnt[5] += (unsigned long long)(v.w >> 16);
   }
-  const unsigned int n0 = min(rq.count[0], rq.cap), n1 = min(rq.count[1], rq.cap), n2 = min(rq.count[2], rq.cap);
-  const unsigned long n = (unsigned long)n0 + n1 + n2;
-  for (unsigned long k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-    const int axis = k < n0 ? 0 : k < (unsigned long)n0 + n1 ? 1 : 2;
-    const unsigned long i = axis == 0 ? k : axis == 1 ? k - n0 : k - n0 - n1;
-    const long z = (long)rq.z[(size_t)axis * rq.cap + i];
+  for (unsigned k = blockIdx.x * blockDim.x + threadIdx.x; k < view.n; k += gridDim.x * blockDim.x) {
+    int axis;
+    long z;
+    view.entry(rq, k, axis, z);
     double *__restrict__ F = axis == 0 ? Fo.f[0] : axis == 1 ? Fo.f[1] : Fo.f[2];
     double pl[8], pr[8], f[8], lam = 0.0;
     ctu_face_states(P, axis == 0 ? Ps.p[0] : axis == 1 ? Ps.p[1] : Ps.p[2], g, axis, z, pp.theta, pl, pr);
@@ -2410,6 +2520,8 @@ void launch_flux_fast(maragpu_ctx *c, const PhysParams &pp, const FluxPlanes<R> 
   const unsigned nb = sg.first[3];
   if (!nb) return;
   k_flux_fast<R, SOLVER><<<nb, kFluxBlock<R>, 0, c->stream>>>(c->Pw, F, c->g, sg, c->cfg.recon, pp, c->redo);
+  if constexpr (SOLVER == RIEMANN_HLLD && sizeof(R) == 8)
+    k_flux_bulk<<<kBulkBlocks, kBulkBlock, 0, c->stream>>>(c->Pw, F, c->g, c->cfg.recon, pp, c->dstats, c->redo);
   k_flux_redo<R, SOLVER><<<kRedoBlocks, kBlock, 0, c->stream>>>(c->Pw, F, c->g, c->cfg.recon, pp, c->dstats, c->redo,
                                                                nb * (kFluxBlock<R> / 64));
 }
@@ -2443,7 +2555,17 @@ void launch_faces(maragpu_ctx *c, const PhysParams &pp, const FaceStates &Ps, co
   const unsigned nb = sg.first[3];
   if (!nb) return;
   k_ctu_faces_fast<SOLVER><<<nb, kFluxBlock<double>, 0, c->stream>>>(c->Pw, Ps, F, c->g, sg, pp, c->redo);
+  if constexpr (SOLVER == RIEMANN_HLLD)
+    k_ctu_faces_bulk<<<kBulkBlocks, kBulkBlock, 0, c->stream>>>(c->Pw, Ps, F, c->g, pp, c->dstats, c->redo);
   k_ctu_faces_redo<SOLVER><<<kRedoBlocks, kBlock, 0, c->stream>>>(c->Pw, Ps, F, c->g, pp, keep, c->dstats, fail, c->redo, nb);
+}
+
+/* blocks of the characteristic sweep along an axis: 8 lanes to an interface */
+inline long char_blocks(const GridDesc &g, int axis)
+{
+  const long n = (long)(axis == 0 ? g.N[0] + 1 : g.n[0]) * (axis == 1 ? g.N[1] + 1 : g.n[1]) *
+                 (axis == 2 ? g.N[2] + 1 : g.n[2]);
+  return nblocks(8 * n);
 }
 
 /* weno-split sweep along an axis: component-wise in one kernel, or the zone fluxes and speeds
@@ -2465,10 +2587,9 @@ void launch_weno_split(maragpu_ctx *c, const PhysParams &pp)
   R *FZ = static_cast<R *>(c->FZ);
   R *AZ = FZ + 8 * g.T;
   k_zone_flux<R><<<nblocks(g.T), kBlock, 0, c->stream>>>(c->Uw, c->Pw, FZ, AZ, g, DIM - 1, pp, c->dstats);
-  const long cnt = (long)(DIM == 1 ? g.N[0] + 1 : g.n[0]) * (DIM == 2 ? g.N[1] + 1 : g.n[1]) *
-                   (DIM == 3 ? g.N[2] + 1 : g.n[2]);
-  k_flux_weno_split_char<R><<<nblocks(8 * cnt), kBlock, 0, c->stream>>>(c->Uw, c->Pw, FZ, AZ, F, g, DIM - 1, pp, c->redo);
-  k_flux_weno_split_char_redo<R><<<std::min(nblocks(8 * cnt), 2048u), kBlock, 0, c->stream>>>(
+  const unsigned nb = (unsigned)char_blocks(g, DIM - 1);
+  k_flux_weno_split_char<R><<<nb, kBlock, 0, c->stream>>>(c->Uw, c->Pw, FZ, AZ, F, g, DIM - 1, pp, c->redo);
+  k_flux_weno_split_char_redo<R><<<std::min(nb, 2048u), kBlock, 0, c->stream>>>(
       c->Uw, c->Pw, FZ, AZ, F, g, DIM - 1, pp, c->dstats, c->redo);
 }
 
@@ -2581,18 +2702,34 @@ int maragpu_create(const maragpu_config *cfg, maragpu_ctx **out)
   }
   if (cfg->godunov == MARAGPU_WENO_SPLIT ? cfg->eigen == MARAGPU_EIG_RMHD
                                          : cfg->riemann == MARAGPU_HLLD || cfg->precision == MARAGPU_FP64) {
-    // a slot for every interface of a sweep or face pass (4 bytes a slot: half a state plane
-    // for an axis), and per-wave counters of the three sweeps
+    // a slot for every interface of the sweeps or of a face pass (4 bytes a slot) in each set, by
+    // the blocks that an XCD takes, and per-wave counters of the three sweeps
+    if (c->g.T > (1L << 30)) return fail_free(c);            // the entries' 30 bits; 500 GB of zones
     RedoQueue &q = c->redo;
-    q.cap = (unsigned int)c->g.T;
-    unsigned waves;
-    if (cfg->godunov == MARAGPU_WENO_SPLIT) waves = 0;       // its queue has no counters
-    else if (cfg->godunov == MARAGPU_PLM_MUSCL) waves = face_grid(c->g, 0, kFluxBlock<double>).first[3];
-    else if (cfg->precision == MARAGPU_MIXED) waves = sweep_grid(c->g, kFluxBlock<float>).first[3] * (kFluxBlock<float> / 64);
-    else waves = sweep_grid(c->g, kFluxBlock<double>).first[3];
-    static_assert(kFluxBlock<double> == 64, "one wave per FP64 block");
-    if (hipMalloc(&q.count, 3 * sizeof(unsigned int)) != hipSuccess ||
-        hipMalloc(&q.z, 3 * (size_t)q.cap * sizeof(unsigned int)) != hipSuccess ||
+    unsigned waves = 0;              // weno-split: its queue has no counters
+    long slots = 0;                  // of a list
+    int sets = 1;
+    if (cfg->godunov == MARAGPU_WENO_SPLIT) {
+      for (int d = 0; d < 3; ++d)
+        slots = std::max(slots, (char_blocks(c->g, d) + kQueueLists - 1) / kQueueLists * (kBlock / 8));
+      sets = 3;
+    }
+    else {
+      const bool mixed = cfg->precision == MARAGPU_MIXED;
+      const int block = mixed ? kFluxBlock<float> : kFluxBlock<double>;
+      const unsigned blocks = cfg->godunov == MARAGPU_PLM_MUSCL ? face_grid(c->g, 0, block).first[3]
+                                                                : sweep_grid(c->g, block).first[3];
+      waves = blocks * (block / 64);
+      slots = (long)blocks / kQueueLists * block;            // each axis has a multiple of 8 blocks
+      if (cfg->riemann == MARAGPU_HLLD && !mixed) {
+        // and what the bulk kernel's blocks of an XCD may leave, which deal the queue out anew
+        slots += kBulkBlocks / kQueueLists * kBulkBlock;
+        sets = 2;
+      }
+    }
+    q.cap = (unsigned)slots;
+    if (hipMalloc(&q.count, kQueueSets * kQueueLists * kCountStride * sizeof(unsigned int)) != hipSuccess ||
+        hipMalloc(&q.z, sets * kQueueLists * (size_t)std::max(q.cap, 1u) * sizeof(unsigned int)) != hipSuccess ||
         hipMalloc(&q.part, (size_t)std::max(waves, 1u) * sizeof(uint4)) != hipSuccess)
       return fail_free(c);
   }

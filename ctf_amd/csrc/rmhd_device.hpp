@@ -53,13 +53,16 @@ template <> struct Tol<double> {
   //     often not at all (p* of 10 and more, field-dominated states): of 829 random interfaces
   //     decided otherwise than by the full solver 820 are above steep, of the rest 1 in 80;
   //   - Alfven speeds that differ by less than weak_delK (a weak normal field): the solve ends
-  //     early, below small_delK, or wanders.
+  //     early, below small_delK, or wanders. They differ by 1.8 to 2.6 |Bn| / sqrt(El + Er), so
+  //     with Bn^2 < weak_Bn2 (El + Er) the solve need not be begun.
   static constexpr int lean_max_it = 9;
+  static constexpr int newton_fast_max_it = 15;  // riemann_hlld's FAST mode: the full solver's
   static constexpr double steep = 27.0;
   static constexpr double reuse_step = 1e-11;
   static constexpr double nested_step = 1e-6;
   static constexpr int nested_max_it = 16;
   static constexpr double weak_delK = 1e-6;
+  static constexpr double weak_Bn2 = 1.5e-13;
   static constexpr double fd_dp = 1e-8;          // HlldEquation48::Jacobian, :313
   static constexpr bool fd_relative = false;
   static constexpr bool fd_one_sided = false;    // the reference's centred difference
@@ -2136,6 +2139,7 @@ __device__ __forceinline__ int riemann_hlld_lean(const double *pl, const double 
   const double gamma = pp.gamma, g1 = pp.g1, gamf = pp.gamf;
   const double Bn = 0.5*(pl[Pm::B1] + pr[Pm::B1]);
   const double Bn2 = Bn*Bn;
+  const bool small_bn = dfabs(Bn) < T::small_bn;
   auto out = [&](double fD, double fE, double f0, double f1, double f2, double h0, double h1, double h2) {
     store_flux<DIM>(store, fD, fE, f0, f1, f2, h0, h1, h2);
   };
@@ -2162,6 +2166,7 @@ __device__ __forceinline__ int riemann_hlld_lean(const double *pl, const double 
     note_lambda(lam_max, am, ap);
     L.set(sl, am);
     Rt.set(sr, ap);
+    if (!small_bn && Bn2 < T::weak_Bn2*(sl.E + sr.E)) return kHlldDefer;
     // both fast waves on one side: the flux is that side's own, stored now so that its state
     // need not be kept (the solve below still decides whether HLLD is counted a success, and,
     // with both on the left, whether an inner wave lies on the right all the same)
@@ -2175,7 +2180,6 @@ __device__ __forceinline__ int riemann_hlld_lean(const double *pl, const double 
 
   // EstimateSolution(0) by anton2dzw (c2p_anton2dzw) on the HLL state, :208-218,543-555
   const double ida = rcp_normal(Rt.lam - L.lam);
-  const bool small_bn = dfabs(Bn) < T::small_bn;
   double p;
   {
     const double D = (Rt.D - L.D)*ida, E = (Rt.E - L.E)*ida, tau_ = E - D;
