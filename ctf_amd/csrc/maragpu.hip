@@ -1270,7 +1270,7 @@ __global__ __launch_bounds__(kBlock) void k_flux_weno_split_char_redo(const doub
  * ------------------------------------------------------------------------ */
 /* the operator's own limited slope (plm_minmod with its theta, :22-31) of a field's plane Pq
  * along S at zone z, zero outside the flat range [sx, T - sx) where the reference computes
- * slopes */
+ * slopes; the values are finite (a failed inversion fails the step whatever follows) */
 __device__ __forceinline__ double ctu_slope(const double *__restrict__ Pq, long T, long sxz, long z, long S, double theta)
 {
 #pragma clang fp contract(off)
@@ -1279,7 +1279,7 @@ __device__ __forceinline__ double ctu_slope(const double *__restrict__ Pq, long 
   const double a = theta * (u0 - ul);
   const double b = 0.5 * (ur - ul);
   const double c = theta * (ur - u0);
-  return minmod(a, b, c);
+  return minmod_finite(a, b, c);
 }
 
 /* the half-slope states, in the axis's frame, of face z | z+S along the axis: from P with its

@@ -919,16 +919,20 @@ __device__ __forceinline__ int cons_to_prim(const double *U, double *P, double g
 /* __plm_minmod of the slopes a (behind), b (centred, with the values' difference halved) and c
  * (ahead): the smallest of the three where all are positive, the largest where all are
  * negative, else zero. The reference's product of signs and the smallest magnitude is the
- * same value; as minima and maxima it takes 7 operations instead of 25, and 4 for what it
- * gives where b or c is not a number (zero with the value behind not a number, else not a
- * number), since a minimum takes its other operand there. The one difference left is an
- * infinite centre with infinite neighbours: zero here, not a number there, and the state is
- * not finite either way. */
-template <typename R> __device__ __forceinline__ R minmod(R a, R b, R c)
+ * same value; as minima and maxima it takes 7 operations instead of 25. */
+template <typename R> __device__ __forceinline__ R minmod_finite(R a, R b, R c)
 {
   const R lo = dfmin(dfmin(a, b), c), hi = dfmax(dfmax(a, b), c);
-  const R lim = dfmax(lo, R(0)) + dfmin(hi, R(0));
-  return __builtin_isunordered(b, c) ? R(0)*c : lim;
+  return dfmax(lo, R(0)) + dfmin(hi, R(0));
+}
+
+/* and, for 4 more operations, what the reference gives where b or c is not a number (zero with
+ * the value behind not a number, else not a number), since a minimum takes its other operand
+ * there. The one difference left is an infinite centre with infinite neighbours: zero here,
+ * not a number there, and the state is not finite either way. */
+template <typename R> __device__ __forceinline__ R minmod(R a, R b, R c)
+{
+  return __builtin_isunordered(b, c) ? R(0)*c : minmod_finite(a, b, c);
 }
 
 /* __plm, weno.c:85-96: v points at the centre zone. HAND_ON: for sweeps that hand a state with
@@ -940,8 +944,7 @@ template <typename R, bool HAND_ON = false> __device__ __forceinline__ R plm(R v
   const R b = R(0.5) * (vp - vm);
   const R c = theta * (vp - v0);
   if constexpr (HAND_ON) {
-    const R lo = dfmin(dfmin(a, b), c), hi = dfmax(dfmax(a, b), c);
-    return (v0 + R(0)*b) + sg*R(0.5)*(dfmax(lo, R(0)) + dfmin(hi, R(0)));
+    return (v0 + R(0)*b) + sg*R(0.5)*minmod_finite(a, b, c);
   }
   return v0 + sg*R(0.5)*minmod(a, b, c);
 }
