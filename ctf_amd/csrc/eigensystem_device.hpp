@@ -662,6 +662,15 @@ __device__ __forceinline__ bool simple_projection(FastLds &lds, const double *P,
     const double s = (lane & 1) ? -e : e;
     const double alfven = (bi + s*W*vn)*rcp(b0 + s*W);
     const double ca2 = b2*rcp(rhoh + b2);
+    {
+      // clusters seen without the magnetosonic speeds: 0, vn and the Alfven speeds, and, in a
+      // weak field, the slow speeds, which lie within (ca^2 / 2 cs^2) |alfven - vn| of the
+      // Alfven ones. With no or a weak field (B below 3e-3 at rho = p = 1) that is every
+      // interface, and the rest of this would be for nothing.
+      const double d = fabs(alfven - vn);
+      const double g = fmin(fmin(d, fabs(vn)), fmin(fabs(alfven), fabs(alfven - xchg<kDppXor1>(alfven))));
+      if (imax(!(g >= 1e-7) || !(d*ca2 >= 1e-7*cs2) || !valid ? 1 : 0)) return false;
+    }
     const double w2 = cs2 + ca2 - cs2*ca2;
     const double den = rcp(1.0 - V2*w2);
     const double rt = sqrt_lean(w2*om*(1.0 - V2*w2 - vn*vn*(1.0 - w2)));

@@ -1186,7 +1186,9 @@ __device__ __forceinline__ void char_flux(const double *__restrict__ Uw, const R
  * At 48x56x44, FP64: 103 us a sweep (2 280 VALU instructions per wave of 8 interfaces, 76 % of the
  * time their issue at 256^3, 34 KB of LDS a block, 4 waves per SIMD), and 4-60 us for the queue;
  * 512 us with the general eigensystem for every interface (10 100 instructions, 235 VGPRs, 2
- * waves). */
+ * waves). Without a field every interface has a cluster and goes on to it: 38 ms a step at 96^3
+ * (30 ms with the general eigensystem at once), 67 ms where the short way first formed all
+ * eigenvalues and the redo ran one wave per SIMD. */
 template <typename R>
 __global__ __launch_bounds__(kBlock, 3) void k_flux_weno_split_char(const double *__restrict__ Uw,
                                                                     const double *__restrict__ P,
@@ -1230,12 +1232,12 @@ __global__ __launch_bounds__(kBlock, 3) void k_flux_weno_split_char(const double
 /* The queued interfaces, with the general eigensystem (eig::g8::rmhd_eigensystem; the identity
  * where it is rejected); a loop over the queue's count, eight lanes to an interface. */
 template <typename R>
-__global__ __launch_bounds__(kBlock) void k_flux_weno_split_char_redo(const double *__restrict__ Uw,
-                                                                      const double *__restrict__ P,
-                                                                      const R *__restrict__ FZ,
-                                                                      const R *__restrict__ AZ, R *__restrict__ Fout,
-                                                                      GridDesc g, int axis, PhysParams pp, DevStats *st,
-                                                                      RedoQueue rq)
+__global__ __launch_bounds__(kBlock, 2) void k_flux_weno_split_char_redo(const double *__restrict__ Uw,
+                                                                         const double *__restrict__ P,
+                                                                         const R *__restrict__ FZ,
+                                                                         const R *__restrict__ AZ, R *__restrict__ Fout,
+                                                                         GridDesc g, int axis, PhysParams pp,
+                                                                         DevStats *st, RedoQueue rq)
 {
   __shared__ __align__(16) double split[kBlock / 8][2 * 48 + 4];     // the pad staggers the groups' banks
   const long T = g.T, S = axis_stride(g, axis);
