@@ -638,6 +638,18 @@ __device__ __forceinline__ bool elim4_step(double (&a)[4][4], double (&rhs)[4], 
   return best > 0.0;
 }
 
+/* Whether the field is so weak that the slow speeds are within 1e-7 of the Alfven ones, which lie
+ * within |Bn| / sqrt(rho h) of vn: they differ by at most (ca^2 / 2 cs^2) of that, ca^2 below
+ * B^2 / rho h. simple_projection returns false there, at the end of its search for the
+ * eigenvalues. */
+__device__ __forceinline__ bool slow_cluster(const double *P, double gamma)
+{
+  const double B2 = P[Bx]*P[Bx] + P[By]*P[By] + P[Bz]*P[Bz];
+  const double gp = opaque(gamma*P[pre]), rhoh = opaque(P[rho] + gp*rcp(gamma - 1.0));
+  const double a = P[Bx]*B2;
+  return B2 < 1e-4*rhoh && a*a < 1e-14*(gp*gp)*rhoh;
+}
+
 /* Lrow, Rrow (row `lane` of L and R) of the state P in the axis's frame, or false where
  * rmhd_eigensystem has to be asked. All lanes of the wave call it together; `valid` = false
  * for a group without an interface. */
@@ -662,15 +674,6 @@ __device__ __forceinline__ bool simple_projection(FastLds &lds, const double *P,
     const double s = (lane & 1) ? -e : e;
     const double alfven = (bi + s*W*vn)*rcp(b0 + s*W);
     const double ca2 = b2*rcp(rhoh + b2);
-    {
-      // clusters seen without the magnetosonic speeds: 0, vn and the Alfven speeds, and, in a
-      // weak field, the slow speeds, which lie within (ca^2 / 2 cs^2) |alfven - vn| of the
-      // Alfven ones. With no or a weak field (B below 3e-3 at rho = p = 1) that is every
-      // interface, and the rest of this would be for nothing.
-      const double d = fabs(alfven - vn);
-      const double g = fmin(fmin(d, fabs(vn)), fmin(fabs(alfven), fabs(alfven - xchg<kDppXor1>(alfven))));
-      if (imax(!(g >= 1e-7) || !(d*ca2 >= 1e-7*cs2) || !valid ? 1 : 0)) return false;
-    }
     const double w2 = cs2 + ca2 - cs2*ca2;
     const double den = rcp(1.0 - V2*w2);
     const double rt = sqrt_lean(w2*om*(1.0 - V2*w2 - vn*vn*(1.0 - w2)));

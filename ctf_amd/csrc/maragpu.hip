@@ -100,11 +100,11 @@ struct DevStats {
  * outside the common path of the lean sweep, k_flux_fast), or to the general eigensystem
  * (weno-split, eigen = RMHD).
  * A set is eight lists, one per XCD: an atomic on a counter takes 8 ns when all waves of the
- * chip meet on it (128^3, every interface handed on: 800 us of 1315 in k_flux_fast). Up to
+ * chip meet on it (128^3, every interface handed on: 850 us of 1315 in k_flux_fast). Up to
  * three sets: the sweeps' own, and what the bulk kernels leave of it; or, for the
  * characteristic sweeps, one per axis. */
 constexpr int kQueueLists = 8, kQueueSets = 3;
-constexpr int kCountStride = 32;         // counters 128 B apart
+constexpr int kCountStride = 16;         // counters 64 B apart (4 B apart: no gain, 1283 us)
 struct RedoQueue {
   unsigned int *count;     // device counters; cleared before the sweeps (clear_queue)
   unsigned int cap;        // slots of a list
@@ -1219,7 +1219,8 @@ __global__ __launch_bounds__(kBlock, 3) void k_flux_weno_split_char(const double
       const double *v = P + axis_plane(q, axis) * T + z;
       Ph[q] = 0.5 * (v[0] + v[S]);
     }
-    done = eig::g8::simple_projection(lds[threadIdx.x >> 6], Ph, lane, valid, pp.gamma, Lrow, Rrow);
+    done = __ballot(valid && !eig::g8::slow_cluster(Ph, pp.gamma)) != 0ull &&
+           eig::g8::simple_projection(lds[threadIdx.x >> 6], Ph, lane, valid, pp.gamma, Lrow, Rrow);
   }
   if (done && valid) {
     const int base = (int)((threadIdx.x & 63) >> 3) * eig::g8::kGroupPad;
