@@ -87,8 +87,8 @@ struct DevStats {
   unsigned long long hlld_newton_iters;
   unsigned long long mlp_guesses;
   unsigned long long mlp_fallbacks;
-  unsigned long long redo;             // mixed form: interfaces recomputed in FP64
-  unsigned long long redo_overflow;    // ... that did not fit the queue (FP32 HLLC kept)
+  unsigned long long redo;             // interfaces handed on and redone (RedoQueue)
+  unsigned long long redo_overflow;    // ... that did not fit the queue: their fluxes are stale
   unsigned long long stage_failed[6];  // failed zones per c2p pass (ghost images included)
   unsigned long long stage_reset[6];   // zones reset by the emergency repair per pass (weno-split)
   unsigned long long eig_identity;     // weno-split interfaces whose eigensystem was rejected
@@ -120,16 +120,24 @@ struct RedoQueue {
  * shorter one fill the redo kernel's grid once. */
 constexpr unsigned kShortQueue = 4096;
 
-/* A set's entries counted through its lists. The counts are uniform: scalar loads. */
+/* A set's entries counted through its lists, and how many did not fit (none: a list has a slot
+ * for every interface of its blocks). The counts are uniform: scalar loads. */
 struct QueueView {
-  unsigned n = 0, first[kQueueLists];
+  unsigned n = 0, over = 0, first[kQueueLists];
   __device__ __forceinline__ explicit QueueView(const RedoQueue &rq)
   {
 #pragma unroll
     for (int l = 0; l < kQueueLists; ++l) {
+      const unsigned c = rq.count[l * kCountStride], taken = min(c, rq.cap);
       first[l] = n;
-      n += min(rq.count[l * kCountStride], rq.cap);
+      n += taken;
+      over += c - taken;
     }
+  }
+  /* one thread of the launch that empties the set calls this */
+  __device__ __forceinline__ void count_overflow(DevStats *st) const
+  {
+    if (over) atomicAdd(&st->redo_overflow, (unsigned long long)over);
   }
   __device__ __forceinline__ void entry(const RedoQueue &rq, unsigned k, int &axis, long &z) const
   {
@@ -896,9 +904,12 @@ __global__ __launch_bounds__(kBlock) void k_flux_redo(const double *__restrict__
                                                       unsigned int nparts)
 {
   QueueView view(rq);
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (first) view.count_overflow(st);
   if (SOLVER == RIEMANN_HLLD && sizeof(FT) == 8 && view.n > kShortQueue) {    // k_flux_bulk's rest
     rq = rq.set(1);
     view = QueueView(rq);
+    if (first) view.count_overflow(st);
   }
   double lam_out = 0.0;
   unsigned long long cnt[7] = {0, 0, 0, 0, 0, 0, 0};
@@ -1246,6 +1257,10 @@ __global__ __launch_bounds__(kBlock, 2) void k_flux_weno_split_char_redo(const d
   double *const Fp = split[threadIdx.x >> 3];
   rq = rq.set(axis);
   const QueueView view(rq);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    view.count_overflow(st);
+    if (view.n) atomicAdd(&st->redo, (unsigned long long)view.n);
+  }
   for (unsigned e = (blockIdx.x * blockDim.x + threadIdx.x) >> 3; e < view.n; e += (gridDim.x * blockDim.x) >> 3) {
     long z;
     int a;
@@ -1368,9 +1383,12 @@ __global__ __launch_bounds__(kBlock) void k_ctu_faces_redo(const double *__restr
                                                            unsigned int nparts)
 {
   QueueView view(rq);
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (first) view.count_overflow(st);
   if (SOLVER == RIEMANN_HLLD && view.n > kShortQueue) {    // k_ctu_faces_bulk's rest
     rq = rq.set(1);
     view = QueueView(rq);
+    if (first) view.count_overflow(st);
   }
   const long T = g.T;
   double lam_out = 0.0;

@@ -100,8 +100,11 @@ typedef struct maragpu_stats {
   int64_t hlld_newton_iterations; /* p* Newton iterations in HLLD */
   int64_t mlp_guesses;          /* learned c2p: zones started from the network's guess */
   int64_t mlp_fallbacks;        /* learned c2p: zones that fell back to the plain cascade */
-  int64_t fp64_redo;            /* mixed form: interfaces whose FP32 HLLD failed, redone in FP64 */
-  int64_t fp64_redo_overflow;   /* ... beyond the redo queue (FP32 HLLC flux kept) */
+  int64_t fp64_redo;            /* interfaces that left a sweep's common path: to the full FP64 solver
+                                   (mixed: those whose FP32 HLLD failed), or with weno-split,
+                                   eigen = RMHD, to the general eigensystem */
+  int64_t fp64_redo_overflow;   /* ... beyond the queue, which holds them all: 0, or the step's
+                                   fluxes are wrong */
   int64_t eig_identity;         /* weno-split, eigen = RMHD: interfaces projected with the
                                    identity because the eigensystem was rejected */
   double device_ms;             /* device time of the step */

@@ -318,3 +318,50 @@ def test_long_queue(gpu, oracle_lib, N, B, godunov, extrap):
         assert st.hlld_success + st.hlld_failure == ok0 + fail0
         assert abs(st.hlld_success - ok0) <= ok_t
     assert (L1(ctx.download()) <= tol).all()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("B0,dB,share", [
+    ((0.0, 0.0, 0.0), 0.0, (1.0, 1.0)),        # no field: every spectrum has a cluster
+    ((1e-4, 2e-4, 1e-4), 3e-5, (1.0, 1.0)),    # the slow speeds within 1e-7 of the Alfven ones
+    ((0.5, 0.6, 0.7), 0.3, (0.0, 0.05)),       # simple spectra but for a few
+])
+def test_characteristic_interfaces_handed_on(gpu, B0, dB, share, precision):
+    """Which interfaces of the characteristic sweep go to the general eigensystem: all of them
+    with clusters everywhere, next to none otherwise (fp64_redo; one stage, so once per interface
+    of the three sweeps, whose transverse lines include the ghosts)."""
+    N = (19, 14, 22)
+    P = gpu.init_turbulence(N, Ng=3, seed=3, v_rms=0.3, v_kmax=4.0, four_velocity=False, B0=B0, dB_rms=dB, A_kmax=3.0)
+    ctx = gpu.Context(gpu.make_config(N=N, godunov="weno-split", eigen="rmhd", extrap="weno5", advance="single",
+                                      precision=precision))
+    ctx.upload(P)
+    e, st = ctx.advance(1e-3)
+    n = [k + 6 for k in N]
+    total = (N[0] + 1) * n[1] * n[2] + n[0] * (N[1] + 1) * n[2] + n[0] * n[1] * (N[2] + 1)
+    assert e == 0 and st.fp64_redo_overflow == 0
+    assert share[0] * total <= st.fp64_redo <= share[1] * total
+
+
+@pytest.mark.parametrize("N,extrap,riemann", [((17, 12, 26), "plm", "hllc"), ((9, 22, 13), "weno5", "hllc"),
+                                              ((12, 31, 10), "weno5", "hll")])
+def test_mixed_full_solver_sweeps(gpu, oracle_lib, N, extrap, riemann):
+    """The mixed form's HLL and HLLC sweeps (three axes in one launch, the full FP32 solver) on
+    grids whose axes differ, against the oracle: the bounds of the mixed form's other steps, L1
+    1e-5 and the fastest speed to 1e-4. The field is oblique: with a normal field that passes
+    zero HLLC multiplies round-off, and the oracle's own speeds move by 5e-5 under FP32
+    rounding of the state (here by 4e-8)."""
+    P0 = gpu.init_turbulence(N, v_rms=0.3, v_kmax=3.0, four_velocity=True, B0=(0.6, 0.6, 0.6), dB_rms=0.2,
+                             A_kmax=2.0, seed=11)
+    kw = dict(N=N, x1=tuple(n / max(N) for n in N), extrap=extrap, riemann=riemann, advance="rk2")
+    so = oracle_lib.solver(Setup(**kw))
+    ctx = gpu.Context(gpu.make_config(precision="mixed", **kw))
+    ctx.upload(P0)
+    Po, dt = P0.copy(), 0.1 / max(N)
+    for _ in range(3):
+        eo, sto = so.advance(Po, dt)
+        eg, stg = ctx.advance(dt)
+        assert eo == eg == 0
+        assert abs(stg.max_lambda - sto.max_lambda) <= 1e-4 * sto.max_lambda
+    it = (slice(3, -3),) * 3
+    a, b = ctx.download()[it], Po[it]
+    assert (np.abs(a - b).sum(axis=(0, 1, 2)) <= 1e-5 * np.abs(b).sum(axis=(0, 1, 2))).all()
