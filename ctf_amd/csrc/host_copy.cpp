@@ -119,8 +119,20 @@ struct Job {
   }
 };
 
+/* The device made current, and the caller's again afterwards: an event belongs to the device
+ * that is current when it is created */
+struct OnDevice {
+  int before = -1;
+  explicit OnDevice(int device)
+  {
+    if (hipGetDevice(&before) != hipSuccess || before == device || hipSetDevice(device) != hipSuccess) before = -1;
+  }
+  ~OnDevice() { if (before >= 0) (void)hipSetDevice(before); }
+};
+
 hipError_t copy(int device, hipStream_t stream, void *dev, void *host, size_t n, bool to_device)
 {
+  const OnDevice on(device);
   std::unique_lock<std::mutex> lock;
   Staging *st = device >= 0 && device < kDevices ? &g_staging[device] : nullptr;
   if (st && n >= kSmall) lock = std::unique_lock<std::mutex>(st->busy, std::try_to_lock);

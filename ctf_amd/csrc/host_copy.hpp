@@ -12,7 +12,7 @@ void staging_retain(int device);
 void staging_release(int device);
 
 /* n bytes from host to dev, or from dev to host, in order with the work already on `stream`
- * (of `device`, which is current and has a context). copy_to_host returns with the bytes in
+ * (of `device`, which has a context; another device may be current). copy_to_host returns with the bytes in
  * place; after copy_to_device the caller synchronises the stream before the host buffer
  * changes hands, as after hipMemcpyAsync. */
 hipError_t copy_to_device(int device, hipStream_t stream, void *dev, const void *host, size_t n);

@@ -1,0 +1,40 @@
+"""The staged copies between host and device (host_copy.cpp) on a stand-in for the HIP runtime
+(tests/host/runtime), for what a machine with one GPU cannot show: a caller whose current
+device is another one, a runtime call that fails half way, and which way a copy takes."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+MB = 1 << 20
+
+
+@pytest.fixture(scope="module")
+def run_copy(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("host_copy") / "host_copy.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-w", "-shared", "-fPIC", "-I",
+                    os.path.join(ROOT, "tests", "host", "runtime"), "-o", out,
+                    os.path.join(ROOT, "tests", "host", "host_copy.cpp")], check=True)
+    lib = ctypes.CDLL(out)
+
+    def run(n, to_device, device=0, current=0, pinned=False, fail_record=-1):
+        src = np.random.default_rng(n).integers(0, 255, n, dtype=np.uint8)
+        dst = np.zeros_like(src)
+        host, dev = (src, dst) if to_device else (dst, src)
+        res = (ctypes.c_int * 4)()
+        lib.run_copy(device, current, int(to_device), host.ctypes.data_as(ctypes.c_void_p),
+                     dev.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(n), int(pinned), fail_record, res)
+        return dict(error=res[0], copies=res[1], in_flight=res[2], device=res[3], equal=np.array_equal(src, dst))
+    return run
+
+
+@pytest.mark.parametrize("to_device", [True, False])
+def test_from_another_current_device(run_copy, to_device):
+    """A context's copies work from a thread whose current device is another one, and leave it
+    that way."""
+    r = run_copy(48 * MB + 13, to_device, device=1, current=0)
+    assert r["error"] == 0 and r["equal"] and r["in_flight"] == 0
+    assert r["copies"] > 1 and r["device"] == 0
