@@ -85,9 +85,12 @@ struct Job {
   }
   bool send(Slot &s, size_t off, size_t len)
   {
-    return ok(to_device ? hipMemcpyAsync(dev + off, s.p, len, hipMemcpyHostToDevice, stream)
-                        : hipMemcpyAsync(s.p, dev + off, len, hipMemcpyDeviceToHost, stream)) &&
-           ok(hipEventRecord(s.done, stream));
+    if (!ok(to_device ? hipMemcpyAsync(dev + off, s.p, len, hipMemcpyHostToDevice, stream)
+                      : hipMemcpyAsync(s.p, dev + off, len, hipMemcpyDeviceToHost, stream)))
+      return false;
+    if (ok(hipEventRecord(s.done, stream))) return true;
+    (void)hipStreamSynchronize(stream);       // the slot is in use and has no event to wait for
+    return false;
   }
 
   /* one thread's share, with the slots s[0], s[1]; both are idle again on return */

@@ -38,3 +38,14 @@ def test_from_another_current_device(run_copy, to_device):
     r = run_copy(48 * MB + 13, to_device, device=1, current=0)
     assert r["error"] == 0 and r["equal"] and r["in_flight"] == 0
     assert r["copies"] > 1 and r["device"] == 0
+
+
+@pytest.mark.parametrize("n,to_device,nth", [
+    (9 * MB, False, 0), (9 * MB, False, 2), (9 * MB, False, 4),      # one thread, five chunks
+    (48 * MB, False, 5), (48 * MB, True, 0), (48 * MB, True, 23),    # several threads
+])
+def test_failed_record_leaves_no_copy_in_flight(run_copy, n, to_device, nth):
+    """A copy that the runtime took but whose event it did not is waited for before the slot is
+    free for the next caller."""
+    r = run_copy(n, to_device, fail_record=nth)
+    assert r["error"] != 0 and r["in_flight"] == 0
