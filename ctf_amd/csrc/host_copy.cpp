@@ -1,11 +1,15 @@
-/* Copies between pageable host buffers and the device.
+/* Copies between host buffers and the device.
  *
- * The runtime's own copy of a pageable buffer is one thread's: 28 GB/s to the device, 17 GB/s
- * back, and 10.5 GB/s back into a freshly allocated array, whose pages that thread also has
- * to fault in. A snapshot of a 256^3 grid (1.15 GB) so cost 40 ms in and 110 ms out, four
- * double-precision steps. Here several threads each take chunks of the buffer in turn, copy
- * them to or from two pinned slots of their own and leave the transfer of one slot to run
- * while they copy the other: 39 GB/s each way, in a new array too (256^3: 29 and 30 ms).
+ * The runtime's own copy of a pageable buffer is one thread's: 36 GB/s to the device up to
+ * 30 MB and 31 above, 18 GB/s back, and 10.5 GB/s back into a freshly allocated array, whose
+ * pages that thread also has to fault in. A snapshot of a 256^3 grid (1.15 GB) so cost 40 ms in
+ * and 110 ms out, four double-precision steps. Here several threads each take chunks of the
+ * buffer in turn, copy them to or from two pinned slots of their own and leave the transfer of
+ * one slot to run while they copy the other: 39 GB/s each way, in a new array too (256^3: 29
+ * and 30 ms). The rule, by what was measured on both sides (GB/s, runtime | staged):
+ *   to the device    2 MB 23 | 17, 8 MB 33 | 29, 30 MB 36 | 35, 41 MB 32 | 36, 154 MB 31 | 38
+ *   to the host      2 MB 15 | 18, 8 MB 18 | 24, 30 MB 18 | 37, 41 MB 10.5 | 30, 154 MB 10.6 | 37
+ *   pinned memory    37 (2 MB) to 56 (154 MB) by the runtime, which transfers it as it is
  *
  * The staging is one per device, at most 8 threads x 2 slots x 2 MB, slots allocated when a
  * copy first needs them and freed with the last context. One copy at a time uses it: a
@@ -24,8 +28,9 @@ namespace maragpu_host {
 namespace {
 
 constexpr size_t kChunk = size_t(2) << 20;      // a slot
-// below this, the runtime's copy: staging 1.1 MB a step made a march through the verbs 12 % slower
-constexpr size_t kSmall = size_t(2) << 20;
+// below these, the runtime's copy (staging 1.1 MB each way a step made a march through the verbs
+// 12 % slower)
+constexpr size_t kSmallToDevice = size_t(32) << 20, kSmallToHost = size_t(2) << 20;
 constexpr size_t kPerThread = size_t(8) << 20;  // bytes that make a further thread worth its start
 constexpr int kThreads = 8;
 constexpr int kDevices = 64;
@@ -122,6 +127,15 @@ struct Job {
   }
 };
 
+/* Memory that the device reads and writes as it is */
+bool pinned(const void *p)
+{
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeHost;
+  (void)hipGetLastError();                    // a pointer the runtime does not know
+  return false;
+}
+
 /* The device made current, and the caller's again afterwards: an event belongs to the device
  * that is current when it is created */
 struct OnDevice {
@@ -138,7 +152,8 @@ hipError_t copy(int device, hipStream_t stream, void *dev, void *host, size_t n,
   const OnDevice on(device);
   std::unique_lock<std::mutex> lock;
   Staging *st = device >= 0 && device < kDevices ? &g_staging[device] : nullptr;
-  if (st && n >= kSmall) lock = std::unique_lock<std::mutex>(st->busy, std::try_to_lock);
+  if (st && n >= (to_device ? kSmallToDevice : kSmallToHost) && !pinned(host))
+    lock = std::unique_lock<std::mutex>(st->busy, std::try_to_lock);
   if (!lock.owns_lock() || !st->slot[0].make() || !st->slot[1].make()) {
     if (to_device) return hipMemcpyAsync(dev, host, n, hipMemcpyHostToDevice, stream);
     const hipError_t e = hipMemcpyAsync(host, dev, n, hipMemcpyDeviceToHost, stream);

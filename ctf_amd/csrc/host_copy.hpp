@@ -1,4 +1,5 @@
-/* Copies between pageable host buffers and the device through pinned staging (host_copy.cpp). */
+/* Copies between host buffers and the device, large pageable ones through pinned staging
+ * (host_copy.cpp). */
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -49,3 +49,17 @@ def test_failed_record_leaves_no_copy_in_flight(run_copy, n, to_device, nth):
     free for the next caller."""
     r = run_copy(n, to_device, fail_record=nth)
     assert r["error"] != 0 and r["in_flight"] == 0
+
+
+@pytest.mark.parametrize("n,to_device,pinned,staged", [
+    (8 * MB, True, False, False),      # the runtime's own upload is the faster one up to here
+    (48 * MB, True, False, True),
+    (1 * MB, False, False, False),
+    (8 * MB, False, False, True),      # its download is not
+    (48 * MB, True, True, False),      # pinned memory needs no staging
+    (48 * MB, False, True, False),
+])
+def test_which_copies_are_staged(run_copy, n, to_device, pinned, staged):
+    r = run_copy(n, to_device, pinned=pinned)
+    assert r["error"] == 0 and r["equal"] and r["in_flight"] == 0
+    assert (r["copies"] > 1) == staged
