@@ -1,13 +1,14 @@
 /* Copies between host buffers and the device.
  *
- * The runtime's own copy of a pageable buffer is one thread's: 36 GB/s to the device up to
- * 30 MB and 31 above, 18 GB/s back, and 10.5 GB/s back into a freshly allocated array, whose
+ * The runtime's own copy of a pageable buffer is one thread's: 28-31 GB/s to the device (36 from
+ * a buffer used just before), 18 GB/s back, and 10.5 GB/s back into a freshly allocated array, whose
  * pages that thread also has to fault in. A snapshot of a 256^3 grid (1.15 GB) so cost 40 ms in
  * and 110 ms out, four double-precision steps. Here several threads each take chunks of the
  * buffer in turn, copy them to or from two pinned slots of their own and leave the transfer of
  * one slot to run while they copy the other: 39 GB/s each way, in a new array too (256^3: 29
- * and 30 ms). The rule, by what was measured on both sides (GB/s, runtime | staged):
- *   to the device    2 MB 23 | 17, 8 MB 33 | 29, 30 MB 36 | 35, 41 MB 32 | 36, 154 MB 31 | 38
+ * and 30 ms). The rule, by what was measured on both sides (GB/s, runtime | staged; six buffers in turn to the device,
+ * a new array each time back):
+ *   to the device    2 MB 22 | 15, 8 MB 26 | 22, 15 MB 28 | 26, 22 MB 28 | 31, 154 MB 31 | 38
  *   to the host      2 MB 15 | 18, 8 MB 18 | 24, 30 MB 18 | 37, 41 MB 10.5 | 30, 154 MB 10.6 | 37
  *   pinned memory    37 (2 MB) to 56 (154 MB) by the runtime, which transfers it as it is
  *
@@ -30,7 +31,7 @@ namespace {
 constexpr size_t kChunk = size_t(2) << 20;      // a slot
 // below these, the runtime's copy (staging 1.1 MB each way a step made a march through the verbs
 // 12 % slower)
-constexpr size_t kSmallToDevice = size_t(32) << 20, kSmallToHost = size_t(2) << 20;
+constexpr size_t kSmallToDevice = size_t(20) << 20, kSmallToHost = size_t(2) << 20;
 constexpr size_t kPerThread = size_t(8) << 20;  // bytes that make a further thread worth its start
 constexpr int kThreads = 8;
 constexpr int kDevices = 64;

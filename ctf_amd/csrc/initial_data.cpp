@@ -15,6 +15,8 @@
  *             round-off); scaled to an rms of dB_rms.
  * The sums are evaluated as three partial 1-D transforms (pruned to the selected modes).
  */
+#include <omp.h>
+
 #include <cmath>
 #include <complex>
 #include <cstdint>
@@ -52,6 +54,16 @@ struct Mode {
   cplx c[3];
 };
 
+/* For a last parallel loop: its team goes to sleep at once. By default the team waits actively for
+ * 200 ms, and a caller that copies or converts what was made here shares the cores with it (a
+ * mixed-precision march of 128^3 on a state just made: 52-75 ms, 35 ms so). The setting is the
+ * calling thread's and put back. */
+struct SleepingTeam {
+  const int before = kmp_get_blocktime();
+  SleepingTeam() { kmp_set_blocktime(0); }
+  ~SleepingTeam() { kmp_set_blocktime(before); }
+};
+
 /* f_c(i,j,k) = sum over modes m and their conjugates of c_m e^{i t.(idx + 1/2)} */
 void synthesize(const std::vector<Mode> &modes, int K, const int *N, std::vector<double> *out)
 {
@@ -65,53 +77,52 @@ void synthesize(const std::vector<Mode> &modes, int K, const int *N, std::vector
         E[d][(size_t)(m + K) * N[d] + i] = cplx(std::cos(ph), std::sin(ph));
       }
   }
+  // per component, the dense coefficient cube with Hermitian symmetry and the partial sums over
+  // the first and second axis, T1[nx][ny][k] and T2[nx][j][k]
+  std::vector<cplx> C[3], T1[3], T2[3];
   for (int comp = 0; comp < 3; ++comp) {
-    // dense coefficient cube with Hermitian symmetry
-    std::vector<cplx> C((size_t)W * W * W, cplx(0.0, 0.0));
+    C[comp].assign((size_t)W * W * W, cplx(0.0, 0.0));
     for (const Mode &md : modes) {
       const size_t a = ((size_t)(md.n[0] + K) * W + (md.n[1] + K)) * W + (md.n[2] + K);
       const size_t b = ((size_t)(-md.n[0] + K) * W + (-md.n[1] + K)) * W + (-md.n[2] + K);
-      C[a] += md.c[comp];
-      C[b] += std::conj(md.c[comp]);
+      C[comp][a] += md.c[comp];
+      C[comp][b] += std::conj(md.c[comp]);
     }
-    // T1[nx][ny][k]
-    std::vector<cplx> T1((size_t)W * W * N[2]);
+    T1[comp].resize((size_t)W * W * N[2]);
+    T2[comp].resize((size_t)W * N[1] * N[2]);
+    out[comp].assign((size_t)N[0] * N[1] * N[2], 0.0);
+  }
+  // T2's plane a takes T1's rows of the same a
 #pragma omp parallel for schedule(static)
-    for (int ab = 0; ab < W * W; ++ab) {
+  for (int row = 0; row < 3 * W; ++row) {
+    const int comp = row / W, a = row % W;
+    for (int ab = a * W; ab < (a + 1) * W; ++ab)
       for (int k = 0; k < N[2]; ++k) {
         cplx s(0.0, 0.0);
-        for (int c = 0; c < W; ++c) s += C[(size_t)ab * W + c] * E[2][(size_t)c * N[2] + k];
-        T1[(size_t)ab * N[2] + k] = s;
+        for (int c = 0; c < W; ++c) s += C[comp][(size_t)ab * W + c] * E[2][(size_t)c * N[2] + k];
+        T1[comp][(size_t)ab * N[2] + k] = s;
       }
-    }
-    // T2[nx][j][k]
-    std::vector<cplx> T2((size_t)W * N[1] * N[2]);
+    for (int j = 0; j < N[1]; ++j)
+      for (int k = 0; k < N[2]; ++k) {
+        cplx s(0.0, 0.0);
+        for (int b = 0; b < W; ++b)
+          s += T1[comp][((size_t)a * W + b) * N[2] + k] * E[1][(size_t)b * N[1] + j];
+        T2[comp][((size_t)a * N[1] + j) * N[2] + k] = s;
+      }
+  }
+  const SleepingTeam last;
 #pragma omp parallel for schedule(static)
-    for (int a = 0; a < W; ++a) {
-      for (int j = 0; j < N[1]; ++j) {
-        for (int k = 0; k < N[2]; ++k) {
-          cplx s(0.0, 0.0);
-          for (int b = 0; b < W; ++b)
-            s += T1[((size_t)a * W + b) * N[2] + k] * E[1][(size_t)b * N[1] + j];
-          T2[((size_t)a * N[1] + j) * N[2] + k] = s;
+  for (int row = 0; row < 3 * N[0]; ++row) {
+    const int comp = row / N[0], i = row % N[0];
+    for (int j = 0; j < N[1]; ++j)
+      for (int k = 0; k < N[2]; ++k) {
+        double s = 0.0;
+        for (int a = 0; a < W; ++a) {
+          const cplx t = T2[comp][((size_t)a * N[1] + j) * N[2] + k] * E[0][(size_t)a * N[0] + i];
+          s += t.real();
         }
+        out[comp][((size_t)i * N[1] + j) * N[2] + k] = s;
       }
-    }
-    std::vector<double> &f = out[comp];
-    f.assign((size_t)N[0] * N[1] * N[2], 0.0);
-#pragma omp parallel for schedule(static)
-    for (int i = 0; i < N[0]; ++i) {
-      for (int j = 0; j < N[1]; ++j) {
-        for (int k = 0; k < N[2]; ++k) {
-          double s = 0.0;
-          for (int a = 0; a < W; ++a) {
-            const cplx t = T2[((size_t)a * N[1] + j) * N[2] + k] * E[0][(size_t)a * N[0] + i];
-            s += t.real();
-          }
-          f[((size_t)i * N[1] + j) * N[2] + k] = s;
-        }
-      }
-    }
   }
 }
 
