@@ -613,7 +613,7 @@ __device__ __forceinline__ int interface_flux_fast(const double *__restrict__ P,
   R ql[8], qr[8];
   reconstruct_states<R, sizeof(R) == 8, true>(P, T, S, axis, z, recon, pp, ql, qr);
   auto store = [&](int q, R f) { Fout[axis_plane(q, axis) * T + z] = f; };
-  if constexpr (sizeof(R) == 8 && SOLVER == RIEMANN_HLLD) return riemann_hlld_lean<1>(ql, qr, pp, lam, fc, store);
+  if constexpr (sizeof(R) == 8 && SOLVER == RIEMANN_HLLD) return riemann_hlld_lean(ql, qr, pp, lam, fc, store);
   else if constexpr (sizeof(R) == 8) return riemann_hllx_lean<SOLVER>(ql, qr, pp, lam, store);
   else {
     static_assert(SOLVER == RIEMANN_HLLD, "FP32: the HLLD sweep");
@@ -1345,7 +1345,7 @@ void k_ctu_faces_fast(const double *__restrict__ P, FaceStates Ps, FluxPlanes<do
       double lam = 0.0;
       FluxCounters fc = {0, 0, 0, 0};
       auto store = [&](int q, double f) { F[axis_plane(q, axis) * T + z] = f; };
-      if constexpr (SOLVER == RIEMANN_HLLD) defer = riemann_hlld_lean<1>(pl, pr, pp, lam, fc, store) != 0;
+      if constexpr (SOLVER == RIEMANN_HLLD) defer = riemann_hlld_lean(pl, pr, pp, lam, fc, store) != 0;
       else defer = riemann_hllx_lean<SOLVER>(pl, pr, pp, lam, store) != 0;
       if (!defer && SOLVER == RIEMANN_HLLD) {
         cnt[1] = 1;

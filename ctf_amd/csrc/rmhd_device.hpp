@@ -1599,8 +1599,10 @@ struct FluxCounters {
  * GROUP = true runs the attempt ladder of one interface on 16 lanes (a row of the wave) that
  * hold the same states: each quad takes one attempt (the fourth repeats the third), each lane
  * of a quad one of the three residual evaluations of its Newton steps. The first attempt in
- * the reference's order that succeeded supplies the flux, so the result is the serial one; f
- * and the counters are returned in the lane for which `lead` is set. The ladder is a serial
+ * the reference's order that succeeded supplies the flux, as in the serial ladder, though not
+ * bit for bit: the two are compiled apart, and at an interface where an attempt ends by
+ * round-off they may take different ones (the mixed form's strong fields: 2e-7 of a march, 3e-5
+ * at a zone). f and the counters are returned in the lane for which `lead` is set. The ladder is a serial
  * chain (up to 3 x 16 x 3 evaluations of some 250 dependent instructions, 50-70 us), and a
  * handful of interfaces that need it would hold the stage that long. */
 constexpr int kHlldDefer = 100;   // common path: the interface needs the full solver
@@ -1818,9 +1820,10 @@ __device__ __forceinline__ int riemann_hlld(const R *pl, const R *pr, R *f, R ga
  * failed nested c2p, a Newton solve that does not settle, a rejected fan) returns
  * kHlldDefer, and the caller hands the interface to the full FP64 solver.
  *
- * What it computes is the reference's flux to round-off; what it leaves out are operations
- * whose result is already known, since the sweep is bound by instruction issue (its HBM
- * traffic is the algorithmic minimum). Against the full solver's common branches in the same
+ * What it keeps has the full solver's flux to round-off (of 6 million random interfaces none
+ * differs by more than the full solver under 1-ulp noise on its input); what it leaves out are
+ * operations whose result is already known, since the sweep is bound by instruction issue (its
+ * HBM traffic is the algorithmic minimum). Against the full solver's common branches in the same
  * kernel: 2 600-3 200 VALU instructions per wave of interfaces where there were 5 300-5 800,
  * 166 VGPRs where there were 213 (3 waves per SIMD, not 2), and at 256^3 WENO5 1.48-1.55 ms
  * a sweep where it took 3.2-3.7 (82 % of the issue rate, from 67 %).
@@ -1838,8 +1841,10 @@ __device__ __forceinline__ int riemann_hlld(const R *pl, const R *pr, R *f, R ga
  *   - The derivative is a one-sided difference from the residual at hand, and the last
  *     Newton step (from a residual within the tolerance) takes the derivative of the step
  *     before it, if the residual fell by 20 times (so the derivative changed by less than a
- *     tenth) and the step is below 1e-11 of p (so what a tenth of it changes is round-off):
- *     four evaluations of the fan per interface where centred differences take seven.
+ *     tenth) and the step is below 1e-11 of p. With a derivative of its own for that step too
+ *     the flux is the same to 3e-15 in turbulence and 9e-14 at jumps of 0.3: the residual at
+ *     hand is by then squared, so the step is far below those bounds. Four evaluations of the
+ *     fan per interface where centred differences take seven.
  * ------------------------------------------------------------------------- */
 /* One side of an interface in the x-normal frame: D, E = tau + D, S, the fluxes and the
  * fast speeds (Mara/rmhd.cpp:133-265). False for a state that prim_to_cons would or might
@@ -1964,19 +1969,18 @@ __device__ __forceinline__ double zone_flux_lean(const double *u, const double *
 }
 
 /* The flux of a lean solver, (D, E = tau + D, S, B) in the axis's frame, to `store` */
-template <int DIM, typename Store>
+template <typename Store>
 __device__ __forceinline__ void store_flux(Store &store, double fD, double fE, double f0, double f1, double f2, double g0,
                                            double g1, double g2)
 {
-  using Pm = Perm<DIM>;
   store((int)ddd, fD);
   store((int)tau, fE - fD);
-  store(Pm::S1, f0);
-  store(Pm::S2, f1);
-  store(Pm::S3, f2);
-  store(Pm::B1, g0);
-  store(Pm::B2, g1);
-  store(Pm::B3, g2);
+  store((int)Sx, f0);
+  store((int)Sy, f1);
+  store((int)Sz, f2);
+  store((int)Bx, g0);
+  store((int)By, g1);
+  store((int)Bz, g2);
 }
 
 /* riemann_hll and riemann_hllc on FastSide states, in the frame whose first axis is the normal
@@ -2001,14 +2005,14 @@ __device__ __forceinline__ int riemann_hllx_lean(const double *pl, const double 
   note_lambda(lam_max, am, ap);
   if (0.0 <= am || !(0.0 <= ap)) {
     const bool left = 0.0 <= am;
-    store_flux<1>(store, left ? l.FD : r.FD, left ? l.S[0] : r.S[0], left ? l.FS[0] : r.FS[0], left ? l.FS[1] : r.FS[1],
+    store_flux(store, left ? l.FD : r.FD, left ? l.S[0] : r.S[0], left ? l.FS[0] : r.FS[0], left ? l.FS[1] : r.FS[1],
                   left ? l.FS[2] : r.FS[2], 0.0, left ? l.FB2 : r.FB2, left ? l.FB3 : r.FB3);
     return 0;
   }
   const double ida = rcp_normal(ap - am), amp = ap*am;
   auto hll = [&](double Fl, double Fr, double Ul, double Ur) { return (ap*Fl - am*Fr + amp*(Ur - Ul))*ida; };
   if constexpr (SOLVER == RIEMANN_HLL) {
-    store_flux<1>(store, hll(l.FD, r.FD, l.D, r.D), hll(l.S[0], r.S[0], l.E, r.E), hll(l.FS[0], r.FS[0], l.S[0], r.S[0]),
+    store_flux(store, hll(l.FD, r.FD, l.D, r.D), hll(l.S[0], r.S[0], l.E, r.E), hll(l.FS[0], r.FS[0], l.S[0], r.S[0]),
                   hll(l.FS[1], r.FS[1], l.S[1], r.S[1]), hll(l.FS[2], r.FS[2], l.S[2], r.S[2]),
                   hll(0.0, 0.0, l.B[0], r.B[0]), hll(l.FB2, r.FB2, l.B[1], r.B[1]), hll(l.FB3, r.FB3, l.B[2], r.B[2]));
     return 0;
@@ -2061,7 +2065,7 @@ __device__ __forceinline__ int riemann_hllx_lean(const double *pl, const double 
       cB2 = k*B2;
       cB3 = k*B3;
     }
-    store_flux<1>(store, FD + lam*(cD - D), S1 + lam*(cE - E), F1 + lam*(c1 - S1), F2 + lam*(c2 - S2), F3 + lam*(c3 - S3),
+    store_flux(store, FD + lam*(cD - D), S1 + lam*(cE - E), F1 + lam*(c1 - S1), F2 + lam*(c2 - S2), F3 + lam*(c3 - S3),
                   0.0, F5 + lam*(cB2 - B2), F6 + lam*(cB3 - B3));
     return 0;
   }
@@ -2132,19 +2136,19 @@ __device__ __forceinline__ void rcp_pair(double x, double y, double &ix, double 
   iy = r*x;
 }
 
-/* `store(q, f)` receives the flux of conserved field q in the lab frame */
-template <int DIM, typename Store>
+/* The states in the frame whose first axis is the normal; `store(q, f)` receives the flux of
+ * conserved field q in that frame */
+template <typename Store>
 __device__ __forceinline__ int riemann_hlld_lean(const double *pl, const double *pr, const PhysParams &pp, double &lam_max,
                                                  FluxCounters &cnt, Store store)
 {
   using T = Tol<double>;
-  using Pm = Perm<DIM>;
   const double gamma = pp.gamma, g1 = pp.g1, gamf = pp.gamf;
-  const double Bn = 0.5*(pl[Pm::B1] + pr[Pm::B1]);
+  const double Bn = 0.5*(pl[Bx] + pr[Bx]);
   const double Bn2 = Bn*Bn;
   const bool small_bn = dfabs(Bn) < T::small_bn;
   auto out = [&](double fD, double fE, double f0, double f1, double f2, double h0, double h1, double h2) {
-    store_flux<DIM>(store, fD, fE, f0, f1, f2, h0, h1, h2);
+    store_flux(store, fD, fE, f0, f1, f2, h0, h1, h2);
   };
 
   FanSide L, Rt;
@@ -2153,8 +2157,8 @@ __device__ __forceinline__ int riemann_hlld_lean(const double *pl, const double 
   {
     FastSide sl, sr;
     {
-      const double Pl[8] = { pl[rho], pl[pre], pl[Pm::v1], pl[Pm::v2], pl[Pm::v3], Bn, pl[Pm::B2], pl[Pm::B3] };
-      const double Pr[8] = { pr[rho], pr[pre], pr[Pm::v1], pr[Pm::v2], pr[Pm::v3], Bn, pr[Pm::B2], pr[Pm::B3] };
+      const double Pl[8] = { pl[rho], pl[pre], pl[vx], pl[vy], pl[vz], Bn, pl[By], pl[Bz] };
+      const double Pr[8] = { pr[rho], pr[pre], pr[vx], pr[vy], pr[vz], Bn, pr[By], pr[Bz] };
       {
         const double ax = Pl[vx] + Pr[vx], ay = Pl[vy] + Pr[vy], az = Pl[vz] + Pr[vz];
         const double om = 1.0 - 0.25*(ax*ax + ay*ay + az*az);

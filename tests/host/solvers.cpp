@@ -22,7 +22,7 @@ void lean(int solver, long n, const double *pl, const double *pr, double gamma, 
     FluxCounters fc = {0, 0, 0, 0};
     auto store = [&](int q, double v) { f[8 * i + q] = v; };
     lam[i] = 0.0;
-    rc[i] = solver == RIEMANN_HLLD ? riemann_hlld_lean<1>(l, r, pp, lam[i], fc, store)
+    rc[i] = solver == RIEMANN_HLLD ? riemann_hlld_lean(l, r, pp, lam[i], fc, store)
           : solver == RIEMANN_HLLC ? riemann_hllx_lean<RIEMANN_HLLC>(l, r, pp, lam[i], store)
                                    : riemann_hllx_lean<RIEMANN_HLL>(l, r, pp, lam[i], store);
     steps[i] = fc.newton_iters;
@@ -66,6 +66,23 @@ void plm_ahead(long n, const double *v, double theta, double *d, double *d_hand_
     d_hand_on[i] = plm<double, true>(a, b, c, 1.0, theta);
     f[i] = plm<float>((float)a, (float)b, (float)c, 1.0f, (float)theta);
     f_hand_on[i] = plm<float, true>((float)a, (float)b, (float)c, 1.0f, (float)theta);
+  }
+}
+
+/* the Jiang-Shu reconstructions of the lean sweeps from n values v[-2..3], and the general ones:
+ * both states of the interface, and the finite-difference flux from both sides */
+void weno5(long n, const double *v, double *lean_f, double *full_f)
+{
+  for (long i = 0; i < n; ++i) {
+    const double *a = v + 6 * i;
+    double *l = lean_f + 4 * i, *f = full_f + 4 * i;
+    weno5_js_pair(a[0], a[1], a[2], a[3], a[4], a[5], l[0], l[1]);
+    l[2] = weno5_js_fd(a[0], a[1], a[2], a[3], a[4]);
+    l[3] = weno5_js_fd(a[5], a[4], a[3], a[2], a[1]);
+    f[0] = weno5<double, true>(a[0], a[1], a[2], a[3], a[4], IS_JS96, 0.0);
+    f[1] = weno5<double, false>(a[1], a[2], a[3], a[4], a[5], IS_JS96, 0.0);
+    f[2] = weno5<double, true, true>(a[0], a[1], a[2], a[3], a[4], IS_JS96, 0.0);
+    f[3] = weno5<double, false, true>(a[1], a[2], a[3], a[4], a[5], IS_JS96, 0.0);
   }
 }
 

@@ -44,6 +44,12 @@ class Solvers:
                            *(o.ctypes.data_as(ctypes.c_void_p) for o in out))
         return out
 
+    def weno5(self, V):
+        V = np.ascontiguousarray(V, dtype=float)
+        F, G = np.zeros((len(V), 4)), np.zeros((len(V), 4))
+        self.lib.weno5(ctypes.c_long(len(V)), *(a.ctypes.data_as(DOUBLES) for a in (V, F, G)))
+        return F, G
+
 
 @pytest.fixture(scope="module")
 def solvers(tmp_path_factory):
@@ -196,3 +202,22 @@ def test_plm_with_infinities_and_not_a_number(solvers, oracle_lib, theta):
         assert (np.isnan(hand_on) | (hand_on.astype(float) == ref)).all()
         # a value that is not a number never goes unseen
         assert np.isnan(hand_on[np.isnan(V).any(axis=1)]).all()
+
+
+@pytest.mark.parametrize("scale", [1e-8, 1.0, 1e8])
+def test_lean_weno5(solvers, scale):
+    """The paired finite-volume states and the finite-difference fluxes against the general
+    reconstruction, smooth and rough values, constant ones exactly: 4e-14 of the largest value
+    (some 50 operations of 2e-16 each, counted four times for the weights, which are fourth
+    powers)."""
+    rng = np.random.default_rng(5)
+    V = rng.uniform(-1, 1, (30000, 6))
+    x = np.arange(6) - 2.5
+    for k in range(10000):
+        V[k] = np.polyval(rng.uniform(-1, 1, 5) * [1e-3, 1e-2, 0.05, 0.2, 1.0], x)
+    V[:100] = V[:100, :1]
+    V *= scale
+    F, G = solvers.weno5(V)
+    assert (np.abs(F - G) <= 4e-14 * np.abs(V).max(axis=1, keepdims=True)).all()
+    assert np.array_equal(F[:100], np.repeat(V[:100, :1], 4, axis=1))
+    assert np.isnan(solvers.weno5(np.where(np.arange(6) == 3, np.nan, V[:1]))[0][:, :3]).all()
