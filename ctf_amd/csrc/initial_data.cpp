@@ -54,15 +54,18 @@ struct Mode {
   cplx c[3];
 };
 
-/* For a last parallel loop: its team goes to sleep at once. By default the team waits actively for
- * 200 ms, and a caller that copies or converts what was made here shares the cores with it (a
- * mixed-precision march of 128^3 on a state just made: 52-75 ms, 35 ms so). The setting is the
- * calling thread's and put back. */
-struct SleepingTeam {
+/* Puts the parallel loops' team to sleep. By default it waits actively for 200 ms after a loop,
+ * and a caller that copies or converts what was made here shares the cores with it (a
+ * mixed-precision march of 128^3 on a state just made: 52-75 ms, 35 ms so). The setting, the
+ * calling thread's, holds for the loop it is made before, and is put back. */
+void rest_team()
+{
   const int before = kmp_get_blocktime();
-  SleepingTeam() { kmp_set_blocktime(0); }
-  ~SleepingTeam() { kmp_set_blocktime(before); }
-};
+  kmp_set_blocktime(0);
+#pragma omp parallel
+  asm volatile("");
+  kmp_set_blocktime(before);
+}
 
 /* f_c(i,j,k) = sum over modes m and their conjugates of c_m e^{i t.(idx + 1/2)} */
 void synthesize(const std::vector<Mode> &modes, int K, const int *N, std::vector<double> *out)
@@ -110,7 +113,6 @@ void synthesize(const std::vector<Mode> &modes, int K, const int *N, std::vector
         T2[comp][((size_t)a * N[1] + j) * N[2] + k] = s;
       }
   }
-  const SleepingTeam last;
 #pragma omp parallel for schedule(static)
   for (int row = 0; row < 3 * N[0]; ++row) {
     const int comp = row / N[0], i = row % N[0];
@@ -236,5 +238,6 @@ extern "C" int mara_init_turbulence(const mara_ic_params *ic, double *P, size_t 
       }
     }
   }
+  rest_team();
   return 0;
 }
