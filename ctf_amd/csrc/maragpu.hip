@@ -924,7 +924,8 @@ __global__ __launch_bounds__(kBlock) void k_flux_redo(const double *__restrict__
   const long T = g.T;
   // Up to kShortQueue interfaces the kernel is bound by the
   // latency of one interface's attempt ladder, and 16 lanes share an interface: 52 -> 29 us
-  // for the 8 a stage of a 64^3 step, 105 -> 39 us at 131x94x113. Above, one lane each, dealt out over the waves first, so that every SIMD has a few.
+  // for the 8 a stage of a 64^3 step, 105 -> 39 us at 131x94x113. Above, one lane each, dealt
+  // out over the waves first, so that every SIMD has a few.
   const unsigned n = view.n;
   const unsigned tid = blockIdx.x * blockDim.x + threadIdx.x, nthreads = gridDim.x * blockDim.x;
   auto redo = [&](unsigned k, auto group) {
@@ -1194,8 +1195,9 @@ __device__ __forceinline__ void char_flux(const double *__restrict__ Uw, const R
  * eigensystem of the averaged primitive state 0.5 (P_z + P_z+S) in FP64 (the eigensystem call at
  * Mara/weno-split.cpp:181), eight lanes to an interface. States with a simple spectrum are done
  * here (eig::g8::simple_projection); the others are queued for k_flux_weno_split_char_redo.
- * At 48x56x44, FP64: 103 us a sweep (2 280 VALU instructions per wave of 8 interfaces, 76 % of the
- * time their issue at 256^3, 34 KB of LDS a block, 4 waves per SIMD), and 4-60 us for the queue;
+ * At 48x56x44, FP64: 103 us a sweep (2 306 VALU instructions per wave of 8 interfaces, 78 % of the
+ * time their issue at 256^3, 34 KB of LDS a block, 4 waves per SIMD), and 4-60 us for the queue (38 us
+ * there; 34 us with the redo at one wave per SIMD, which takes 1.5 times as long where all are queued);
  * 512 us with the general eigensystem for every interface (10 100 instructions, 235 VGPRs, 2
  * waves). Without a field every interface has a cluster and goes on to it: 38 ms a step at 96^3
  * (30 ms with the general eigensystem at once), 67 ms where the short way first formed all
@@ -2687,7 +2689,7 @@ int maragpu_create(const maragpu_config *cfg, maragpu_ctx **out)
   maragpu_host::staging_retain(dev);
   c->cfg = *cfg;
   c->g = make_grid(*cfg);
-  if (c->g.T >= (1L << 32)) { maragpu_host::staging_release(dev); delete c; return MARAGPU_E_INVALID; }   // 32-bit queue slots
+  if (c->g.T >= (1L << 32)) { maragpu_host::staging_release(dev); delete c; return MARAGPU_E_INVALID; }   // 32-bit zone indices
   if (hipStreamCreate(&c->stream) != hipSuccess) { maragpu_host::staging_release(dev); delete c; return MARAGPU_E_HIP; }
   const size_t nd = 8 * (size_t)c->g.T;
   const size_t fbytes = nd * (cfg->precision == MARAGPU_MIXED ? sizeof(float) : sizeof(double));
